@@ -26,6 +26,7 @@
 
 #include "pfh_collectives.hpp"
 #include "pfh_plan.hpp"
+#include "pfh_line.hpp"
 #include "pfh_tune_cache.hpp"
 
 using namespace pfh;
@@ -332,37 +333,65 @@ static bool mode_needs_pre(int mode)
     return !(mode == M_COPY_C || mode == M_COPY_R || mode == M_C2C || mode == M_R2C || mode == M_DHT);
 }
 
-// Picks a compile-time specialized kernel for power-of-two C2C / R2C / C2R
-// lines (k_line_fast); PFH_FAST=0 disables it, PFH_FAST512=<0|1|2> selects
-// the 512-point f32 variant (16x32 with 16 registers, 8x8x8, 16x32 with 32).
 static int env_int(const char *name, int dflt)
 {
     const char *e = std::getenv(name);
     return e ? std::atoi(e) : dflt;
 }
 
-static void choose_fast(Step &st, int tbytes)
+// The line plan (k_line_plan) of an FFT length; radices 0 if there is none.
+static void find_line_plan(int m, int tbytes, int r[3], int &em)
 {
-    st.fast = false;
+    r[0] = 0;
+#define PFH_LINE_FIND(TT, A, B, C, E)                                                \
+    if ((int)sizeof(TT) == tbytes && (A) * (B) * ((C) ? (C) : 1) == m) {            \
+        r[0] = A;                                                                    \
+        r[1] = B;                                                                    \
+        r[2] = C;                                                                    \
+        em = E;                                                                      \
+    }
+    PFH_FAST_ROUTE_PLANS(PFH_LINE_FIND)
+#undef PFH_LINE_FIND
+}
+
+// k_line_plan for a stage whose mode and FFT length it has: radices, values
+// per thread and the flag that routes the launch. Arrays of 4 GiB and more
+// are left out (its offsets have 32 bits; a stage of one line digit, which
+// every local plan is, offsets from its tile and has no such bound).
+static bool choose_line_plan(Step &st, int tbytes)
+{
+    static const int enabled = env_int("PFH_LINE_PLAN", 1);
+    if (!enabled || st.big_bytes >= (1LL << 32)) return false;
+    const bool dht = st.mode == M_DHT && !(st.flags & (F_PRE_REV | F_PRE_ALT | F_POST_REV | F_POST_ALT | F_WEIGHTS));
+    const bool r2r = st.mode == M_DCT1 || st.mode == M_DST1 || st.mode == M_DCT2 || st.mode == M_DCT2_ODD ||
+                     st.mode == M_DCT3 || st.mode == M_DCT3_ODD || st.mode == M_DCT4 || st.mode == M_DCT4_ODD ||
+                     st.mode == M_DHT_ODD;
+    if (!(st.mode == M_C2C || st.mode == M_R2C || st.mode == M_C2R || dht || r2r)) return false;
+    int r[3], em = 0;
+    find_line_plan(st.m, tbytes, r, em);
+    if (r[0] == 0) return false;
+    st.fast = st.line_plan = true;
+    for (int i = 0; i < 3; ++i) st.fr[i] = r[i];
+    st.fem = em;
+    st.radices.assign(r, r + (r[2] ? 3 : 2));
+    return true;
+}
+
+// Picks a compile-time specialized kernel: k_line_fast's plans for the
+// batched kernels and for stages larger than the last-level cache (its
+// non-temporal instances), k_line_plan otherwise. PFH_FAST=0 disables both,
+// PFH_FAST512=<0|1|2> selects k_line_fast's 512-point f32 variant (16x32 with
+// 16 registers, 8x8x8, 16x32 with 32).
+static void choose_fast(Step &st, int tbytes, const Tuning &tu)
+{
+    st.fast = st.line_plan = false;
     static const int enabled = env_int("PFH_FAST", 1);
     static const int v512 = env_int("PFH_FAST512", 0);
+    static const int nt_mb = env_int("PFH_NT_MB", 256);
     if (!enabled) return;
-    // even DHT lines run the R2C plan with a Hartley store (no input /
-    // output reversal, sign alternation or end weights)
-    const bool dht = st.mode == M_DHT && !(st.flags & (F_PRE_REV | F_PRE_ALT | F_POST_REV | F_POST_ALT | F_WEIGHTS));
-    // real-input R2R modes: the first pass gathers the pre-processed values
-    // from global memory, the store applies the generic post-processing.
-    // f32 only: on MI355X the 256-point f32 DCT-II stage of a 256x384x240
-    // field took 101 us against 161 us generic, the f64 one 174 against 164.
-    static const int fast_r2r = env_int("PFH_FAST_R2R", 2);
-    const bool r2r_mode = st.mode == M_DCT1 || st.mode == M_DST1 || st.mode == M_DCT2 || st.mode == M_DCT2_ODD ||
-                          st.mode == M_DCT3 || st.mode == M_DCT3_ODD || st.mode == M_DCT4 || st.mode == M_DCT4_ODD ||
-                          st.mode == M_DHT_ODD;
-    // PFH_FAST_R2R: 0 off, 1 f32 only, 2 f32 and f64 (f64 256x384x240 R2R
-    // forward + inverse on MI355X: 1.39 against 1.49 ms with the generic
-    // kernel for the DCT stages)
-    const bool r2r = r2r_mode && (tbytes == 4 ? fast_r2r >= 1 : fast_r2r >= 2);
-    if (!(st.mode == M_C2C || st.mode == M_R2C || st.mode == M_C2R || dht || r2r)) return;
+    const bool large = nt_mb > 0 && st.io_bytes > ((int64_t)nt_mb << 20);
+    if (tu.allow_line_plan && !large && choose_line_plan(st, tbytes)) return;
+    const bool has_mode = st.mode == M_C2C || st.mode == M_R2C || st.mode == M_C2R;
     const int m = st.m;
     int r0 = 0, r1 = 0, r2 = 0, em = 0;
     if (tbytes == 4) {
@@ -380,19 +409,9 @@ static void choose_fast(Step &st, int tbytes)
         case 240: r0 = 16; r1 = 3; r2 = 5; em = 16; break;
         case 320: r0 = 16; r1 = 4; r2 = 5; em = 16; break;
         case 384: r0 = 16; r1 = 8; r2 = 3; em = 16; break;
-        case 385: // real-input plan: DST-I lines of length 384 and the odd 385-point
-                  // DCT-II / DCT-III / DST-II / DST-III / DHT lines (never C2C)
-            if (r2r) { r0 = 11; r1 = 7; r2 = 5; em = 11; }
-            break;
         default: break;
         }
-    } else if (st.mode == M_R2C || st.mode == M_C2R || dht || r2r) {
-        // route-only f64 plans (never C2C, so never a batched line)
-        if (m == 120) { r0 = 8; r1 = 3; r2 = 5; em = 8; }
-        if (m == 192) { r0 = 8; r1 = 8; r2 = 3; em = 8; }
-        if (m == 385 && r2r) { r0 = 11; r1 = 7; r2 = 5; em = 11; }
     }
-    if (r0 == 0 && (m < 64 || (m & (m - 1)) != 0)) return;
     if (r0 != 0) {
         // mixed radix plan chosen above
     } else if (tbytes == 4) {
@@ -406,7 +425,7 @@ static void choose_fast(Step &st, int tbytes)
             else { r0 = 16; r1 = 32; em = 16; }
             break;
         case 1024: r0 = 32; r1 = 32; em = 32; break;
-        default: return;
+        default: break;
         }
     } else {
         switch (m) {
@@ -414,11 +433,14 @@ static void choose_fast(Step &st, int tbytes)
         case 128: r0 = 4; r1 = 4; r2 = 8; em = 8; break;
         case 256: r0 = 4; r1 = 8; r2 = 8; em = 8; break;
         case 512: r0 = 8; r1 = 8; r2 = 8; em = 8; break;
-        default: return;
+        default: break;
         }
     }
-    if (r0 == 32) return; // the direct first pass covers radix <= 16
-    if (!fast_plan_available(tbytes, r0, r1, r2, em)) return;
+    // (radix 32: the direct first pass covers radix <= 16)
+    if (!has_mode || r0 == 0 || r0 == 32 || !fast_plan_available(tbytes, r0, r1, r2, em)) {
+        if (tu.allow_line_plan) choose_line_plan(st, tbytes);
+        return;
+    }
     st.fast = true;
     st.fr[0] = r0;
     st.fr[1] = r1;
@@ -511,7 +533,7 @@ static pfh_status fill_transform(Step &st, const StageSpec &sp, std::vector<doub
     const int max_r = tu.max_radix ? tu.max_radix : (tbytes == 4 ? 16 : 8);
     st.long_only = !radix_plan(st.m, st.radices, max_r); // more passes than a stage holds: pieces only
     if (st.long_only) st.radices.clear();
-    if (tu.allow_fast && !st.long_only) choose_fast(st, tbytes);
+    if (tu.allow_fast && !st.long_only) choose_fast(st, tbytes, tu);
 
     // tables
     st.tw_base = (int64_t)(tab.size() / 2);
@@ -521,7 +543,7 @@ static pfh_status fill_transform(Step &st, const StageSpec &sp, std::vector<doub
     for (size_t p = 0; p < st.radices.size(); ++p) {
         const int R = st.radices[p];
         st.twoff[p] = here();
-        if (is_generic_radix(R)) { // roots exp(-2 pi i e / R) precede the pass twiddles
+        if (!st.line_plan && is_generic_radix(R)) { // roots exp(-2 pi i e / R) precede the pass twiddles
             for (int e = 0; e < R; ++e) {
                 push_cexp(tab, e, R);
                 ++off;
@@ -537,9 +559,11 @@ static pfh_status fill_transform(Step &st, const StageSpec &sp, std::vector<doub
         Ns *= R;
     }
     const int m = st.m;
+    // k_line_plan computes X_k and X_{m-k} from one table entry, k <= m / 2
+    const int half = st.line_plan ? m / 2 : m;
     auto split_table = [&]() { // exp(-2 pi i k / 2m), k = 0..m
         int o = here();
-        for (int k = 0; k <= m; ++k) {
+        for (int k = 0; k <= half; ++k) {
             push_cexp(tab, k, 2LL * m);
             ++off;
         }
@@ -552,7 +576,7 @@ static pfh_status fill_transform(Step &st, const StageSpec &sp, std::vector<doub
     case M_DCT2:
         st.post0 = split_table();
         st.post1 = here();
-        for (int k = 0; k < n; ++k) { push_cexp(tab, k, 4 * n); ++off; }
+        for (int k = 0; k < (st.line_plan ? m + 1 : n); ++k) { push_cexp(tab, k, 4 * n); ++off; }
         break;
     case M_DCT2_ODD:
         st.post0 = here();
@@ -560,13 +584,13 @@ static pfh_status fill_transform(Step &st, const StageSpec &sp, std::vector<doub
         break;
     case M_C2R:
         st.pre0 = here();
-        for (int j = 0; j < m; ++j) { push_cexp(tab, j, n, true); ++off; }
+        for (int j = 0; j < (st.line_plan ? half + 1 : m); ++j) { push_cexp(tab, j, n, true); ++off; }
         break;
     case M_DCT3:
         st.pre0 = here();
         for (int k = 0; k <= m; ++k) { push_cexp(tab, k, 4 * n, true); ++off; }
         st.pre1 = here();
-        for (int j = 0; j < m; ++j) { push_cexp(tab, j, n, true); ++off; }
+        for (int j = 0; j < (st.line_plan ? half + 1 : m); ++j) { push_cexp(tab, j, n, true); ++off; }
         break;
     case M_DCT3_ODD:
         st.pre0 = here();
@@ -663,6 +687,7 @@ static pfh_status step_geometry(Step &st)
 // the pre-processing) covered, rounded up to a power of two.
 static int threads_per_line(const Step &st, int tbytes)
 {
+    if (st.line_plan) return line_plan_tpl(st.fr[0], st.fr[1], st.fr[2], st.fem);
     bool wide_plan = false;
     for (int R : st.radices) wide_plan = wide_plan || is_wide_radix(R);
     const int emax = st.fast ? st.fem : kEmax;
@@ -680,9 +705,47 @@ static int threads_per_line(const Step &st, int tbytes)
     return pow2ceil(need);
 }
 
+// Launch shape of a k_line_plan stage. Column sides: tiles of a power of two
+// of lines whose points are runs of 256 bytes (complex) or 128 bytes (real),
+// halved while the workgroup is too large, or, down to 128-byte (complex) and
+// 64-byte runs, while two workgroups do not share a CU's LDS. Rows: about 256
+// threads.
+static pfh_status size_line_plan(Step &st, const DeviceInfo &dev, int tbytes, const Tuning &tu)
+{
+    const int cb = 2 * tbytes;
+    const int tpl = line_plan_tpl(st.fr[0], st.fr[1], st.fr[2], st.fem);
+    st.ls = line_plan_stride(st.fr[0], st.fr[1], st.fr[2]);
+    auto lds_of = [&](int l) { return (size_t)(st.twn + (int64_t)l * st.ls) * (size_t)cb; };
+    int lt = 1;
+    const bool col = st.in_col || st.out_col;
+    if (col) {
+        if (st.in_col) lt = std::max(lt, st.in_cplx ? 256 / cb : 128 / tbytes);
+        if (st.out_col) lt = std::max(lt, st.out_cplx ? 256 / cb : 128 / tbytes);
+        if (g_column_lines > 0) lt = pow2ceil(g_column_lines);
+        while (lt > 1 && (int64_t)(lt / 2) >= st.nlines) lt /= 2;
+        while (lt > 1 && lt * tpl > kLinePlanThreads) lt /= 2;
+        const int least = std::max(st.in_col ? (st.in_cplx ? 128 / cb : 64 / tbytes) : 1,
+                                   st.out_col ? (st.out_cplx ? 128 / cb : 64 / tbytes) : 1);
+        while (lt / 2 >= least && lds_of(lt) > dev.lds_limit / 2) lt /= 2;
+    } else {
+        lt = (int)std::max<int64_t>(1, std::min<int64_t>(256 / tpl, st.nlines));
+    }
+    while (lt > 1 && lds_of(lt) > dev.lds_limit) lt /= 2;
+    if (lds_of(lt) > dev.lds_limit) return set_err(PFH_ERR_UNSUPPORTED, "line does not fit in LDS");
+    st.lt = st.lc = lt;
+    st.tpl = tpl;
+    st.threads = lt * tpl;
+    st.lds_bytes = lds_of(lt);
+    set_tiles(st, tu);
+    st.flags &= ~F_NT;
+    st.flags |= F_LINE_PLAN;
+    return PFH_OK;
+}
+
 // Launch shape (tile, threads per line, LDS) of a step whose line grid is set.
 static pfh_status size_step(Step &st, const DeviceInfo &dev, int tbytes, const Tuning &tu)
 {
+    if (st.line_plan) return size_line_plan(st, dev, tbytes, tu);
     const int cb = 2 * tbytes;
     const int in_eb = st.in_cplx ? cb : tbytes, out_eb = st.out_cplx ? cb : tbytes;
     // column access: enough lines per tile that each point of the tile is a
@@ -738,37 +801,6 @@ static pfh_status size_step(Step &st, const DeviceInfo &dev, int tbytes, const T
     st.threads = lc * tpl;
     st.lds_bytes = lds_of(lt);
     set_tiles(st, tu);
-    // Real column sides of the compile-time R2R (load and store) and DHT
-    // (store) stages: lines 2i and 2i + 1 of a tile are neighbouring
-    // elements when the fastest line digit has stride 1 and an even extent
-    // and every other line stride and the point stride are even; a lane
-    // then moves both with one 2-element access (PFH_CPAIR=0: one element).
-    static const int cpair_env = env_int("PFH_CPAIR", 1);
-    st.flags &= ~(F_CPAIR_IN | F_CPAIR_OUT | F_RPAIR_IN | F_RPAIR_OUT);
-    const bool kind2 = st.mode != M_C2C && st.mode != M_R2C && st.mode != M_C2R && st.mode != M_DHT;
-    auto pairs_ok = [&](bool in) {
-        const LineGeom &g = st.g;
-        if (g.nd < 1 || g.ext[0] % 2 != 0 || (in ? g.is[0] : g.os[0]) != 1 || (in ? st.ips : st.ops) % 2 != 0)
-            return false;
-        for (int d = 1; d < g.nd; ++d)
-            if ((in ? g.is[d] : g.os[d]) % 2 != 0) return false;
-        return st.lt % 2 == 0;
-    };
-    if (cpair_env && st.fast && !st.long_only) {
-        if (kind2 && st.in_col && !st.in_cplx && pairs_ok(true)) st.flags |= F_CPAIR_IN;
-        if ((kind2 || st.mode == M_DHT) && st.out_col && !st.out_cplx && pairs_ok(false)) st.flags |= F_CPAIR_OUT;
-        // rows of the R2R stages: an even number of points and even line
-        // offsets keep every point pair 2-element aligned
-        auto rows_ok = [&](bool in) {
-            const LineGeom &g = st.g;
-            if ((in ? st.ips : st.ops) != 1 || (in ? st.nin : st.nout) % 2 != 0) return false;
-            for (int d = 0; d < g.nd; ++d)
-                if ((in ? g.is[d] : g.os[d]) % 2 != 0) return false;
-            return true;
-        };
-        if (kind2 && !st.in_col && !st.in_cplx && rows_ok(true)) st.flags |= F_RPAIR_IN;
-        if (kind2 && !st.out_col && !st.out_cplx && rows_ok(false)) st.flags |= F_RPAIR_OUT;
-    }
     // Non-temporal global accesses (the compile-time radix plans only) once
     // the stage's input and output together exceed the 256 MB last-level
     // cache (PFH_NT_MB overrides the threshold, 0 turns them off): measured
@@ -1290,7 +1322,7 @@ static pfh_status core_pieces(PlanImpl &P, const Step &outer, int64_t m, const L
 static pfh_status expand_long(PlanImpl &P, Step &s, int tb, int64_t xb[3])
 {
     s.pieces.clear();
-    s.fast = false;
+    s.fast = s.line_plan = false;
     if (s.g.nd + 1 > kMaxDigits) return set_err(PFH_ERR_UNSUPPORTED, "too many line digits for a long line");
     LineSide in, out;
     in.buf = s.in_buf;
@@ -1803,6 +1835,8 @@ static pfh_status build_op(PlanImpl &P, int op, bool in_place, OpPlan &out)
     for (int e = 0; e < K; ++e) {
         std::vector<double> scratch;
         Step probe;
+        probe.big_bytes = std::max(specs[e].in_natural.bytes(), specs[e].out_natural.bytes());
+        probe.io_bytes = specs[e].in_natural.bytes() + specs[e].out_natural.bytes();
         const pfh_error_info saved = g_err;
         if (fill_transform(probe, specs[e], scratch, tb, P.tuning) == PFH_OK && !probe.long_only &&
             !wants_pieces(probe))
@@ -1815,6 +1849,8 @@ static pfh_status build_op(PlanImpl &P, int op, bool in_place, OpPlan &out)
     for (int r = 0; r < 3; ++r) out.x_bytes[r] = 0;
     for (int e = 0; e < K; ++e) {
         Step s;
+        s.big_bytes = std::max(X[e].bytes(), Y[e].bytes());
+        s.io_bytes = X[e].bytes() + Y[e].bytes();
         st = fill_transform(s, specs[e], P.host_tables, tb, P.tuning);
         if (st) return st;
         s.in = X[e];
@@ -2391,11 +2427,6 @@ static StageArgs<T> fill_args(const PlanImpl &P, const Step &s, void *const bufs
     a.ops = s.ops;
     a.mode = s.mode;
     a.flags = s.flags;
-    // paired column accesses need 2-element alignment of the array bases
-    if ((a.flags & F_CPAIR_IN) && reinterpret_cast<uintptr_t>(a.src) % (2 * sizeof(T)) != 0) a.flags &= ~F_CPAIR_IN;
-    if ((a.flags & F_CPAIR_OUT) && reinterpret_cast<uintptr_t>(a.dst) % (2 * sizeof(T)) != 0) a.flags &= ~F_CPAIR_OUT;
-    if ((a.flags & F_RPAIR_IN) && reinterpret_cast<uintptr_t>(a.src) % (2 * sizeof(T)) != 0) a.flags &= ~F_RPAIR_IN;
-    if ((a.flags & F_RPAIR_OUT) && reinterpret_cast<uintptr_t>(a.dst) % (2 * sizeof(T)) != 0) a.flags &= ~F_RPAIR_OUT;
     a.n = s.n;
     a.nin = s.nin;
     a.nout = s.nout;
@@ -3886,6 +3917,7 @@ static Tuning batch_candidate(int block, int col_lines, bool plane, bool persist
     t.col_lines = col_lines;
     t.block_cap = kMaxThreadsWide;
     t.allow_fast = true;
+    t.allow_line_plan = false;
     t.allow_xcd = false;
     t.slab_mb = 0;
     t.fill_block = true;
@@ -4038,6 +4070,7 @@ pfh_status pfh_batch_create(const pfh_desc *descs, int count, int autotune, pfh_
     if (!b) return set_err(PFH_ERR_ALLOCATION_FAILED, "batch");
     Tuning t;
     t.allow_fast = true;
+    t.allow_line_plan = false;
     t.allow_xcd = false;
     t.block = 256;
     t.block_cap = kMaxThreadsWide;

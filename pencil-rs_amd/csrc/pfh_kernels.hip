@@ -451,22 +451,14 @@ __device__ __forceinline__ void radix_pass_generic(cpx<T> *ln, const cpx<T> *roo
 // lines per round. Threads beyond lc * tpl get nothing.
 template <typename T>
 __device__ __forceinline__ void tile_mapping(const StageArgs<T> &a, int col, int tid, int l, int tl, int &ll, int &p0,
-                                             int &step, int &lstep, int &cnt, bool pair = false)
+                                             int &step, int &lstep, int &cnt)
 {
     const int lt = a.lt, lc = a.lc, tpl = a.tpl;
     if (col) {
         const int rows = lc * tpl / lt;
-        if (pair) {
-            // lines 2i and 2i + 1 per lane (paired column accesses)
-            const int hl = lt >> 1;
-            ll = 2 * (tid % hl);
-            p0 = tid / hl;
-            step = 2 * rows;
-        } else {
-            ll = tid % lt;
-            p0 = tid / lt;
-            step = rows;
-        }
+        ll = tid % lt;
+        p0 = tid / lt;
+        step = rows;
         lstep = 0;
         cnt = tid < rows * lt ? 1 : 0;
     } else {
@@ -478,49 +470,8 @@ __device__ __forceinline__ void tile_mapping(const StageArgs<T> &a, int col, int
     }
 }
 
-// Real-input R2R modes whose FFT input is a signed permutation of the line
-// (plus zeros): DST-I (odd extension of length 2n + 2), DCT-II (even
-// points forward, odd points backward) and DCT-IV (pairs x_2j, x_n-1-2j,
-// the pre-twiddle applied by the first pass). Their compile-time-mode
-// kernels put each loaded value straight into its FFT-input slot(s).
-template <int MODE>
-constexpr bool scatter_mode()
-{
-    return MODE == M_DST1 || MODE == M_DCT2 || MODE == M_DCT4;
-}
-
-// Point p of a raw real line into the FFT input of a scatter mode, after the
-// stage's input reversal / alternating sign / edge weights (the values the
-// gathered pre-processing reads through xin).
-template <typename T, int MODE>
-__device__ __forceinline__ void scatter_real(const StageArgs<T> &a, cpx<T> *lln, int p, T v)
-{
-    const int n = a.n;
-    int q = p;
-    if (a.flags & (F_PRE_REV | F_PRE_ALT | F_WEIGHTS)) {
-        if ((a.flags & F_PRE_ALT) && (p & 1)) v = -v;
-        if (a.flags & F_WEIGHTS) {
-            if (p == 0) v = v * a.prew0;
-            if (p == n - 1) v = v * a.prew1;
-        }
-        if (a.flags & F_PRE_REV) q = n - 1 - p;
-    }
-    if constexpr (MODE == M_DST1) {
-        // o_{q+1} = x_q, o_{2n+1-q} = -x_q (o_0 = o_{n+1} = 0)
-        LRset(lln, q + 1, v);
-        LRset(lln, 2 * n + 1 - q, -v);
-    } else if constexpr (MODE == M_DCT2) {
-        // v_i = x_2i (i < n / 2), v_i = x_{2(n-1-i)+1} (i >= n / 2)
-        LRset(lln, (q & 1) ? n - 1 - (q >> 1) : (q >> 1), v);
-    } else {
-        // z_j = (x_2j, x_{n-1-2j}): real slot 2j or 2j + 1
-        LRset(lln, (q & 1) ? n - q : q, v);
-    }
-}
-
-// Line ll of the tile, points p0, p0 + step, ... : global -> LDS (the FFT
-// input of a scatter mode when MODE is one).
-template <typename T, bool NT, int MODE = -1>
+// Line ll of the tile, points p0, p0 + step, ... : global -> LDS.
+template <typename T, bool NT>
 __device__ __forceinline__ void load_line(const StageArgs<T> &a, cpx<T> *data, int64_t tile, int ll, int p0, int step)
 {
     const bool cin = complex_input(a.mode);
@@ -577,78 +528,8 @@ __device__ __forceinline__ void load_line(const StageArgs<T> &a, cpx<T> *data, i
                     }
                 }
             }
-        } else if (a.in_col && (a.flags & F_CPAIR_IN)) {
-            // lines ll and ll + 1: neighbouring elements, one 2-element load
-            const cpx<T> *s2 = reinterpret_cast<const cpx<T> *>(reinterpret_cast<const T *>(a.src) + io);
-            const int64_t ips2 = a.ips >> 1;
-            cpx<T> *lln1 = lln + a.ls;
-            if constexpr (MODE == M_DST1) {
-                if (p0 == 0) {
-                    LRset(lln, 0, (T)0);
-                    LRset(lln, a.n + 1, (T)0);
-                    LRset(lln1, 0, (T)0);
-                    LRset(lln1, a.n + 1, (T)0);
-                }
-            }
-            for (int base = p0; base < a.nin; base += step * Regs<T>::gunroll) {
-                cpx<T> v[Regs<T>::gunroll];
-#pragma unroll
-                for (int u = 0; u < Regs<T>::gunroll; ++u) {
-                    const int p = base + u * step;
-                    if (p < a.nin) v[u] = gld<NT>(s2 + (int64_t)p * ips2);
-                }
-#pragma unroll
-                for (int u = 0; u < Regs<T>::gunroll; ++u) {
-                    const int p = base + u * step;
-                    if (p < a.nin) {
-                        if constexpr (scatter_mode<MODE>()) {
-                            scatter_real<T, MODE>(a, lln, p, v[u].x);
-                            scatter_real<T, MODE>(a, lln1, p, v[u].y);
-                        } else {
-                            LRset(lln, p, v[u].x);
-                            LRset(lln1, p, v[u].y);
-                        }
-                    }
-                }
-            }
-        } else if (!a.in_col && (a.flags & F_RPAIR_IN)) {
-            // points 2i and 2i + 1 of the row in one 2-element load
-            const cpx<T> *s2 = reinterpret_cast<const cpx<T> *>(reinterpret_cast<const T *>(a.src) + io);
-            const int np = a.nin >> 1;
-            if constexpr (MODE == M_DST1) {
-                if (p0 == 0) {
-                    LRset(lln, 0, (T)0);
-                    LRset(lln, a.n + 1, (T)0);
-                }
-            }
-            for (int base = p0; base < np; base += step * Regs<T>::gunroll) {
-                cpx<T> v[Regs<T>::gunroll];
-#pragma unroll
-                for (int u = 0; u < Regs<T>::gunroll; ++u) {
-                    const int i = base + u * step;
-                    if (i < np) v[u] = gld<NT>(s2 + i);
-                }
-#pragma unroll
-                for (int u = 0; u < Regs<T>::gunroll; ++u) {
-                    const int i = base + u * step;
-                    if (i < np) {
-                        if constexpr (scatter_mode<MODE>()) {
-                            scatter_real<T, MODE>(a, lln, 2 * i, v[u].x);
-                            scatter_real<T, MODE>(a, lln, 2 * i + 1, v[u].y);
-                        } else {
-                            Lset(lln, i, v[u]);
-                        }
-                    }
-                }
-            }
         } else {
             const T *s = reinterpret_cast<const T *>(a.src) + io;
-            if constexpr (MODE == M_DST1) {
-                if (p0 == 0) {
-                    LRset(lln, 0, (T)0);
-                    LRset(lln, a.n + 1, (T)0);
-                }
-            }
             for (int base = p0; base < a.nin; base += step * (2 * Regs<T>::gunroll)) {
                 T v[2 * Regs<T>::gunroll];
 #pragma unroll
@@ -660,8 +541,7 @@ __device__ __forceinline__ void load_line(const StageArgs<T> &a, cpx<T> *data, i
                 for (int u = 0; u < 2 * Regs<T>::gunroll; ++u) {
                     const int p = base + u * step;
                     if (p < a.nin) {
-                        if constexpr (scatter_mode<MODE>()) scatter_real<T, MODE>(a, lln, p, v[u]);
-                        else LRset(lln, p, v[u]);
+                        LRset(lln, p, v[u]);
                     }
                 }
             }
@@ -672,18 +552,18 @@ __device__ __forceinline__ void load_line(const StageArgs<T> &a, cpx<T> *data, i
 // Tile load: global -> LDS. lc lines are computed at a time (lc * tpl
 // threads) and the tile holds lt = lc * rounds lines. Threads beyond
 // lc * tpl only join the barrier.
-template <typename T, bool NT, int MODE = -1>
+template <typename T, bool NT>
 __device__ __forceinline__ void stage_load(const StageArgs<T> &a, cpx<T> *data, int64_t tile, int tid, int l, int tl)
 {
     int ll, p0, step, lstep, cnt;
-    tile_mapping(a, a.in_col, tid, l, tl, ll, p0, step, lstep, cnt, a.in_col && (a.flags & F_CPAIR_IN));
+    tile_mapping(a, a.in_col, tid, l, tl, ll, p0, step, lstep, cnt);
 #pragma unroll 1
     for (int i = 0; i < cnt; ++i) {
         // an opaque copy of the first point per line keeps the compiler from
         // hoisting per-point work out of the loop (and spilling it)
         int p = p0;
         asm volatile("" : "+v"(p));
-        load_line<T, NT, MODE>(a, data, tile, ll + i * lstep, p, step);
+        load_line<T, NT>(a, data, tile, ll + i * lstep, p, step);
     }
     __syncthreads();
 }
@@ -770,24 +650,6 @@ __device__ __forceinline__ void store_line(const StageArgs<T> &a, const cpx<T> *
                         if (k < a.nout) gst<NT>(d + (int64_t)k * a.ops, v[u]);
                     }
                 }
-            } else if (MG == 2 && !a.out_col && (a.flags & F_RPAIR_OUT)) {
-                // outputs 2i and 2i + 1 of the row in one 2-element store
-                cpx<T> *d2 = reinterpret_cast<cpx<T> *>(reinterpret_cast<T *>(a.dst) + oo);
-                const int np = a.nout >> 1;
-                for (int base = k0; base < np; base += tpl * U) {
-                    cpx<T> v[U];
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        const int i = base + u * tpl;
-                        if (i < np)
-                            v[u] = mk(post_real<T, MG, MODE>(a, Z, tws, 2 * i), post_real<T, MG, MODE>(a, Z, tws, 2 * i + 1));
-                    }
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        const int i = base + u * tpl;
-                        if (i < np) gst<NT>(d2 + i, v[u]);
-                    }
-                }
             } else {
                 T *d = reinterpret_cast<T *>(a.dst) + oo;
                 for (int base = k0; base < a.nout; base += tpl * U) {
@@ -822,36 +684,6 @@ __device__ __forceinline__ void stage_store(const StageArgs<T> &a, const cpx<T> 
         int k = k0;
         asm volatile("" : "+v"(k));
         store_line<T, MG, NT, MODE>(a, data, tws, tile, lo + i * lstep, k, step);
-    }
-}
-
-// Lines lo and lo + 1 of the tile (neighbouring output elements), points
-// k0, k0 + step, ...: real post-processing of both, one 2-element store.
-template <typename T, int MG, bool NT, int MODE = -1>
-__device__ __forceinline__ void store_line_pair(const StageArgs<T> &a, const cpx<T> *data, const cpx<T> *tws,
-                                                int64_t tile, int lo, int k0, int step)
-{
-    const int64_t line = tile * a.lt + lo;
-    if (line >= a.nlines) return;
-    int64_t io, oo;
-    line_offsets(a.g, line, io, oo);
-    const cpx<T> *Z0 = data + lo * a.ls;
-    const cpx<T> *Z1 = Z0 + a.ls;
-    cpx<T> *d = reinterpret_cast<cpx<T> *>(reinterpret_cast<T *>(a.dst) + oo);
-    const int64_t ops2 = a.ops >> 1;
-    constexpr int U = Regs<T>::gunroll;
-    for (int base = k0; base < a.nout; base += step * U) {
-        cpx<T> v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = base + u * step;
-            if (k < a.nout) v[u] = mk(post_real<T, MG, MODE>(a, Z0, tws, k), post_real<T, MG, MODE>(a, Z1, tws, k));
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = base + u * step;
-            if (k < a.nout) gst<NT>(d + (int64_t)k * ops2, v[u]);
-        }
     }
 }
 
@@ -1080,40 +912,6 @@ __device__ __forceinline__ void fast_first(const StageArgs<T> &a, cpx<T> *ln, bo
     __syncthreads();
 }
 
-// First pass of a real-input R2R line whose raw values are already in the
-// LDS line (stage_load): the pre-processing gathers each FFT input value from
-// LDS (reordering, odd / even extension, pre-twiddles), then, after every
-// thread of the tile has read its values, the radix-R0 butterflies write the
-// pass output over the raw line.
-template <typename T, int R, int EM, int M, int MODE = -1>
-__device__ __forceinline__ void fast_first_pre_lds(const StageArgs<T> &a, cpx<T> *ln, const cpx<T> *tws, int tl,
-                                                   int tpl)
-{
-    constexpr int MB = fast_mb<EM, R>();
-    constexpr int NB = M / R;
-    cpx<T> v[MB][R];
-    const LdsReal<T> rd{ln};
-#pragma unroll
-    for (int b = 0; b < MB; ++b) {
-        const int j = tl + tpl * b;
-        if (j < NB) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) v[b][r] = pre_real<T, LdsReal<T>, MODE>(a, rd, tws, j + r * NB);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < MB; ++b) {
-        const int j = tl + tpl * b;
-        if (j < NB) {
-            Dft<T, R>::run(v[b]);
-#pragma unroll
-            for (int r = 0; r < R; ++r) Lset(ln, j * R + r, v[b][r]);
-        }
-    }
-    __syncthreads();
-}
-
 // a pass in LDS with compile-time geometry
 template <typename T, int R, int EM, int M>
 __device__ __forceinline__ void fast_mid(cpx<T> *ln, const cpx<T> *twp, int Ns, int tl, int tpl)
@@ -1144,35 +942,6 @@ __device__ __forceinline__ void fast_mid(cpx<T> *ln, const cpx<T> *twp, int Ns, 
             const int base = (j - k) * R + k;
 #pragma unroll
             for (int r = 0; r < R; ++r) Lset(ln, base + r * Ns, v[b][r]);
-        }
-    }
-    __syncthreads();
-}
-
-// first pass (Ns = 1) in LDS, each input value j times pre[j] (the DCT-IV
-// pre-twiddle of a scattered line)
-template <typename T, int R, int EM, int M>
-__device__ __forceinline__ void fast_first_tw(cpx<T> *ln, const cpx<T> *pre, int tl, int tpl)
-{
-    constexpr int MB = fast_mb<EM, R>();
-    constexpr int NB = M / R;
-    cpx<T> v[MB][R];
-#pragma unroll
-    for (int b = 0; b < MB; ++b) {
-        const int j = tl + tpl * b;
-        if (j < NB) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) v[b][r] = cmul(L(ln, j + r * NB), pre[j + r * NB]);
-            Dft<T, R>::run(v[b]);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < MB; ++b) {
-        const int j = tl + tpl * b;
-        if (j < NB) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) Lset(ln, j * R + r, v[b][r]);
         }
     }
     __syncthreads();
@@ -1364,91 +1133,11 @@ __device__ __forceinline__ void fast_r2c_store(const StageArgs<T> &a, const cpx<
     }
 }
 
-// DHT store of an even line from the half-length transform of its real
-// pairs in LDS: H_k = Re X_k - Im X_k, with X_k = conj(X_{n-k}) above the
-// Nyquist index m (the generic kernel's post-processing of M_DHT).
-template <typename T, bool NT>
-__device__ __forceinline__ void fast_dht_store(const StageArgs<T> &a, const cpx<T> *data, const cpx<T> *tws,
-                                               int64_t tile, int tid, int l, int tl)
-{
-    const int lt = a.lt, tpl = a.tpl;
-    const cpx<T> *w = tws + a.post0;
-    const int m = a.m;
-    constexpr int U = Regs<T>::unroll;
-    if (a.out_col && (a.flags & F_CPAIR_OUT)) {
-        // lines lo and lo + 1: neighbouring elements, one 2-element store
-        const int hl = lt >> 1;
-        const int lo = 2 * (tid % hl), k0 = tid / hl, step = 2 * tpl;
-        const int64_t line = tile * lt + lo;
-        if (line >= a.nlines) return;
-        int64_t io, oo;
-        line_offsets(a.g, line, io, oo);
-        const cpx<T> *Z0 = data + lo * a.ls;
-        const cpx<T> *Z1 = Z0 + a.ls;
-        cpx<T> *d = reinterpret_cast<cpx<T> *>(reinterpret_cast<T *>(a.dst) + oo);
-        const int64_t ops2 = a.ops >> 1;
-        for (int base = k0; base < a.nout; base += step * U) {
-            cpx<T> v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int k = base + u * step;
-                if (k < a.nout) {
-                    const bool low = k <= m;
-                    const int kk = low ? k : 2 * m - k;
-                    const cpx<T> x0 = split(Z0, w, m, kk), x1 = split(Z1, w, m, kk);
-                    v[u] = scal(low ? mk(x0.x - x0.y, x1.x - x1.y) : mk(x0.x + x0.y, x1.x + x1.y), a.scale);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int k = base + u * step;
-                if (k < a.nout) gst<NT>(d + (int64_t)k * ops2, v[u]);
-            }
-        }
-        return;
-    }
-    int lo, k0;
-    if (a.out_col) {
-        lo = tid % lt;
-        k0 = tid / lt;
-    } else {
-        lo = l;
-        k0 = tl;
-    }
-    const int64_t line = tile * lt + lo;
-    if (line >= a.nlines) return;
-    int64_t io, oo;
-    line_offsets(a.g, line, io, oo);
-    const cpx<T> *Z = data + lo * a.ls;
-    T *d = reinterpret_cast<T *>(a.dst) + oo;
-    for (int base = k0; base < a.nout; base += tpl * U) {
-        T v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = base + u * tpl;
-            if (k < a.nout) {
-                const bool low = k <= m;
-                const cpx<T> x = split(Z, w, m, low ? k : 2 * m - k);
-                v[u] = (low ? x.x - x.y : x.x + x.y) * a.scale;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = base + u * tpl;
-            if (k < a.nout) gst<NT>(d + (int64_t)k * a.ops, v[u]);
-        }
-    }
-}
-
 // One tile of a fast stage: tws holds the staged tables, data the tile's
 // lines. Threads beyond the stage's lt x tpl shape (a batched launch sized
 // for its largest item) take indexes past every line and only join the
-// barriers. NT: non-temporal global loads and stores. KIND: 0 = C2C lines
-// only (the batched kernels), 1 = route stages of the C2C / R2C / C2R / DHT
-// modes, 2 = route stages of the real-input R2R modes (their gathers and
-// post-processing live in an instantiation of their own, so the other
-// route kernels keep their smaller code).
-template <typename T, int R0, int R1, int R2, int EM, bool NT, int KIND = 1, int MODE = -1>
+// barriers. NT: non-temporal global loads and stores.
+template <typename T, int R0, int R1, int R2, int EM, bool NT>
 __device__ __forceinline__ void fast_body(const StageArgs<T> &a, int64_t tile, const cpx<T> *tws, cpx<T> *data)
 {
     constexpr int M = R0 * R1 * (R2 ? R2 : 1);
@@ -1460,71 +1149,37 @@ __device__ __forceinline__ void fast_body(const StageArgs<T> &a, int64_t tile, c
     const int tl = act ? tid % tpl : (1 << 28);
     cpx<T> *ln = data + l * a.ls;
     const int mode = a.mode;
-    if constexpr (KIND == 2) {
-        // real-input R2R modes: the raw lines go to LDS with coalesced loads
-        // (the generic kernel's tile load), the first pass gathers its
-        // pre-processed inputs from there; generic post-processing at the
-        // store. (Gathering straight from global memory, 4-byte loads at
-        // the reorder's strides, made the 256x384x240 f32 R2R stages run at
-        // 0.8-2.0 TB/s.) The compile-time scatter modes place the values
-        // at their FFT-input slots as they load, so the first pass reads
-        // complex values without the per-value index arithmetic.
-        __syncthreads(); // the pre-processing reads the staged tables
-        stage_load<T, NT, MODE>(a, data, tile, tid, l, act ? tl : (1 << 28));
-        if constexpr (MODE == M_DCT4) fast_first_tw<T, R0, EM, M>(ln, tws + a.pre0, tl, tpl);
-        else if constexpr (scatter_mode<MODE>()) fast_mid<T, R0, EM, M>(ln, tws, 1, tl, tpl);
-        else fast_first_pre_lds<T, R0, EM, M, MODE>(a, ln, tws, tl, tpl);
-        if constexpr (R2 != 0) fast_mid<T, R1, EM, M>(ln, tws + a.twoff[1], R0, tl, tpl);
-        fast_mid<T, RL, EM, M>(ln, tws + a.twoff[R2 ? 2 : 1], M / RL, tl, tpl);
-        if (act) {
-            // the generic kernel's store (column side: consecutive threads
-            // on consecutive lines, or on consecutive line pairs)
-            if (a.out_col && (a.flags & F_CPAIR_OUT)) {
-                const int hl = lt >> 1;
-                store_line_pair<T, 2, NT, MODE>(a, data, tws, tile, 2 * (tid % hl), tid / hl, 2 * tpl);
-            } else {
-                const int lo = a.out_col ? tid % lt : l, k0 = a.out_col ? tid / lt : tl;
-                store_line<T, 2, NT, MODE>(a, data, tws, tile, lo, k0, tpl);
-            }
-        }
-        return;
+    if (mode == M_C2R) {
+        fast_c2r_load<T, M, NT>(a, data, tws, tile, tid, l, tl);
+        fast_mid<T, R0, EM, M>(ln, tws, 1, tl, tpl);
     } else {
-        const bool dht = KIND == 1 && mode == M_DHT;
-        if (mode == M_C2R) {
-            fast_c2r_load<T, M, NT>(a, data, tws, tile, tid, l, tl);
-            fast_mid<T, R0, EM, M>(ln, tws, 1, tl, tpl);
-        } else {
-            // column access: lanes across the tile's lines; row access: along a line
-            const int fl = !act ? 0 : (a.in_col ? tid % lt : l);
-            const int ft = !act ? (1 << 28) : (a.in_col ? tid / lt : tl);
-            const int64_t line = tile * lt + fl;
-            int64_t io = 0, oo = 0;
-            const bool valid = act && line < a.nlines;
-            if (valid) line_offsets(a.g, line, io, oo);
-            fast_first<T, R0, EM, M, NT>(a, data + fl * a.ls, valid, io, ft, tpl, mode == M_C2C,
-                                         (a.flags & F_CONJ_IN) != 0);
-        }
-        if constexpr (R2 != 0) fast_mid<T, R1, EM, M>(ln, tws + a.twoff[1], R0, tl, tpl);
-        if (mode == M_R2C || dht) {
-            fast_mid<T, RL, EM, M>(ln, tws + a.twoff[R2 ? 2 : 1], M / RL, tl, tpl);
-            if (act) {
-                if (mode == M_R2C) fast_r2c_store<T, NT>(a, data, tws, tile, tid, l, tl);
-                else fast_dht_store<T, NT>(a, data, tws, tile, tid, l, tl);
-            }
-            return;
-        }
-        const int fl = !act ? 0 : (a.out_col ? tid % lt : l);
-        const int ft = !act ? (1 << 28) : (a.out_col ? tid / lt : tl);
+        // column access: lanes across the tile's lines; row access: along a line
+        const int fl = !act ? 0 : (a.in_col ? tid % lt : l);
+        const int ft = !act ? (1 << 28) : (a.in_col ? tid / lt : tl);
         const int64_t line = tile * lt + fl;
         int64_t io = 0, oo = 0;
         const bool valid = act && line < a.nlines;
         if (valid) line_offsets(a.g, line, io, oo);
-        fast_last<T, RL, EM, M, NT>(a, data + fl * a.ls, tws + a.twoff[R2 ? 2 : 1], valid, oo, ft, tpl,
-                                    mode == M_C2R);
+        fast_first<T, R0, EM, M, NT>(a, data + fl * a.ls, valid, io, ft, tpl, mode == M_C2C,
+                                     (a.flags & F_CONJ_IN) != 0);
     }
+    if constexpr (R2 != 0) fast_mid<T, R1, EM, M>(ln, tws + a.twoff[1], R0, tl, tpl);
+    if (mode == M_R2C) {
+        fast_mid<T, RL, EM, M>(ln, tws + a.twoff[R2 ? 2 : 1], M / RL, tl, tpl);
+        if (act) fast_r2c_store<T, NT>(a, data, tws, tile, tid, l, tl);
+        return;
+    }
+    const int fl = !act ? 0 : (a.out_col ? tid % lt : l);
+    const int ft = !act ? (1 << 28) : (a.out_col ? tid / lt : tl);
+    const int64_t line = tile * lt + fl;
+    int64_t io = 0, oo = 0;
+    const bool valid = act && line < a.nlines;
+    if (valid) line_offsets(a.g, line, io, oo);
+    fast_last<T, RL, EM, M, NT>(a, data + fl * a.ls, tws + a.twoff[R2 ? 2 : 1], valid, oo, ft, tpl,
+                                mode == M_C2R);
 }
 
-template <typename T, int R0, int R1, int R2, int EM, bool NT, int KIND = 1, int MODE = -1>
+template <typename T, int R0, int R1, int R2, int EM, bool NT>
 __global__ __launch_bounds__(512) void k_line_fast(const StageArgs<T> a)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -1538,7 +1193,7 @@ __global__ __launch_bounds__(512) void k_line_fast(const StageArgs<T> a)
         if (tile >= a.ntiles) return;
     }
     for (int i = tid; i < a.twn; i += nthr) tws[i] = a.tw[i];
-    fast_body<T, R0, R1, R2, EM, NT, KIND, MODE>(a, tile, tws, tws + a.twn);
+    fast_body<T, R0, R1, R2, EM, NT>(a, tile, tws, tws + a.twn);
 }
 
 // Persistent batched fast stage: the work list of k_line_batch, every item
@@ -1568,7 +1223,7 @@ __global__ __launch_bounds__(512) void k_line_fast_batch(const StageArgs<T> *__r
         const int64_t tile = w - prefix[q];
         __syncthreads(); // the previous tile is done with LDS
         for (int i = tid; i < a.twn; i += nthr) tws[i] = a.tw[i];
-        fast_body<T, R0, R1, R2, EM, false, 0>(a, tile, tws, tws + a.twn);
+        fast_body<T, R0, R1, R2, EM, false>(a, tile, tws, tws + a.twn);
     }
 }
 
@@ -1606,7 +1261,7 @@ __global__ __launch_bounds__(512) void k_line_multi_batch(const StageArgs<T> *__
 #define PFH_MULTI_CASE(TT, A, B, C, E)                                                                        \
     if constexpr (std::is_same<T, TT>::value && E != 32) {                                                   \
         if (r0 == A && r1 == B && r2 == C && em == E) {                                                      \
-            fast_body<T, A, B, C, E, false, 0>(a, tile, tws, tws + a.twn);                                  \
+            fast_body<T, A, B, C, E, false>(a, tile, tws, tws + a.twn);                                  \
             continue;                                                                                        \
         }                                                                                                    \
     }
@@ -1620,32 +1275,14 @@ hipError_t launch_line_fast(const StageArgs<T> &a, int r0, int r1, int r2, int e
                             int64_t grid, hipStream_t s)
 {
     if (grid <= 0) return hipSuccess;
-    // real-input R2R modes: their own instantiation, ordinary accesses; the
-    // plans and modes of PFH_R2R_MODE_PLANS also with the mode as a
-    // compile-time constant
-    const bool r2r = !(a.mode == M_C2C || a.mode == M_R2C || a.mode == M_C2R || a.mode == M_DHT);
-    static const bool mode_kernels = [] {
-        const char *e = std::getenv("PFH_R2R_MODE_KERNELS");
-        return e == nullptr || std::atoi(e) != 0;
-    }();
-    if (r2r && mode_kernels) {
-#define PFH_MODE_CASE(TT, A, B, C, E, MD)                                                                     \
-        if constexpr (std::is_same<T, TT>::value)                                                             \
-            if (r0 == A && r1 == B && r2 == C && em == E && a.mode == MD) {                                   \
-                hipLaunchKernelGGL((k_line_fast<T, A, B, C, E, false, 2, MD>), dim3((unsigned)grid),          \
-                                   dim3(threads), lds_bytes, s, a);                                           \
-                return hipGetLastError();                                                                     \
-            }
-        PFH_R2R_MODE_PLANS(PFH_MODE_CASE)
-#undef PFH_MODE_CASE
+    if (a.flags & F_LINE_PLAN) {
+        if (a.mode == M_C2C) return launch_line_plan<T, 0>(a, r0, r1, r2, em, threads, lds_bytes, grid, s);
+        if (a.mode == M_R2C || a.mode == M_C2R || a.mode == M_DHT)
+            return launch_line_plan<T, 1>(a, r0, r1, r2, em, threads, lds_bytes, grid, s);
+        return launch_line_plan<T, 2>(a, r0, r1, r2, em, threads, lds_bytes, grid, s);
     }
 #define PFH_FAST_CASE(TT, A, B, C, E)                                                                           \
     if constexpr (std::is_same<T, TT>::value) if (r0 == A && r1 == B && r2 == C && em == E) {                               \
-        if (r2r) {                                                                                              \
-            hipLaunchKernelGGL((k_line_fast<T, A, B, C, E, false, 2>), dim3((unsigned)grid), dim3(threads),     \
-                               lds_bytes, s, a);                                                                \
-            return hipGetLastError();                                                                           \
-        }                                                                                                       \
         if (a.flags & F_NT)                                                                                     \
             hipLaunchKernelGGL((k_line_fast<T, A, B, C, E, true>), dim3((unsigned)grid), dim3(threads), lds_bytes, \
                                s, a);                                                                           \
@@ -1655,7 +1292,6 @@ hipError_t launch_line_fast(const StageArgs<T> &a, int r0, int r1, int r2, int e
         return hipGetLastError();                                                                               \
     }
     PFH_FAST_PLANS(PFH_FAST_CASE)
-    PFH_FAST_ROUTE_PLANS(PFH_FAST_CASE)
 #undef PFH_FAST_CASE
     return hipErrorInvalidValue;
 }
@@ -1681,7 +1317,6 @@ bool fast_plan_available(int tbytes, int r0, int r1, int r2, int em)
 #define PFH_FAST_HAS(TT, A, B, C, E) \
     if ((int)sizeof(TT) == tbytes && r0 == A && r1 == B && r2 == C && em == E) return true;
     PFH_FAST_PLANS(PFH_FAST_HAS)
-    PFH_FAST_ROUTE_PLANS(PFH_FAST_HAS)
 #undef PFH_FAST_HAS
     return false;
 }
@@ -1710,31 +1345,6 @@ hipError_t set_fast_lds_limit(size_t bytes)
     }
     PFH_FAST_PLANS(PFH_FAST_ATTR)
 #undef PFH_FAST_ATTR
-#define PFH_FAST_ATTR_ROUTE(TT, A, B, C, E)                                                              \
-    {                                                                                                     \
-        hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(&k_line_fast<TT, A, B, C, E, false>), bytes); \
-        if (e == hipSuccess)                                                                              \
-            e = raise_lds_limit(reinterpret_cast<const void *>(&k_line_fast<TT, A, B, C, E, true>), bytes); \
-        if (e != hipSuccess) return e;                                                                    \
-    }
-    PFH_FAST_ROUTE_PLANS(PFH_FAST_ATTR_ROUTE)
-#undef PFH_FAST_ATTR_ROUTE
-#define PFH_FAST_ATTR_R2R(TT, A, B, C, E)                                                                \
-    {                                                                                                     \
-        hipError_t e = raise_lds_limit(reinterpret_cast<const void *>(&k_line_fast<TT, A, B, C, E, false, 2>), bytes); \
-        if (e != hipSuccess) return e;                                                                    \
-    }
-    PFH_FAST_PLANS(PFH_FAST_ATTR_R2R)
-    PFH_FAST_ROUTE_PLANS(PFH_FAST_ATTR_R2R)
-#undef PFH_FAST_ATTR_R2R
-#define PFH_FAST_ATTR_MODE(TT, A, B, C, E, MD)                                                           \
-    {                                                                                                     \
-        hipError_t e =                                                                                    \
-            raise_lds_limit(reinterpret_cast<const void *>(&k_line_fast<TT, A, B, C, E, false, 2, MD>), bytes); \
-        if (e != hipSuccess) return e;                                                                    \
-    }
-    PFH_R2R_MODE_PLANS(PFH_FAST_ATTR_MODE)
-#undef PFH_FAST_ATTR_MODE
     return hipSuccess;
 }
 

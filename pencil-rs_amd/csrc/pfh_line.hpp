@@ -1,0 +1,43 @@
+// Compile-time line plans: the radix sequence, the threads per line and the
+// LDS layout of k_line_plan (pfh_line.hip), shared with the host planner.
+#pragma once
+
+#include "pfh_stage.hpp"
+
+namespace pfh {
+
+// Butterflies of radix R a thread holds in one pass (em values per thread).
+__host__ __device__ constexpr int line_plan_mb(int em, int R) { return em / R > 0 ? em / R : 1; }
+
+__host__ __device__ constexpr int line_plan_need(int m, int em, int R)
+{
+    return (m / R + line_plan_mb(em, R) - 1) / line_plan_mb(em, R);
+}
+
+// Threads per line: the fewest that cover every pass's butterflies. Any
+// number, not a power of two: the 385-point line of a DST-I takes 39 threads,
+// of which the radix 5 / 7 / 11 passes keep 99 / 71 / 90% busy (64 threads:
+// 60 / 86 / 55%).
+__host__ __device__ constexpr int line_plan_tpl(int r0, int r1, int r2, int em)
+{
+    const int m = r0 * r1 * (r2 ? r2 : 1);
+    int t = line_plan_need(m, em, r0);
+    if (line_plan_need(m, em, r1) > t) t = line_plan_need(m, em, r1);
+    if (r2 && line_plan_need(m, em, r2) > t) t = line_plan_need(m, em, r2);
+    return t;
+}
+
+// LDS stride of a line (complex values, odd): between passes the line is kept
+// as m / r0 rows of r0 values at the odd row stride r0 | 1, before the first
+// and after the last pass as m (+ 1) values in natural order.
+__host__ __device__ constexpr int line_plan_stride(int r0, int r1, int r2)
+{
+    const int m = r0 * r1 * (r2 ? r2 : 1);
+    const int rows = m / r0 * (r0 | 1);
+    return (rows > m + 1 ? rows : m + 1) | 1;
+}
+
+// Most threads of a workgroup of k_line_plan.
+constexpr int kLinePlanThreads = 512;
+
+} // namespace pfh

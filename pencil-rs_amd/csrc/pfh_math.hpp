@@ -327,6 +327,71 @@ struct Dft<T, 16> {
     }
 };
 
+// N = A x B with coprime A and B (Good-Thomas): input B n1 + A n2 mod N,
+// output k with k mod A, k mod B; the A- and B-point butterflies need no
+// twiddles between them.
+template <typename T, int A, int B>
+struct DftCoprime {
+    __host__ __device__ static __forceinline__ void run(cpx<T> *v)
+    {
+        constexpr int N = A * B;
+        cpx<T> t[A][B];
+#pragma unroll
+        for (int n2 = 0; n2 < B; ++n2) {
+            cpx<T> c[A];
+#pragma unroll
+            for (int n1 = 0; n1 < A; ++n1) c[n1] = v[(B * n1 + A * n2) % N];
+            Dft<T, A>::run(c);
+#pragma unroll
+            for (int k1 = 0; k1 < A; ++k1) t[k1][n2] = c[k1];
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < A; ++k1) Dft<T, B>::run(t[k1]);
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = t[k % A][k % B];
+    }
+};
+template <typename T>
+struct Dft<T, 6> : DftCoprime<T, 2, 3> {};
+template <typename T>
+struct Dft<T, 10> : DftCoprime<T, 2, 5> {};
+template <typename T>
+struct Dft<T, 12> : DftCoprime<T, 4, 3> {};
+template <typename T>
+struct Dft<T, 14> : DftCoprime<T, 2, 7> {};
+template <typename T>
+struct Dft<T, 15> : DftCoprime<T, 3, 5> {};
+
+template <typename T>
+struct Dft<T, 9> {
+    __host__ __device__ static __forceinline__ void run(cpx<T> *v)
+    {
+        // j = r1 + 3 r2, k = k2 + 3 k1; twiddles exp(-2 pi i r1 k2 / 9)
+        constexpr double c1 = 0.76604444311897803520239265055541668, s1 = 0.64278760968653932632264340990726343;
+        constexpr double c2 = 0.17364817766693034885171662676931479, s2 = 0.98480775301220805936674302458952301;
+        constexpr double c4 = -0.93969262078590838405410927732473147, s4 = 0.34202014332566873304409961468225959;
+        cpx<T> t[3][3];
+#pragma unroll
+        for (int r1 = 0; r1 < 3; ++r1) {
+            cpx<T> c[3] = {v[r1], v[r1 + 3], v[r1 + 6]};
+            Dft<T, 3>::run(c);
+#pragma unroll
+            for (int k2 = 0; k2 < 3; ++k2) t[r1][k2] = c[k2];
+        }
+        t[1][1] = cmul(t[1][1], mk((T)c1, (T)-s1));
+        t[1][2] = cmul(t[1][2], mk((T)c2, (T)-s2));
+        t[2][1] = cmul(t[2][1], mk((T)c2, (T)-s2));
+        t[2][2] = cmul(t[2][2], mk((T)c4, (T)-s4));
+#pragma unroll
+        for (int k2 = 0; k2 < 3; ++k2) {
+            cpx<T> c[3] = {t[0][k2], t[1][k2], t[2][k2]};
+            Dft<T, 3>::run(c);
+#pragma unroll
+            for (int k1 = 0; k1 < 3; ++k1) v[k2 + 3 * k1] = c[k1];
+        }
+    }
+};
+
 // exp(-2 pi i e / 32) = (W32c(e), -W32s(e)), e = 0..21
 __host__ __device__ inline double W32c(int e)
 {

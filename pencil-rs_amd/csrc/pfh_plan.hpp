@@ -92,6 +92,9 @@ struct Step {
     bool fast = false;
     int fr[3] = {0, 0, 0};
     int fem = 16;
+    bool line_plan = false; // fast runs k_line_plan (radices and em of a line plan)
+    int64_t big_bytes = 0;  // larger of the stage's arrays in bytes (0: not known when planned)
+    int64_t io_bytes = 0;   // their sum
     int digit_axis[kMaxDigits] = {-1, -1, -1, -1, -1}; // logical axis of each line digit (-1: extras)
     // Long lines: a stage whose line does not fit one workgroup (or whose
     // FFT length has a large prime factor) runs as `pieces`, in order; a
@@ -147,6 +150,8 @@ struct Tuning {
     int block = 0;       // target threads per block (0: 256)
     int block_cap = 0;   // upper bound on threads per block (0: the kernel's launch bound)
     bool allow_fast = true;
+    bool allow_line_plan = true; // route and local stages on k_line_plan (the batched kernels carry
+                                 // the plans of PFH_FAST_PLANS only)
     bool allow_xcd = true;
     int slab_mb = -1;    // slab intermediate target in MiB (0: no slab pipelining, -1: default)
     bool fill_block = false; // column-access tiles also take `block` threads (batched launches)

@@ -1,0 +1,106 @@
+"""GPU parity of the compile-time line plans (pfh_line.hip): every planned
+length on row lines with a partial last tile, and routes whose stages take
+column sides with partial tiles, in every mode, against numpy / the oracle.
+Bounds: the suite's 2e-6 (f32) and 1e-12 (f64) relative L2, which hold for
+these lengths with a rounding error of a few eps per radix pass; 4x over the
+three stages of a route."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+import pencil_fft_hip as pf
+from util import complex_of, rel_l2, tol, uniform_complex, uniform_real
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [np.float32, np.float64]
+OPS = [O.FORWARD, O.INVERSE, O.BACKWARD, O.ADJ_FORWARD, O.ADJ_INVERSE, O.ADJ_BACKWARD]
+
+
+def _smooth(n):
+    for p in (2, 3, 5, 7):
+        while n % p == 0:
+            n //= p
+    return n == 1
+
+
+LENGTHS = [n for n in range(8, 513) if _smooth(n)] + [385]
+
+
+def _tdev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _host(t):
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+def test_every_length_c2c_and_half_length_real(gpu, dt):
+    rng = np.random.default_rng(31)
+    for n in LENGTHS:
+        lines = 256 // n * 2 + 7  # a partial last tile
+        x = uniform_complex(rng, (lines, n), complex_of(dt))
+        plan = pf.LocalC2cPlan(n, dtype=torch.from_numpy(x).dtype)
+        got = _host(plan.forward(_tdev(x)))
+        assert rel_l2(got, np.fft.fft(x.astype(np.complex128))) <= tol(dt), n
+        got = _host(plan.inverse(_tdev(x)))
+        assert rel_l2(got, np.fft.ifft(x.astype(np.complex128))) <= tol(dt), n
+        r = uniform_real(rng, (lines, 2 * n), dt)
+        rplan = pf.LocalR2cPlan(2 * n, dtype=torch.from_numpy(r).dtype)
+        spec = rplan.forward(_tdev(r))
+        assert rel_l2(_host(spec), np.fft.rfft(r.astype(np.float64))) <= tol(dt), n
+        assert rel_l2(_host(rplan.inverse(spec)), r) <= 2 * tol(dt), n
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("kind", list(range(1, 10)))
+def test_real_kinds_on_row_lines(gpu, kind, dt):
+    """n, n / 2, 2n, n - 1 or n + 1 is a planned length: even and odd lines,
+    both parities of the half length, forward and inverse."""
+    rng = np.random.default_rng(kind)
+    for n in (16, 17, 19, 24, 30, 45, 50, 64, 65, 63, 75, 126, 129, 180, 225, 240, 256, 384, 385, 512):
+        x = uniform_real(rng, (11, n), dt)
+        td = torch.from_numpy(x).dtype
+        plan = pf.LocalDhtPlan(n, dtype=td) if kind == 9 else pf.LocalR2rPlan(n, kind, dtype=td)
+        for op, fn in ((O.FORWARD, plan.forward), (O.INVERSE, plan.inverse)):
+            ref = O.r2r_lines(x.astype(np.float64), kind, op)
+            assert rel_l2(_host(fn(_tdev(x))), ref) <= tol(dt), (n, kind, op)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("permute", [True, False])
+@pytest.mark.parametrize("kinds", [(1, 2, 3), (4, 5, 6), (7, 8, 9), (9, 1, 5)])
+def test_real_kinds_on_column_sides(gpu, kinds, permute, dt):
+    shape = (25, 36, 49)
+    rng = np.random.default_rng(sum(kinds))
+    td = torch.float32 if dt == np.float32 else torch.float64
+    plan = pf.R2rPlan(shape, list(kinds), dtype=td, extra_shape=(2,), permute_dims=permute)
+    x = uniform_real(rng, 2 * int(np.prod(shape)), dt)
+    for op in OPS:
+        ref = O.transform(O.KIND_R2R, x.astype(np.float64), op, shape=shape, extra=2, r2r=list(kinds),
+                          permute_dims=permute)
+        assert rel_l2(_host(plan.execute(op, _tdev(x))), ref) <= 4 * tol(dt), op
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("permute", [True, False])
+@pytest.mark.parametrize("shape", [(35, 27, 90), (50, 15, 28), (9, 200, 18)])
+def test_complex_and_half_complex_routes(gpu, shape, permute, dt):
+    rng = np.random.default_rng(shape[0])
+    td = torch.float32 if dt == np.float32 else torch.float64
+    cd = torch.complex64 if dt == np.float32 else torch.complex128
+    n = 3 * int(np.prod(shape))
+    for kind, plan in ((O.KIND_C2C, pf.C2cPlan(shape, dtype=cd, extra_shape=(3,), permute_dims=permute)),
+                       (O.KIND_R2C, pf.R2cPlan(shape, dtype=td, extra_shape=(3,), permute_dims=permute))):
+        x = uniform_complex(rng, n, complex_of(dt)) if kind == O.KIND_C2C else uniform_real(rng, n, dt)
+        wide = x.astype(np.complex128 if kind == O.KIND_C2C else np.float64)
+        spec = O.transform(kind, wide, O.FORWARD, shape=shape, extra=3, permute_dims=permute)
+        for op in OPS:
+            fwd_like = op in (O.FORWARD, O.ADJ_INVERSE, O.ADJ_BACKWARD)
+            src = x if fwd_like else spec.astype(complex_of(dt))
+            ref = O.transform(kind, src.astype(np.complex128 if np.iscomplexobj(src) else np.float64), op,
+                              shape=shape, extra=3, permute_dims=permute)
+            assert rel_l2(_host(plan.execute(op, _tdev(src))), ref) <= 4 * tol(dt), (kind, op)
