@@ -342,16 +342,21 @@ static int env_int(const char *name, int dflt)
 // The line plan (k_line_plan) of an FFT length; radices 0 if there is none.
 static void find_line_plan(int m, int tbytes, int r[3], int &em)
 {
+    using Entry = std::array<int, 4>;
+    static const std::map<int, Entry> plans[2] = {
+#define PFH_LINE_F32(TT, A, B, C, E) {sizeof(TT) == 4 ? (A) * (B) * ((C) ? (C) : 1) : 0, {A, B, C, E}},
+#define PFH_LINE_F64(TT, A, B, C, E) {sizeof(TT) == 8 ? (A) * (B) * ((C) ? (C) : 1) : 0, {A, B, C, E}},
+        {PFH_FAST_ROUTE_PLANS(PFH_LINE_F32)},
+        {PFH_FAST_ROUTE_PLANS(PFH_LINE_F64)},
+#undef PFH_LINE_F32
+#undef PFH_LINE_F64
+    };
     r[0] = 0;
-#define PFH_LINE_FIND(TT, A, B, C, E)                                                \
-    if ((int)sizeof(TT) == tbytes && (A) * (B) * ((C) ? (C) : 1) == m) {            \
-        r[0] = A;                                                                    \
-        r[1] = B;                                                                    \
-        r[2] = C;                                                                    \
-        em = E;                                                                      \
-    }
-    PFH_FAST_ROUTE_PLANS(PFH_LINE_FIND)
-#undef PFH_LINE_FIND
+    const std::map<int, Entry> &t = plans[tbytes == 4 ? 0 : 1];
+    const auto it = t.find(m);
+    if (m < 2 || it == t.end()) return;
+    for (int i = 0; i < 3; ++i) r[i] = it->second[i];
+    em = it->second[3];
 }
 
 // k_line_plan for a stage whose mode and FFT length it has: radices, values
@@ -367,6 +372,7 @@ static bool choose_line_plan(Step &st, int tbytes)
                      st.mode == M_DCT3 || st.mode == M_DCT3_ODD || st.mode == M_DCT4 || st.mode == M_DCT4_ODD ||
                      st.mode == M_DHT_ODD;
     if (!(st.mode == M_C2C || st.mode == M_R2C || st.mode == M_C2R || dht || r2r)) return false;
+    if (r2r && st.m > kLinePlanRealMax) return false;
     int r[3], em = 0;
     find_line_plan(st.m, tbytes, r, em);
     if (r[0] == 0) return false;
@@ -884,13 +890,14 @@ static bool wants_pieces(const Step &s)
 
 // Pass tables of a radix split (roots of generic radices, then the pass
 // twiddles), offsets relative to the block; appended to tab when non-null.
-static int pass_tables(const std::vector<int> &radices, std::vector<double> *tab, std::array<int, kMaxPasses> &twoff)
+static int pass_tables(const std::vector<int> &radices, std::vector<double> *tab, std::array<int, kMaxPasses> &twoff,
+                       bool line_plan = false)
 {
     int off = 0, Ns = 1;
     for (size_t p = 0; p < radices.size(); ++p) {
         const int R = radices[p];
         twoff[p] = off;
-        if (is_generic_radix(R)) {
+        if (!line_plan && is_generic_radix(R)) {
             if (tab)
                 for (int e = 0; e < R; ++e) push_cexp(*tab, e, R);
             off += R;
@@ -923,8 +930,8 @@ static pfh_status plan_table(PlanImpl &P, const std::string &name, int64_t &offs
     return PFH_OK;
 }
 
-// Forward DFT of a 5-smooth length in long double (decimation in time over
-// the factors 2, 3, 5; w = exp(-2 pi i e / n) for the full length n).
+// Forward DFT of a 7-smooth length in long double (decimation in time over
+// the factors 2, 3, 5, 7; w = exp(-2 pi i e / n) for the full length n).
 using cxl = std::complex<long double>;
 static void host_dft_rec(const cxl *in, size_t stride, cxl *out, size_t len, const std::vector<cxl> &w, size_t wstep)
 {
@@ -932,7 +939,7 @@ static void host_dft_rec(const cxl *in, size_t stride, cxl *out, size_t len, con
         out[0] = in[0];
         return;
     }
-    const size_t p = (len % 2 == 0) ? 2 : (len % 3 == 0) ? 3 : (len % 5 == 0) ? 5 : len;
+    const size_t p = (len % 2 == 0) ? 2 : (len % 3 == 0) ? 3 : (len % 5 == 0) ? 5 : (len % 7 == 0) ? 7 : len;
     const size_t q = len / p;
     if (p == len) {
         for (size_t k = 0; k < len; ++k) {
@@ -943,7 +950,7 @@ static void host_dft_rec(const cxl *in, size_t stride, cxl *out, size_t len, con
         return;
     }
     for (size_t r = 0; r < p; ++r) host_dft_rec(in + r * stride, stride * p, out + r * q, q, w, wstep * p);
-    cxl t[5];
+    cxl t[7];
     for (size_t k = 0; k < q; ++k) {
         for (size_t r = 0; r < p; ++r) t[r] = out[r * q + k];
         for (size_t s = 0; s < p; ++s) {
@@ -977,9 +984,9 @@ static cxl chirp(int64_t j, int64_t m, int s)
     return cxl(cosl(a), sinl(a));
 }
 
-static bool five_smooth(int64_t v)
+static bool seven_smooth(int64_t v)
 {
-    for (int p : {2, 3, 5})
+    for (int p : {2, 3, 5, 7})
         while (v % p == 0) v /= p;
     return v == 1;
 }
@@ -1008,10 +1015,25 @@ static bool piece_fits(int64_t m, const DeviceInfo &dev, int tb, const Tuning &t
     return fits;
 }
 
-// N1 (the first piece's length) of a split N1 x N2 = m whose pieces both
-// fit one workgroup, N1 as close to sqrt(m) as the divisors allow; 0: none.
-static int64_t split_factor(int64_t m, const DeviceInfo &dev, int tb, const Tuning &tu)
+// Does a C2C piece of this length run on k_line_plan?
+static bool has_line_plan(int64_t m, int tb, const Tuning &tu)
 {
+    if (!tu.allow_fast || !tu.allow_line_plan || m < 1 || m > INT32_MAX) return false;
+    Step p;
+    p.mode = M_C2C;
+    p.m = (int)m;
+    return choose_line_plan(p, tb);
+}
+
+// N1 (the first piece's length) of a split N1 x N2 = m whose pieces both
+// fit one workgroup: the most pieces with a line plan, then N1 as close to
+// sqrt(m) as the divisors allow; 0: none.
+static int64_t split_factor(PlanImpl &P, int64_t m, int tb)
+{
+    const DeviceInfo &dev = P.dev;
+    const Tuning &tu = P.tuning;
+    const auto memo = P.split_memo.find(m);
+    if (memo != P.split_memo.end()) return memo->second;
     int64_t best = 0;
     double best_d = 1e300;
     for (int64_t a = 2; a * a <= m; ++a) {
@@ -1019,51 +1041,73 @@ static int64_t split_factor(int64_t m, const DeviceInfo &dev, int tb, const Tuni
         for (int64_t n1 : {a, m / a}) {
             const int64_t n2 = m / n1;
             if (!piece_fits(n1, dev, tb, tu) || !piece_fits(n2, dev, tb, tu)) continue;
-            const double d = std::fabs(std::log((double)n1) - 0.5 * std::log((double)m));
+            const int plans = (has_line_plan(n1, tb, tu) ? 1 : 0) + (has_line_plan(n2, tb, tu) ? 1 : 0);
+            const double d = std::fabs(std::log((double)n1) - 0.5 * std::log((double)m)) - 100.0 * plans;
             if (d < best_d) {
                 best_d = d;
                 best = n1;
             }
         }
     }
+    P.split_memo[m] = best;
     return best;
 }
 
-// Radix passes of a generic line stage of length len.
-static int radix_passes(int64_t len, int tb, const Tuning &tu)
+// Relative cost per value of one piece of length len: a line plan streams at
+// about 4.5 TB/s on MI355X with two radix passes and at 3.6 with three, the
+// generic kernel at about 1.8 TB/s with four and in proportion to them.
+static double piece_cost(int64_t len, int tb, const Tuning &tu)
 {
+    int lp[3], em = 0;
+    find_line_plan((int)len, tb, lp, em);
+    if (has_line_plan(len, tb, tu)) return lp[2] ? 1.25 : 1.0;
     std::vector<int> r;
     const int max_r = tu.max_radix ? tu.max_radix : (tb == 4 ? 16 : 8);
-    return radix_plan((int)len, r, max_r) ? (int)r.size() : 64;
+    return radix_plan((int)len, r, max_r) ? std::max(1.0, 0.62 * (double)r.size()) : 64.0;
+}
+
+// Does an FFT of length m that fits one generic stage run faster as a split
+// into two line plans?
+static bool split_pays(PlanImpl &P, int64_t m, int tb, int64_t &n1)
+{
+    const Tuning &tu = P.tuning;
+    n1 = 0;
+    if (has_line_plan(m, tb, tu)) return false;
+    n1 = split_factor(P, m, tb);
+    return n1 > 0 && piece_cost(n1, tb, tu) + piece_cost(m / n1, tb, tu) < piece_cost(m, tb, tu);
 }
 
 // Length of Bluestein's cyclic convolution for an FFT of length m: a
-// 5-smooth M >= 2m - 1 that runs as one piece or a split, the one with the
-// fewest M x (radix passes of its pieces) among those up to 25% above the
-// smallest. For m = 10007: 20480 = 128 x 160 (2 + 3 passes) rather than
-// 20250 = 135 x 150 (4 + 4 passes).
-static int64_t bluestein_length(int64_t m, const DeviceInfo &dev, int tb, const Tuning &tu)
+// 7-smooth M >= 2m - 1 that runs as one piece or a split, the cheapest (M x
+// the cost of its pieces) among those up to 25% above the smallest. For m =
+// 10007: 20160 = 140 x 144, two passes each.
+static int64_t bluestein_length(PlanImpl &P, int64_t m, int tb)
 {
+    const Tuning &tu = P.tuning;
+    const auto memo = P.bluestein_memo.find(m);
+    if (memo != P.bluestein_memo.end()) return memo->second;
     int64_t best = 0;
     double best_cost = 0;
     const int64_t lo = 2 * m - 1;
     for (int64_t M = lo; M <= 4 * m && M <= ((int64_t)1 << 25); ++M) {
         if (best && (double)M > 1.25 * (double)lo) break;
-        if (!five_smooth(M)) continue;
-        int passes = 0;
-        if (piece_fits(M, dev, tb, tu)) {
-            passes = radix_passes(M, tb, tu);
+        if (!seven_smooth(M)) continue;
+        double cost;
+        int64_t n1 = 0;
+        if (piece_fits(M, P.dev, tb, tu) && !split_pays(P, M, tb, n1)) {
+            cost = piece_cost(M, tb, tu);
         } else {
-            const int64_t n1 = split_factor(M, dev, tb, tu);
+            if (n1 <= 0) n1 = split_factor(P, M, tb);
             if (n1 <= 0) continue;
-            passes = radix_passes(n1, tb, tu) + radix_passes(M / n1, tb, tu);
+            cost = piece_cost(n1, tb, tu) + piece_cost(M / n1, tb, tu);
         }
-        const double cost = (double)M * passes;
+        cost *= (double)M;
         if (!best || cost < best_cost) {
             best = M;
             best_cost = cost;
         }
     }
+    P.bluestein_memo[m] = best;
     return best;
 }
 
@@ -1115,9 +1159,16 @@ static pfh_status twiddle_table(PlanImpl &P, int64_t M, int64_t &off, int &bsh)
     });
 }
 
-// One generic C2C line stage of length N over the given digits.
+// Splits up to this length keep all their twiddles in one table (8 MiB f32 at
+// 2^20), read along neighbouring lines: one rounding and one load per value;
+// longer ones multiply three table entries.
+constexpr int64_t kFullTwiddles = 1 << 20;
+
+// One C2C line stage of length N over the given digits: a line plan where the
+// length has one and every array of the piece (big_bytes the largest) is
+// below 4 GiB, else the generic kernel.
 static pfh_status make_piece(PlanImpl &P, Step &p, int64_t N, std::vector<PieceDigit> digs, int64_t ips,
-                             int64_t ops, int in_buf, int out_buf, const PieceX &x, int tb)
+                             int64_t ops, int in_buf, int out_buf, const PieceX &x, int tb, int64_t big_bytes)
 {
     p = Step();
     p.mode = M_C2C;
@@ -1126,13 +1177,52 @@ static pfh_status make_piece(PlanImpl &P, Step &p, int64_t N, std::vector<PieceD
     p.flags = x.flags;
     p.scale = x.scale;
     const int max_r = P.tuning.max_radix ? P.tuning.max_radix : (tb == 4 ? 16 : 8);
-    if (!radix_plan((int)N, p.radices, max_r)) return set_err(PFH_ERR_UNSUPPORTED, "long-line piece radix plan");
+    p.big_bytes = big_bytes;
+    if (!(P.tuning.allow_fast && P.tuning.allow_line_plan && choose_line_plan(p, tb)) &&
+        !radix_plan((int)N, p.radices, max_r))
+        return set_err(PFH_ERR_UNSUPPORTED, "long-line piece radix plan");
     int64_t base = 0;
     std::array<int, kMaxPasses> twoff{};
-    const int twn = pass_tables(p.radices, nullptr, twoff);
-    pfh_status st = plan_table(P, "pass:" + std::to_string(N) + ":" + std::to_string(max_r), base,
-                               [&](std::vector<double> &t) { pass_tables(p.radices, &t, twoff); });
+    const int twn = pass_tables(p.radices, nullptr, twoff, p.line_plan);
+    pfh_status st = plan_table(P, "pass:" + std::to_string(N) + ":" + (p.line_plan ? "line" : std::to_string(max_r)),
+                               base, [&](std::vector<double> &t) { pass_tables(p.radices, &t, twoff, p.line_plan); });
     if (st) return st;
+    if (p.line_plan && (x.flags & F_XTW)) {
+        const int RL = p.radices.back();
+        const int64_t n2 = x.tw_m / N;
+        p.xtw_full = x.tw_m <= kFullTwiddles;
+        if (p.xtw_full)
+            st = plan_table(P, "twf:" + std::to_string(N) + ":" + std::to_string(n2), p.xtwr,
+                            [&](std::vector<double> &t) {
+                                // products of two long-double tables: a trigonometric call per entry would take
+                                // 0.2 s for 2^20 entries
+                                int64_t B = 1;
+                                while (B * B < x.tw_m) B *= 2;
+                                std::vector<cxl> lo((size_t)B), hi((size_t)(x.tw_m / B + 1));
+                                auto root = [&](int64_t q) {
+                                    const long double a = -2.0L * kPiL * (long double)q / (long double)x.tw_m;
+                                    return cxl(cosl(a), sinl(a));
+                                };
+                                for (int64_t q = 0; q < B; ++q) lo[(size_t)q] = root(q);
+                                for (size_t h = 0; h < hi.size(); ++h) hi[h] = root((int64_t)h * B);
+                                t.reserve(t.size() + 2 * (size_t)x.tw_m);
+                                for (int64_t k = 0; k < N; ++k)
+                                    for (int64_t d = 0; d < n2; ++d) {
+                                        const int64_t q = k * d;
+                                        const cxl a = lo[(size_t)(q % B)], b = hi[(size_t)(q / B)];
+                                        t.push_back((double)(a.real() * b.real() - a.imag() * b.imag()));
+                                        t.push_back((double)(a.real() * b.imag() + a.imag() * b.real()));
+                                    }
+                            });
+        else
+            st = plan_table(P, "twr:" + std::to_string(RL) + ":" + std::to_string(n2), p.xtwr,
+                            [&](std::vector<double> &t) {
+                                for (int r = 0; r < RL; ++r)
+                                    for (int64_t d = 0; d < n2; ++d)
+                                        push_cexp(t, (long long)r * d, (long long)RL * n2);
+                            });
+        if (st) return st;
+    }
     p.tw_base = base;
     p.twn = twn;
     p.twoff = twoff;
@@ -1187,7 +1277,9 @@ static pfh_status fft_pieces(PlanImpl &P, const Step &outer, int64_t N, const Li
                              std::vector<Step> &pieces)
 {
     const int nd = outer.g.nd;
-    if (piece_fits(N, P.dev, tb, P.tuning)) {
+    const int64_t big = std::max(outer.big_bytes, outer.nlines * N * 2 * tb);
+    int64_t split = 0;
+    if (piece_fits(N, P.dev, tb, P.tuning) && !split_pays(P, N, tb, split)) {
         std::vector<PieceDigit> digs;
         for (int d = 0; d < nd; ++d) digs.push_back({outer.g.ext[d], in.dig[d], out.dig[d], false});
         PieceX x = xout;
@@ -1197,12 +1289,12 @@ static pfh_status fft_pieces(PlanImpl &P, const Step &outer, int64_t N, const Li
         x.valid_in = xin.valid_in;
         x.mul_out = 1;
         Step p;
-        pfh_status st = make_piece(P, p, N, digs, in.point, out.point, in.buf, out.buf, x, tb);
+        pfh_status st = make_piece(P, p, N, digs, in.point, out.point, in.buf, out.buf, x, tb, big);
         if (st) return st;
         pieces.push_back(p);
         return PFH_OK;
     }
-    const int64_t N1 = split_factor(N, P.dev, tb, P.tuning);
+    const int64_t N1 = split_factor(P, N, tb);
     if (N1 <= 0) return set_err(PFH_ERR_UNSUPPORTED, "no split of the long line into workgroup pieces");
     const int64_t N2 = N / N1;
     const LineSide rs = region_side(outer, rs_buf, N);
@@ -1221,7 +1313,7 @@ static pfh_status fft_pieces(PlanImpl &P, const Step &outer, int64_t N, const Li
         if (st) return st;
         x.tw_m = (int)N;
         Step p;
-        st = make_piece(P, p, N1, digs, N2 * in.point, N2, in.buf, rs_buf, x, tb);
+        st = make_piece(P, p, N1, digs, N2 * in.point, N2, in.buf, rs_buf, x, tb, big);
         if (st) return st;
         pieces.push_back(p);
     }
@@ -1234,7 +1326,7 @@ static pfh_status fft_pieces(PlanImpl &P, const Step &outer, int64_t N, const Li
         x.flags = xout.flags & (F_CONJ_OUT | F_XOUT);
         x.mul_out = (int)N1;
         Step p;
-        pfh_status st = make_piece(P, p, N2, digs, 1, N1 * out.point, rs_buf, out.buf, x, tb);
+        pfh_status st = make_piece(P, p, N2, digs, 1, N1 * out.point, rs_buf, out.buf, x, tb, big);
         if (st) return st;
         pieces.push_back(p);
     }
@@ -1264,7 +1356,7 @@ static pfh_status core_pieces(PlanImpl &P, const Step &outer, int64_t m, const L
         xo.valid_out = (int)m;
         return fft_pieces(P, outer, m, in, out, xi, xo, rs_buf, xb, tb, pieces);
     }
-    const int64_t M = bluestein_length(m, P.dev, tb, P.tuning);
+    const int64_t M = bluestein_length(P, m, tb);
     if (M <= 0) return set_err(PFH_ERR_UNSUPPORTED, "no Bluestein length for this line");
     const int s = (conj & F_CONJ_IN) ? 1 : -1;
     int64_t c_off = 0, bh_off = 0;
@@ -2468,6 +2560,7 @@ static StageArgs<T> fill_args(const PlanImpl &P, const Step &s, void *const bufs
     a.xtab_in = s.xtab_in >= 0 ? tabs + s.xtab_in : nullptr;
     a.xtab_out = s.xtab_out >= 0 ? tabs + s.xtab_out : nullptr;
     a.xtw = s.xtw >= 0 ? tabs + s.xtw : nullptr;
+    a.xtwr = s.xtwr >= 0 ? tabs + s.xtwr : nullptr;
     a.xdig = s.xdig;
     a.xmul_in = s.xmul_in;
     a.xmul_out = s.xmul_out;
@@ -2475,6 +2568,7 @@ static StageArgs<T> fill_args(const PlanImpl &P, const Step &s, void *const bufs
     a.xvalid_out = s.xvalid_out;
     a.xtw_m = s.xtw_m;
     a.xtw_bsh = s.xtw_bsh;
+    a.xtw_full = s.xtw_full;
     return a;
 }
 
@@ -2587,6 +2681,11 @@ static pfh_status launch_pieces(const PlanImpl &P, const Step &s, void *const bu
             sp.in_buf = 0;
             sp.out_buf = 1;
             const StageArgs<T> a = fill_args<T>(P, sp, io, gate);
+            if (pc.fast) {
+                PFH_HIP_CHECK(launch_line_fast<T>(a, pc.fr[0], pc.fr[1], pc.fr[2], pc.fem, pc.threads, pc.lds_bytes,
+                                                  pc.grid, stream));
+                continue;
+            }
             bool wide = false;
             for (int R : pc.radices) wide = wide || is_wide_radix(R);
             PFH_HIP_CHECK(launch_line_stage<T>(a, wide, pc.threads, pc.lds_bytes, pc.grid, stream));
@@ -3214,8 +3313,11 @@ static pfh_status local_execute_impl(pfh_plan plan, int op, const void *src, siz
                                                                   wv.first_code, wv.gate, wv.status, stream));
             }
         }
-        for (int64_t c0 = 0; c0 < batch; c0 += tmpl.long_lines) {
-            const int64_t cnt = std::min<int64_t>(tmpl.long_lines, batch - c0);
+        // (chunks of equal size: a short last chunk costs its launches)
+        const int64_t nchunk = (batch + tmpl.long_lines - 1) / tmpl.long_lines;
+        const int64_t per = nchunk > 0 ? (batch + nchunk - 1) / nchunk : 1;
+        for (int64_t c0 = 0; c0 < batch; c0 += per) {
+            const int64_t cnt = std::min<int64_t>(per, batch - c0);
             // the chunk's pieces are planned once per (op, cnt): planning them
             // (factorizations, the Bluestein length search, piece sizing)
             // took about 0.2 ms of host time per call for 10007-point lines

@@ -86,7 +86,8 @@ template <typename T>
 hipError_t launch_line_fast(const StageArgs<T> &a, int r0, int r1, int r2, int em, int threads, size_t lds_bytes,
                             int64_t grid, hipStream_t s);
 // Stages with a line plan (pfh_line.hip, F_LINE_PLAN set). KIND 0: C2C, 1:
-// R2C / C2R / DHT of even length, 2: the other real-to-real modes.
+// R2C / C2R / DHT of even length, 2: the other real-to-real modes, 3: C2C
+// pieces of long lines.
 // launch_line_fast dispatches to them.
 template <typename T, int KIND>
 hipError_t launch_line_plan(const StageArgs<T> &a, int r0, int r1, int r2, int em, int threads, size_t lds_bytes,
@@ -101,6 +102,8 @@ PFH_LINE_DECLARE(float, 2)
 PFH_LINE_DECLARE(double, 0)
 PFH_LINE_DECLARE(double, 1)
 PFH_LINE_DECLARE(double, 2)
+PFH_LINE_DECLARE(float, 3)
+PFH_LINE_DECLARE(double, 3)
 #undef PFH_LINE_DECLARE
 bool fast_plan_available(int tbytes, int r0, int r1, int r2, int em);
 bool multi_batch_plan_available(int tbytes, int r0, int r1, int r2, int em);

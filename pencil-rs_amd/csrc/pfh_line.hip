@@ -77,6 +77,21 @@ __device__ __forceinline__ void gwrite(void *base, uint32_t off, V v)
     *reinterpret_cast<V *>(static_cast<char *>(base) + off) = v;
 }
 
+// Coordinate of line digit xdig of a line (pieces of long lines).
+__device__ __forceinline__ uint32_t line_digit(const LineGeom &g, uint32_t line, int xdig)
+{
+    uint32_t x = line, c = 0;
+#pragma unroll
+    for (int d = 0; d < kMaxDigits; ++d) {
+        if (d < g.nd) {
+            const uint32_t q = fastdiv(x, g.dmag[d], g.dsh[d]);
+            if (d == xdig) c = x - q * (uint32_t)g.ext[d];
+            x = q;
+        }
+    }
+    return c;
+}
+
 __device__ __forceinline__ bool complex_in(int mode) { return mode == M_C2C || mode == M_C2R; }
 __device__ __forceinline__ bool complex_out(int mode) { return mode == M_C2C || mode == M_R2C; }
 
@@ -527,7 +542,8 @@ __device__ __forceinline__ void merge_dct3(const StageArgs<T> &a, typename P::V 
 } // namespace
 
 // KIND 0: C2C lines; 1: R2C / C2R / DHT lines of even length (the half-length
-// transform of real pairs); 2: the other real-to-real modes.
+// transform of real pairs); 2: the other real-to-real modes; 3: C2C pieces of
+// long lines (load and store factors, zero padding, crop, split twiddles).
 // Lines past the end of the last tile repeat the last line's loads and store
 // nothing.
 template <typename T, int R0, int R1, int R2, int EM, int KIND>
@@ -574,7 +590,56 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
     const V *twl = tws + a.twoff[R2 ? 2 : 1];
     const bool cj = (a.flags & F_CONJ_IN) != 0;
 
-    if constexpr (KIND == 0) {
+    // pieces of long lines: coordinates of the line digit that the factors and
+    // full indexes run over (iline, oline may be relative to the tile)
+    uint32_t idco = 0, odco = 0;
+    if constexpr (KIND == 3) {
+        if (a.xdig >= 0) {
+            const uint32_t last = nlines - 1;
+            idco = line_digit(a.g, tile0 + (uint32_t)il < nlines ? tile0 + (uint32_t)il : last, a.xdig);
+            odco = line_digit(a.g, tile0 + (uint32_t)ol < nlines ? tile0 + (uint32_t)ol : last, a.xdig);
+        }
+    }
+    if constexpr (KIND == 3) {
+        constexpr int N0 = P::template rounds<R0>(), NB0 = M / R0;
+        cpx<T> v[N0][R0];
+        const uint32_t st = (uint32_t)a.ips * (uint32_t)(2 * sizeof(T));
+        const uint32_t off = line_offset<false>(a.g, iline, 2 * sizeof(T)) + (uint32_t)it * st;
+        const bool pad = (a.flags & F_XIN) != 0;
+        const uint32_t fmul = (uint32_t)a.xmul_in, f0 = idco + (uint32_t)it * fmul, fend = (uint32_t)a.xvalid_in;
+#pragma unroll
+        for (int b = 0; b < N0; ++b) {
+            if (P::template has<R0>(b, it + TPL * b)) {
+#pragma unroll
+                for (int r = 0; r < R0; ++r) {
+                    const uint32_t p = (uint32_t)(b * TPL + r * NB0);
+                    v[b][r] = mk((T)0, (T)0);
+                    if (!pad || f0 + p * fmul < fend) v[b][r] = gread<cpx<T>>(src, off + p * st);
+                }
+            }
+        }
+        stage_tables();
+        if (cj) {
+#pragma unroll
+            for (int b = 0; b < N0; ++b)
+#pragma unroll
+                for (int r = 0; r < R0; ++r) v[b][r].y = -v[b][r].y;
+        }
+        if (pad && a.xtab_in != nullptr) {
+#pragma unroll
+            for (int b = 0; b < N0; ++b) {
+                if (P::template has<R0>(b, it + TPL * b)) {
+#pragma unroll
+                    for (int r = 0; r < R0; ++r) {
+                        const uint32_t f = f0 + (uint32_t)(b * TPL + r * NB0) * fmul;
+                        if (f < fend) v[b][r] = cmul(v[b][r], gread<cpx<T>>(a.xtab_in, f * (uint32_t)(2 * sizeof(T))));
+                    }
+                }
+            }
+        }
+        P::first_store(iln, it, v);
+        P::mid(iln, tw1, it);
+    } else if constexpr (KIND == 0) {
         constexpr int N0 = P::template rounds<R0>(), NB0 = M / R0;
         cpx<T> v[N0][R0];
         const uint32_t st = (uint32_t)a.ips * (uint32_t)(2 * sizeof(T));
@@ -683,7 +748,57 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
     }
 
     const T sc = a.scale;
-    if constexpr (KIND == 0) {
+    if constexpr (KIND == 3) {
+        constexpr int NL = P::template rounds<RL>(), NB = M / RL;
+        if (!store) return;
+        cpx<T> v[NL][RL];
+        P::last(oln, twl, ot, v);
+        const uint32_t st = (uint32_t)a.ops * (uint32_t)(2 * sizeof(T));
+        const uint32_t off = line_offset<true>(a.g, oline, 2 * sizeof(T)) + (uint32_t)ot * st;
+        if (a.flags & F_XTW) {
+            // exp(-2 pi i d k / (m n2)), k = j + r NB: neighbouring lines d read
+            // neighbouring table entries
+            const uint32_t n2 = (uint32_t)(a.xtw_m / M), lo = (1u << a.xtw_bsh) - 1u;
+            const V *hi = reinterpret_cast<const V *>(a.xtw) + lo + 1;
+#pragma unroll
+            for (int b = 0; b < NL; ++b) {
+                const int j = ot + TPL * b;
+                if (P::template has<RL>(b, j)) {
+                    if (a.xtw_full) {
+                        const uint32_t w0 = ((uint32_t)j * n2 + odco) * (uint32_t)(2 * sizeof(T));
+#pragma unroll
+                        for (int r = 0; r < RL; ++r)
+                            v[b][r] = cmul(v[b][r], gread<cpx<T>>(a.xtwr, w0 + (uint32_t)(r * NB) * n2 * (uint32_t)(2 * sizeof(T))));
+                    } else {
+                        const uint32_t q = odco * (uint32_t)j;
+                        const cpx<T> w = cmul(get<T>(reinterpret_cast<const V *>(a.xtw) + (q & lo)), get<T>(hi + (q >> a.xtw_bsh)));
+                        v[b][0] = cmul(v[b][0], w);
+#pragma unroll
+                        for (int r = 1; r < RL; ++r)
+                            v[b][r] = cmul(v[b][r], cmul(w, gread<cpx<T>>(a.xtwr, ((uint32_t)r * n2 + odco) * (uint32_t)(2 * sizeof(T)))));
+                    }
+                }
+            }
+        }
+        const T sy = (a.flags & F_CONJ_OUT) ? -sc : sc;
+        const bool crop = (a.flags & F_XOUT) != 0;
+        const uint32_t fmul = (uint32_t)a.xmul_out, f0 = odco + (uint32_t)ot * fmul, fend = (uint32_t)a.xvalid_out;
+#pragma unroll
+        for (int b = 0; b < NL; ++b) {
+            if (P::template has<RL>(b, ot + TPL * b)) {
+#pragma unroll
+                for (int r = 0; r < RL; ++r) {
+                    const uint32_t p = (uint32_t)(b * TPL + r * NB), f = f0 + p * fmul;
+                    cpx<T> w = mk(v[b][r].x * sc, v[b][r].y * sy);
+                    if (crop) {
+                        if (f >= fend) continue;
+                        if (a.xtab_out != nullptr) w = cmul(w, gread<cpx<T>>(a.xtab_out, f * (uint32_t)(2 * sizeof(T))));
+                    }
+                    gwrite<cpx<T>>(dst, off + p * st, w);
+                }
+            }
+        }
+    } else if constexpr (KIND == 0) {
         constexpr int NL = P::template rounds<RL>(), NB = M / RL;
         if (!store) return;
         cpx<T> v[NL][RL];
@@ -804,7 +919,8 @@ hipError_t launch_line_plan<LineT, PFH_LINE_KIND>(const StageArgs<LineT> &a, int
                                                   size_t lds_bytes, int64_t grid, hipStream_t s)
 {
 #define PFH_LINE_CASE(TT, A, B, C, E)                                                                      \
-    if constexpr (sizeof(TT) == sizeof(LineT))                                                             \
+    if constexpr (sizeof(TT) == sizeof(LineT) &&                                                           \
+                  (PFH_LINE_KIND != 2 || (A) * (B) * ((C) ? (C) : 1) <= kLinePlanRealMax))                 \
         if (r0 == A && r1 == B && r2 == C && em == E)                                                      \
             return launch_one<LineT, A, B, C, E, PFH_LINE_KIND>(a, threads, lds_bytes, grid, s);
     PFH_FAST_ROUTE_PLANS(PFH_LINE_CASE)

@@ -37,6 +37,9 @@ __host__ __device__ constexpr int line_plan_stride(int r0, int r1, int r2)
     return (rows > m + 1 ? rows : m + 1) | 1;
 }
 
+// Longest FFT length of the real-to-real modes' plans (other than DHT).
+constexpr int kLinePlanRealMax = 512;
+
 // Most threads of a workgroup of k_line_plan.
 constexpr int kLinePlanThreads = 512;
 

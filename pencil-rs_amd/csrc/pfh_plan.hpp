@@ -104,8 +104,8 @@ struct Step {
     std::vector<Step> pieces;
     int launch = 0;
     int long_kind = 0;
-    int64_t xtab_in = -1, xtab_out = -1, xtw = -1; // table offsets (complex entries), -1: none
-    int xdig = -1, xmul_in = 1, xmul_out = 1, xvalid_in = 0, xvalid_out = 0, xtw_m = 0, xtw_bsh = 0;
+    int64_t xtab_in = -1, xtab_out = -1, xtw = -1, xtwr = -1; // table offsets (complex entries), -1: none
+    int xdig = -1, xmul_in = 1, xmul_out = 1, xvalid_in = 0, xvalid_out = 0, xtw_m = 0, xtw_bsh = 0, xtw_full = 0;
 };
 
 // Two consecutive steps run slab by slab over an axis that neither
@@ -182,6 +182,9 @@ struct PlanImpl {
     // twiddle/pre/post tables of every step of every op, one device buffer
     std::vector<double> host_tables; // complex pairs, f64
     std::map<std::string, int64_t> table_index; // long-line tables already in host_tables (name -> offset)
+    // long-line choices already made by this plan (length -> split, Bluestein
+    // length): a local plan expands its chunks again at its first executes
+    std::map<int64_t, int64_t> split_memo, bluestein_memo;
     bool tables_frozen = false;                 // host_tables uploaded: no table may be added
     void *dev_tables = nullptr;
     int64_t table_entries = 0;

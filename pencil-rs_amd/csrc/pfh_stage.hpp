@@ -165,6 +165,10 @@ struct StageArgs {
     int xmul_in, xmul_out;
     int xvalid_in, xvalid_out;
     int xtw_m, xtw_bsh;
+    // k_line_plan: the split's twiddles at [k][d], exp(-2 pi i d k / xtw_m), d < n2 = xtw_m / m (xtw_full), or
+    // at [r][d], exp(-2 pi i d r / (RL n2)), r < RL (the last radix), a factor of the two-level table's
+    const cpx<T> *xtwr;
+    int xtw_full;
 };
 
 // Pre- and post-processing of a long real line (k_long_prep / k_long_post,
@@ -217,212 +221,282 @@ struct PlaneArgs {
 
 // Line plans {R0, R1, R2, EM}: the radix sequence and the values per thread
 // and pass of the route stages that k_line_plan runs (pfh_line.hip): every
-// length 2^a 3^b 5^c 7^d from 8 to 512 that three radices up to 16 reach, and
+// length 2^a 3^b 5^c 7^d from 8 to 1024 that three radices up to 16 reach, and
 // the 385-point FFT of a DST-I line of 384 points. Of the splits of a length
 // the one with the fewest lane instructions is taken, idle lanes of partial
 // passes and about 14 per value and LDS exchange included; lengths below 64
 // keep at most 8 values per thread, so that a wave still covers long runs.
 #define PFH_FAST_ROUTE_PLANS(X) \
-    X(float, 2, 4, 0, 4)      \
-    X(float, 3, 3, 0, 3)      \
-    X(float, 2, 5, 0, 6)      \
-    X(float, 2, 6, 0, 6)      \
-    X(float, 2, 7, 0, 8)      \
-    X(float, 3, 5, 0, 6)      \
-    X(float, 4, 4, 0, 4)      \
-    X(float, 3, 6, 0, 6)      \
-    X(float, 4, 5, 0, 5)      \
-    X(float, 3, 7, 0, 7)      \
-    X(float, 4, 6, 0, 8)      \
-    X(float, 5, 5, 0, 5)      \
-    X(float, 3, 3, 3, 3)      \
-    X(float, 4, 7, 0, 8)      \
-    X(float, 5, 6, 0, 6)      \
-    X(float, 4, 8, 0, 8)      \
-    X(float, 5, 7, 0, 7)      \
-    X(float, 6, 6, 0, 6)      \
-    X(float, 5, 8, 0, 8)      \
-    X(float, 6, 7, 0, 7)      \
-    X(float, 3, 3, 5, 6)      \
-    X(float, 6, 8, 0, 8)      \
-    X(float, 7, 7, 0, 7)      \
-    X(float, 2, 5, 5, 6)      \
-    X(float, 3, 3, 6, 6)      \
-    X(float, 7, 8, 0, 8)      \
-    X(float, 2, 5, 6, 6)      \
-    X(float, 3, 3, 7, 7)      \
-    X(float, 8, 8, 0, 8)      \
-    X(float, 5, 14, 0, 15)    \
-    X(float, 6, 12, 0, 12)    \
-    X(float, 5, 15, 0, 15)    \
-    X(float, 8, 10, 0, 10)    \
-    X(float, 9, 9, 0, 9)      \
-    X(float, 7, 12, 0, 14)    \
-    X(float, 9, 10, 0, 10)    \
-    X(float, 8, 12, 0, 16)    \
-    X(float, 7, 14, 0, 14)    \
-    X(float, 10, 10, 0, 10)   \
-    X(float, 7, 15, 0, 15)    \
-    X(float, 9, 12, 0, 12)    \
-    X(float, 8, 14, 0, 16)    \
-    X(float, 8, 15, 0, 16)    \
-    X(float, 5, 5, 5, 5)      \
-    X(float, 3, 3, 14, 15)    \
-    X(float, 8, 16, 0, 16)    \
-    X(float, 3, 3, 15, 15)    \
-    X(float, 10, 14, 0, 14)   \
-    X(float, 12, 12, 0, 12)   \
-    X(float, 3, 7, 7, 15)     \
-    X(float, 10, 15, 0, 15)   \
-    X(float, 10, 16, 0, 16)   \
-    X(float, 2, 9, 9, 10)     \
-    X(float, 12, 14, 0, 14)   \
-    X(float, 5, 5, 7, 15)     \
-    X(float, 12, 15, 0, 15)   \
-    X(float, 3, 7, 9, 9)      \
-    X(float, 12, 16, 0, 16)   \
-    X(float, 14, 14, 0, 14)   \
-    X(float, 2, 10, 10, 10)   \
-    X(float, 14, 15, 0, 15)   \
-    X(float, 3, 6, 12, 12)    \
-    X(float, 14, 16, 0, 16)   \
-    X(float, 15, 15, 0, 15)   \
-    X(float, 15, 16, 0, 16)   \
-    X(float, 3, 9, 9, 9)      \
-    X(float, 5, 7, 7, 15)     \
-    X(float, 5, 5, 10, 10)    \
-    X(float, 3, 7, 12, 14)    \
-    X(float, 16, 16, 0, 16)   \
-    X(float, 3, 9, 10, 10)    \
-    X(float, 4, 5, 14, 16)    \
-    X(float, 2, 12, 12, 12)   \
-    X(float, 3, 7, 14, 15)    \
-    X(float, 4, 5, 15, 16)    \
-    X(float, 3, 7, 15, 15)    \
-    X(float, 5, 8, 8, 16)     \
-    X(float, 3, 9, 12, 12)    \
-    X(float, 4, 7, 12, 14)    \
-    X(float, 7, 7, 7, 7)      \
-    X(float, 5, 5, 14, 15)    \
-    X(float, 3, 8, 15, 16)    \
-    X(float, 5, 5, 15, 15)    \
-    X(float, 3, 9, 14, 14)    \
-    X(float, 3, 8, 16, 16)    \
-    X(float, 5, 7, 11, 14)    \
-    X(float, 2, 14, 14, 14)   \
-    X(float, 4, 10, 10, 12)   \
-    X(float, 5, 9, 9, 10)     \
-    X(float, 2, 14, 15, 15)   \
-    X(float, 3, 12, 12, 12)   \
-    X(float, 7, 7, 9, 9)      \
-    X(float, 2, 14, 16, 16)   \
-    X(float, 2, 15, 15, 16)   \
-    X(float, 4, 8, 15, 16)    \
-    X(float, 6, 9, 9, 12)     \
-    X(float, 5, 7, 14, 15)    \
-    X(float, 5, 10, 10, 10)   \
-    X(float, 6, 7, 12, 14)    \
-    X(float, 8, 8, 8, 16)     \
-    X(double, 2, 4, 0, 4)     \
-    X(double, 3, 3, 0, 3)     \
-    X(double, 2, 5, 0, 6)     \
-    X(double, 2, 6, 0, 6)     \
-    X(double, 2, 7, 0, 8)     \
-    X(double, 3, 5, 0, 6)     \
-    X(double, 4, 4, 0, 4)     \
-    X(double, 3, 6, 0, 6)     \
-    X(double, 4, 5, 0, 5)     \
-    X(double, 3, 7, 0, 7)     \
-    X(double, 4, 6, 0, 8)     \
-    X(double, 5, 5, 0, 5)     \
-    X(double, 3, 3, 3, 3)     \
-    X(double, 4, 7, 0, 8)     \
-    X(double, 5, 6, 0, 6)     \
-    X(double, 4, 8, 0, 8)     \
-    X(double, 5, 7, 0, 7)     \
-    X(double, 6, 6, 0, 6)     \
-    X(double, 5, 8, 0, 8)     \
-    X(double, 6, 7, 0, 7)     \
-    X(double, 3, 3, 5, 6)     \
-    X(double, 6, 8, 0, 8)     \
-    X(double, 7, 7, 0, 7)     \
-    X(double, 2, 5, 5, 6)     \
-    X(double, 3, 3, 6, 6)     \
-    X(double, 7, 8, 0, 8)     \
-    X(double, 2, 5, 6, 6)     \
-    X(double, 3, 3, 7, 7)     \
-    X(double, 8, 8, 0, 8)     \
-    X(double, 5, 14, 0, 15)   \
-    X(double, 6, 12, 0, 12)   \
-    X(double, 5, 15, 0, 15)   \
-    X(double, 8, 10, 0, 10)   \
-    X(double, 9, 9, 0, 9)     \
-    X(double, 7, 12, 0, 14)   \
-    X(double, 9, 10, 0, 10)   \
-    X(double, 8, 12, 0, 16)   \
-    X(double, 7, 14, 0, 14)   \
-    X(double, 10, 10, 0, 10)  \
-    X(double, 7, 15, 0, 15)   \
-    X(double, 9, 12, 0, 12)   \
-    X(double, 8, 14, 0, 16)   \
-    X(double, 8, 15, 0, 16)   \
-    X(double, 5, 5, 5, 5)     \
-    X(double, 3, 3, 14, 15)   \
-    X(double, 8, 16, 0, 16)   \
-    X(double, 3, 3, 15, 15)   \
-    X(double, 10, 14, 0, 14)  \
-    X(double, 12, 12, 0, 12)  \
-    X(double, 3, 7, 7, 15)    \
-    X(double, 10, 15, 0, 15)  \
-    X(double, 10, 16, 0, 16)  \
-    X(double, 2, 9, 9, 10)    \
-    X(double, 12, 14, 0, 14)  \
-    X(double, 5, 5, 7, 15)    \
-    X(double, 12, 15, 0, 15)  \
-    X(double, 3, 7, 9, 9)     \
-    X(double, 12, 16, 0, 16)  \
-    X(double, 14, 14, 0, 14)  \
-    X(double, 2, 10, 10, 10)  \
-    X(double, 14, 15, 0, 15)  \
-    X(double, 3, 6, 12, 12)   \
-    X(double, 14, 16, 0, 16)  \
-    X(double, 15, 15, 0, 15)  \
-    X(double, 15, 16, 0, 16)  \
-    X(double, 3, 9, 9, 9)     \
-    X(double, 5, 7, 7, 15)    \
-    X(double, 5, 5, 10, 10)   \
-    X(double, 3, 7, 12, 14)   \
-    X(double, 16, 16, 0, 16)  \
-    X(double, 3, 9, 10, 10)   \
-    X(double, 4, 5, 14, 16)   \
-    X(double, 2, 12, 12, 12)  \
-    X(double, 3, 7, 14, 15)   \
-    X(double, 4, 5, 15, 16)   \
-    X(double, 3, 7, 15, 15)   \
-    X(double, 5, 8, 8, 16)    \
-    X(double, 3, 9, 12, 12)   \
-    X(double, 4, 7, 12, 14)   \
-    X(double, 7, 7, 7, 7)     \
-    X(double, 5, 5, 14, 15)   \
-    X(double, 3, 8, 15, 16)   \
-    X(double, 5, 5, 15, 15)   \
-    X(double, 3, 9, 14, 14)   \
-    X(double, 3, 8, 16, 16)   \
-    X(double, 5, 7, 11, 14)   \
-    X(double, 2, 14, 14, 14)  \
-    X(double, 4, 10, 10, 12)  \
-    X(double, 5, 9, 9, 10)    \
-    X(double, 2, 14, 15, 15)  \
-    X(double, 3, 12, 12, 12)  \
-    X(double, 7, 7, 9, 9)     \
-    X(double, 2, 14, 16, 16)  \
-    X(double, 2, 15, 15, 16)  \
-    X(double, 4, 8, 15, 16)   \
-    X(double, 6, 9, 9, 12)    \
-    X(double, 5, 7, 14, 15)   \
-    X(double, 5, 10, 10, 10)  \
-    X(double, 6, 7, 12, 14)   \
-    X(double, 8, 8, 8, 16)   
+    X(float, 2, 4, 0, 4)       \
+    X(float, 3, 3, 0, 3)       \
+    X(float, 2, 5, 0, 6)       \
+    X(float, 2, 6, 0, 6)       \
+    X(float, 2, 7, 0, 8)       \
+    X(float, 3, 5, 0, 6)       \
+    X(float, 4, 4, 0, 4)       \
+    X(float, 3, 6, 0, 6)       \
+    X(float, 4, 5, 0, 5)       \
+    X(float, 3, 7, 0, 7)       \
+    X(float, 4, 6, 0, 8)       \
+    X(float, 5, 5, 0, 5)       \
+    X(float, 3, 3, 3, 3)       \
+    X(float, 4, 7, 0, 8)       \
+    X(float, 5, 6, 0, 6)       \
+    X(float, 4, 8, 0, 8)       \
+    X(float, 5, 7, 0, 7)       \
+    X(float, 6, 6, 0, 6)       \
+    X(float, 5, 8, 0, 8)       \
+    X(float, 6, 7, 0, 7)       \
+    X(float, 3, 3, 5, 6)       \
+    X(float, 6, 8, 0, 8)       \
+    X(float, 7, 7, 0, 7)       \
+    X(float, 2, 5, 5, 6)       \
+    X(float, 3, 3, 6, 6)       \
+    X(float, 7, 8, 0, 8)       \
+    X(float, 2, 5, 6, 6)       \
+    X(float, 3, 3, 7, 7)       \
+    X(float, 8, 8, 0, 8)       \
+    X(float, 5, 14, 0, 15)     \
+    X(float, 6, 12, 0, 12)     \
+    X(float, 5, 15, 0, 15)     \
+    X(float, 8, 10, 0, 10)     \
+    X(float, 9, 9, 0, 9)       \
+    X(float, 7, 12, 0, 14)     \
+    X(float, 9, 10, 0, 10)     \
+    X(float, 8, 12, 0, 16)     \
+    X(float, 7, 14, 0, 14)     \
+    X(float, 10, 10, 0, 10)    \
+    X(float, 7, 15, 0, 15)     \
+    X(float, 9, 12, 0, 12)     \
+    X(float, 8, 14, 0, 16)     \
+    X(float, 8, 15, 0, 16)     \
+    X(float, 5, 5, 5, 5)       \
+    X(float, 3, 3, 14, 15)     \
+    X(float, 8, 16, 0, 16)     \
+    X(float, 3, 3, 15, 15)     \
+    X(float, 10, 14, 0, 14)    \
+    X(float, 12, 12, 0, 12)    \
+    X(float, 3, 7, 7, 15)      \
+    X(float, 10, 15, 0, 15)    \
+    X(float, 10, 16, 0, 16)    \
+    X(float, 2, 9, 9, 10)      \
+    X(float, 12, 14, 0, 14)    \
+    X(float, 5, 5, 7, 15)      \
+    X(float, 12, 15, 0, 15)    \
+    X(float, 3, 7, 9, 9)       \
+    X(float, 12, 16, 0, 16)    \
+    X(float, 14, 14, 0, 14)    \
+    X(float, 2, 10, 10, 10)    \
+    X(float, 14, 15, 0, 15)    \
+    X(float, 3, 6, 12, 12)     \
+    X(float, 14, 16, 0, 16)    \
+    X(float, 15, 15, 0, 15)    \
+    X(float, 15, 16, 0, 16)    \
+    X(float, 3, 9, 9, 9)       \
+    X(float, 5, 7, 7, 15)      \
+    X(float, 5, 5, 10, 10)     \
+    X(float, 3, 7, 12, 14)     \
+    X(float, 16, 16, 0, 16)    \
+    X(float, 3, 9, 10, 10)     \
+    X(float, 4, 5, 14, 16)     \
+    X(float, 2, 12, 12, 12)    \
+    X(float, 3, 7, 14, 15)     \
+    X(float, 4, 5, 15, 16)     \
+    X(float, 3, 7, 15, 15)     \
+    X(float, 5, 8, 8, 16)      \
+    X(float, 3, 9, 12, 12)     \
+    X(float, 4, 7, 12, 14)     \
+    X(float, 7, 7, 7, 7)       \
+    X(float, 5, 5, 14, 15)     \
+    X(float, 3, 8, 15, 16)     \
+    X(float, 5, 5, 15, 15)     \
+    X(float, 3, 9, 14, 14)     \
+    X(float, 3, 8, 16, 16)     \
+    X(float, 5, 7, 11, 14)     \
+    X(float, 2, 14, 14, 14)    \
+    X(float, 4, 10, 10, 12)    \
+    X(float, 5, 9, 9, 10)      \
+    X(float, 2, 14, 15, 15)    \
+    X(float, 3, 12, 12, 12)    \
+    X(float, 7, 7, 9, 9)       \
+    X(float, 2, 14, 16, 16)    \
+    X(float, 2, 15, 15, 16)    \
+    X(float, 4, 8, 15, 16)     \
+    X(float, 6, 9, 9, 12)      \
+    X(float, 5, 7, 14, 15)     \
+    X(float, 5, 10, 10, 10)    \
+    X(float, 6, 7, 12, 14)     \
+    X(float, 8, 8, 8, 16)      \
+    X(float, 5, 7, 15, 15)     \
+    X(float, 3, 12, 15, 15)    \
+    X(float, 5, 8, 14, 16)     \
+    X(float, 7, 9, 9, 14)      \
+    X(float, 4, 12, 12, 12)    \
+    X(float, 3, 14, 14, 15)    \
+    X(float, 5, 8, 15, 16)     \
+    X(float, 3, 14, 15, 15)    \
+    X(float, 5, 8, 16, 16)     \
+    X(float, 8, 9, 9, 9)       \
+    X(float, 4, 12, 14, 14)    \
+    X(float, 3, 15, 15, 15)    \
+    X(float, 7, 7, 14, 14)     \
+    X(float, 7, 10, 10, 14)    \
+    X(float, 3, 15, 16, 16)    \
+    X(float, 9, 9, 9, 9)       \
+    X(float, 7, 7, 15, 15)     \
+    X(float, 5, 10, 15, 15)    \
+    X(float, 7, 9, 12, 14)     \
+    X(float, 3, 16, 16, 16)    \
+    X(float, 4, 14, 14, 16)    \
+    X(float, 8, 10, 10, 10)    \
+    X(float, 9, 9, 10, 10)     \
+    X(float, 4, 14, 15, 16)    \
+    X(float, 6, 12, 12, 12)    \
+    X(float, 7, 9, 14, 14)     \
+    X(float, 8, 8, 14, 16)     \
+    X(float, 4, 15, 15, 16)    \
+    X(float, 7, 9, 15, 15)     \
+    X(float, 8, 8, 15, 16)     \
+    X(float, 9, 9, 12, 12)     \
+    X(float, 5, 14, 14, 15)    \
+    X(float, 10, 10, 10, 10)   \
+    X(float, 7, 12, 12, 14)    \
+    X(float, 8, 8, 16, 16)     \
+    X(double, 2, 4, 0, 4)      \
+    X(double, 3, 3, 0, 3)      \
+    X(double, 2, 5, 0, 6)      \
+    X(double, 2, 6, 0, 6)      \
+    X(double, 2, 7, 0, 8)      \
+    X(double, 3, 5, 0, 6)      \
+    X(double, 4, 4, 0, 4)      \
+    X(double, 3, 6, 0, 6)      \
+    X(double, 4, 5, 0, 5)      \
+    X(double, 3, 7, 0, 7)      \
+    X(double, 4, 6, 0, 8)      \
+    X(double, 5, 5, 0, 5)      \
+    X(double, 3, 3, 3, 3)      \
+    X(double, 4, 7, 0, 8)      \
+    X(double, 5, 6, 0, 6)      \
+    X(double, 4, 8, 0, 8)      \
+    X(double, 5, 7, 0, 7)      \
+    X(double, 6, 6, 0, 6)      \
+    X(double, 5, 8, 0, 8)      \
+    X(double, 6, 7, 0, 7)      \
+    X(double, 3, 3, 5, 6)      \
+    X(double, 6, 8, 0, 8)      \
+    X(double, 7, 7, 0, 7)      \
+    X(double, 2, 5, 5, 6)      \
+    X(double, 3, 3, 6, 6)      \
+    X(double, 7, 8, 0, 8)      \
+    X(double, 2, 5, 6, 6)      \
+    X(double, 3, 3, 7, 7)      \
+    X(double, 8, 8, 0, 8)      \
+    X(double, 5, 14, 0, 15)    \
+    X(double, 6, 12, 0, 12)    \
+    X(double, 5, 15, 0, 15)    \
+    X(double, 8, 10, 0, 10)    \
+    X(double, 9, 9, 0, 9)      \
+    X(double, 7, 12, 0, 14)    \
+    X(double, 9, 10, 0, 10)    \
+    X(double, 8, 12, 0, 16)    \
+    X(double, 7, 14, 0, 14)    \
+    X(double, 10, 10, 0, 10)   \
+    X(double, 7, 15, 0, 15)    \
+    X(double, 9, 12, 0, 12)    \
+    X(double, 8, 14, 0, 16)    \
+    X(double, 8, 15, 0, 16)    \
+    X(double, 5, 5, 5, 5)      \
+    X(double, 3, 3, 14, 15)    \
+    X(double, 8, 16, 0, 16)    \
+    X(double, 3, 3, 15, 15)    \
+    X(double, 10, 14, 0, 14)   \
+    X(double, 12, 12, 0, 12)   \
+    X(double, 3, 7, 7, 15)     \
+    X(double, 10, 15, 0, 15)   \
+    X(double, 10, 16, 0, 16)   \
+    X(double, 2, 9, 9, 10)     \
+    X(double, 12, 14, 0, 14)   \
+    X(double, 5, 5, 7, 15)     \
+    X(double, 12, 15, 0, 15)   \
+    X(double, 3, 7, 9, 9)      \
+    X(double, 12, 16, 0, 16)   \
+    X(double, 14, 14, 0, 14)   \
+    X(double, 2, 10, 10, 10)   \
+    X(double, 14, 15, 0, 15)   \
+    X(double, 3, 6, 12, 12)    \
+    X(double, 14, 16, 0, 16)   \
+    X(double, 15, 15, 0, 15)   \
+    X(double, 15, 16, 0, 16)   \
+    X(double, 3, 9, 9, 9)      \
+    X(double, 5, 7, 7, 15)     \
+    X(double, 5, 5, 10, 10)    \
+    X(double, 3, 7, 12, 14)    \
+    X(double, 16, 16, 0, 16)   \
+    X(double, 3, 9, 10, 10)    \
+    X(double, 4, 5, 14, 16)    \
+    X(double, 2, 12, 12, 12)   \
+    X(double, 3, 7, 14, 15)    \
+    X(double, 4, 5, 15, 16)    \
+    X(double, 3, 7, 15, 15)    \
+    X(double, 5, 8, 8, 16)     \
+    X(double, 3, 9, 12, 12)    \
+    X(double, 4, 7, 12, 14)    \
+    X(double, 7, 7, 7, 7)      \
+    X(double, 5, 5, 14, 15)    \
+    X(double, 3, 8, 15, 16)    \
+    X(double, 5, 5, 15, 15)    \
+    X(double, 3, 9, 14, 14)    \
+    X(double, 3, 8, 16, 16)    \
+    X(double, 5, 7, 11, 14)    \
+    X(double, 2, 14, 14, 14)   \
+    X(double, 4, 10, 10, 12)   \
+    X(double, 5, 9, 9, 10)     \
+    X(double, 2, 14, 15, 15)   \
+    X(double, 3, 12, 12, 12)   \
+    X(double, 7, 7, 9, 9)      \
+    X(double, 2, 14, 16, 16)   \
+    X(double, 2, 15, 15, 16)   \
+    X(double, 4, 8, 15, 16)    \
+    X(double, 6, 9, 9, 12)     \
+    X(double, 5, 7, 14, 15)    \
+    X(double, 5, 10, 10, 10)   \
+    X(double, 6, 7, 12, 14)    \
+    X(double, 8, 8, 8, 16)     \
+    X(double, 5, 7, 15, 15)    \
+    X(double, 3, 12, 15, 15)   \
+    X(double, 5, 8, 14, 16)    \
+    X(double, 7, 9, 9, 14)     \
+    X(double, 4, 12, 12, 12)   \
+    X(double, 3, 14, 14, 15)   \
+    X(double, 5, 8, 15, 16)    \
+    X(double, 3, 14, 15, 15)   \
+    X(double, 5, 8, 16, 16)    \
+    X(double, 8, 9, 9, 9)      \
+    X(double, 4, 12, 14, 14)   \
+    X(double, 3, 15, 15, 15)   \
+    X(double, 7, 7, 14, 14)    \
+    X(double, 7, 10, 10, 14)   \
+    X(double, 3, 15, 16, 16)   \
+    X(double, 9, 9, 9, 9)      \
+    X(double, 7, 7, 15, 15)    \
+    X(double, 5, 10, 15, 15)   \
+    X(double, 7, 9, 12, 14)    \
+    X(double, 3, 16, 16, 16)   \
+    X(double, 4, 14, 14, 16)   \
+    X(double, 8, 10, 10, 10)   \
+    X(double, 9, 9, 10, 10)    \
+    X(double, 4, 14, 15, 16)   \
+    X(double, 6, 12, 12, 12)   \
+    X(double, 7, 9, 14, 14)    \
+    X(double, 8, 8, 14, 16)    \
+    X(double, 4, 15, 15, 16)   \
+    X(double, 7, 9, 15, 15)    \
+    X(double, 8, 8, 15, 16)    \
+    X(double, 9, 9, 12, 12)    \
+    X(double, 5, 14, 14, 15)   \
+    X(double, 10, 10, 10, 10)  \
+    X(double, 7, 12, 12, 14)   \
+    X(double, 8, 8, 16, 16)
 
 // Plans of k_line_fast and the batched kernels: {R0, R1, R2, EM}.
 #define PFH_FAST_PLANS(X)      \

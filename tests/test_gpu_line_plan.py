@@ -104,3 +104,17 @@ def test_complex_and_half_complex_routes(gpu, shape, permute, dt):
             ref = O.transform(kind, src.astype(np.complex128 if np.iscomplexobj(src) else np.float64), op,
                               shape=shape, extra=3, permute_dims=permute)
             assert rel_l2(_host(plan.execute(op, _tdev(src))), ref) <= 4 * tol(dt), (kind, op)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("n", [16500, 20160, 32768, 65536, 100000, 122500, 1031, 2 * 1031, 10007])
+def test_pieces_of_long_lines(gpu, n, dt):
+    """Splits whose pieces have line plans (16500: one of them does not),
+    Bluestein lines, odd line counts and partial last tiles; equal chunks."""
+    rng = np.random.default_rng(n)
+    for lines in (1, 5):
+        x = uniform_complex(rng, (lines, n), complex_of(dt))
+        plan = pf.LocalC2cPlan(n, dtype=torch.from_numpy(x).dtype)
+        ref = np.fft.fft(x.astype(np.complex128))
+        assert rel_l2(_host(plan.forward(_tdev(x))), ref) <= tol(dt), lines
+        assert rel_l2(_host(plan.inverse(_tdev(ref.astype(complex_of(dt))))), x) <= tol(dt), lines
