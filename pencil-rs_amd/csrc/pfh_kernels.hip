@@ -1600,6 +1600,22 @@ hipError_t launch_line_stage(const StageArgs<T> &a, bool wide, int threads, size
                              hipStream_t s)
 {
     if (grid <= 0) return hipSuccess;
+    if (a.mode == M_COPY_C || a.mode == M_COPY_R) {
+        CopyAxes c{};
+        c.nd = a.g.nd + 1;
+        c.ext[0] = a.nin;
+        c.is[0] = a.ips;
+        c.os[0] = a.ops;
+        for (int d = 0; d < a.g.nd; ++d) {
+            c.ext[d + 1] = a.g.ext[d];
+            c.is[d + 1] = a.g.is[d];
+            c.os[d + 1] = a.g.os[d];
+        }
+        bool done = false;
+        const hipError_t e = launch_copy_axes(c, a.src, a.dst, (int)sizeof(T) * (a.mode == M_COPY_C ? 2 : 1), a.gate, s,
+                                              done);
+        if (e != hipSuccess || done) return e;
+    }
     const int mg = (a.mode == M_COPY_C || a.mode == M_COPY_R)
                        ? 0
                        : ((a.mode == M_C2C || a.mode == M_R2C || a.mode == M_R2C_ODD || a.mode == M_C2R ||
@@ -1857,6 +1873,22 @@ hipError_t launch_permute_words(const PermuteArgs &p, const void *src, void *dst
 {
     const int64_t total = p.len * p.extra;
     if (total <= 0) return hipSuccess;
+    {
+        CopyAxes c{};
+        c.nd = p.nd + 1;
+        int64_t run = 1;
+        for (int d = p.nd - 1; d >= 0; --d) {
+            c.ext[d] = p.dext[d];
+            c.is[d] = p.sstride[d];
+            c.os[d] = run;
+            run *= p.dext[d];
+        }
+        c.ext[p.nd] = p.extra;
+        c.is[p.nd] = c.os[p.nd] = p.len;
+        bool done = false;
+        const hipError_t e = launch_copy_axes(c, src, dst, word, nullptr, s, done);
+        if (e != hipSuccess || done) return e;
+    }
     int64_t g = (total + 255) / 256;
     if (g > 65536) g = 65536;
     switch (word) {

@@ -144,6 +144,16 @@ hipError_t launch_inplace_begin(int *gate, const int *poison, int *status, hipSt
 
 hipError_t launch_permute_words(const PermuteArgs &p, const void *src, void *dst, int word, hipStream_t s);
 
+// Bit-exact copy between two layouts (pfh_copy.hip): axis i has extent
+// ext[i], source stride is[i] and destination stride os[i] in words; done is
+// false where the layouts are left to the caller's own kernel.
+struct CopyAxes {
+    int nd;
+    int64_t ext[16], is[16], os[16];
+};
+hipError_t launch_copy_axes(const CopyAxes &c, const void *src, void *dst, int word, const int *gate, hipStream_t s,
+                            bool &done);
+
 // Pointwise operations (pfh_pointwise.hip).
 struct ScaleAxesArgs {
     int nd;              // spatial positions
