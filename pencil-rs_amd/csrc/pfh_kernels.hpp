@@ -162,6 +162,8 @@ struct ScaleAxesArgs {
     int64_t len, extra;  // elements per extra block, extra blocks
     int64_t mext[8];     // extent of each memory position (slowest first)
     int64_t foff[8];     // offset of that position's axis in the factor array
+    uint32_t dmag[8];    // make_fastdiv constants of mext (set by the launcher)
+    int dsh[8];
 };
 constexpr int kSumSquaresParts = 1024;
 
