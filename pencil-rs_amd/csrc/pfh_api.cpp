@@ -359,11 +359,33 @@ static void find_line_plan(int m, int tbytes, int r[3], int &em)
     em = it->second[3];
 }
 
+// Does k_line_blue beat the generic kernel for an FFT length without a line
+// plan? Always for a prime factor of 17 and more, whose generic pass is O(p^2)
+// (MI355X, 2^21 points of C2C lines, f32 / f64 us: n = 97 192 / 215 generic, 18 /
+// 30 Bluestein; 209 73 / 78, 26 / 52). With 11 and 13 the generic kernel has
+// direct butterflies: it keeps products of two of them (143: 18 / 28 against 22 /
+// 35 us) and f64 lengths above 350 (462: 47 against 55 us; 330: 42 against 39).
+static bool blue_pays(int m, int tbytes)
+{
+    int wide = 0, rest = m;
+    for (int p : {11, 13})
+        while (rest % p == 0) {
+            rest /= p;
+            ++wide;
+        }
+    for (int p : {2, 3, 5, 7})
+        while (rest % p == 0) rest /= p;
+    if (rest > 1) return true;
+    return wide < 2 && (tbytes == 4 || m <= 350);
+}
+
 // k_line_plan for a stage whose mode and FFT length it has: radices, values
 // per thread and the flag that routes the launch. Arrays of 4 GiB and more
 // are left out (its offsets have 32 bits; a stage of one line digit, which
 // every local plan is, offsets from its tile and has no such bound).
-static bool choose_line_plan(Step &st, int tbytes)
+// in_stage: a whole stage (its tables go with the plan), not a piece of a
+// long line.
+static bool choose_line_plan(Step &st, int tbytes, bool in_stage)
 {
     static const int enabled = env_int("PFH_LINE_PLAN", 1);
     if (!enabled || st.big_bytes >= (1LL << 32)) return false;
@@ -371,10 +393,24 @@ static bool choose_line_plan(Step &st, int tbytes)
     const bool r2r = st.mode == M_DCT1 || st.mode == M_DST1 || st.mode == M_DCT2 || st.mode == M_DCT2_ODD ||
                      st.mode == M_DCT3 || st.mode == M_DCT3_ODD || st.mode == M_DCT4 || st.mode == M_DCT4_ODD ||
                      st.mode == M_DHT_ODD;
-    if (!(st.mode == M_C2C || st.mode == M_R2C || st.mode == M_C2R || dht || r2r)) return false;
-    if (r2r && st.m > kLinePlanRealMax) return false;
+    const bool odd = st.mode == M_R2C_ODD || st.mode == M_C2R_ODD;
+    if (!(st.mode == M_C2C || st.mode == M_R2C || st.mode == M_C2R || odd || dht || r2r)) return false;
     int r[3], em = 0;
     find_line_plan(st.m, tbytes, r, em);
+    if (r2r && st.m > kLinePlanRealMax) r[0] = 0;
+    st.blue = 0;
+    // a length without a plan: Bluestein in the workgroup. Below 16 points the
+    // generic kernel's single pass stays. (PFH_BLUESTEIN_PRIME, a request for
+    // the pieces of long lines, turns it off.)
+    static const int blue = env_int("PFH_LINE_BLUE", 1);
+    if (r[0] == 0 && blue && in_stage && std::getenv("PFH_BLUESTEIN_PRIME") == nullptr && st.m >= 16 && st.m <= kBlueMax &&
+        blue_pays(st.m, tbytes)) {
+        for (int M = 2 * st.m - 1; M <= 1024 && r[0] == 0; ++M)
+            if (blue_length(M)) {
+                find_line_plan(M, tbytes, r, em);
+                st.blue = M;
+            }
+    }
     if (r[0] == 0) return false;
     st.fast = st.line_plan = true;
     for (int i = 0; i < 3; ++i) st.fr[i] = r[i];
@@ -391,12 +427,13 @@ static bool choose_line_plan(Step &st, int tbytes)
 static void choose_fast(Step &st, int tbytes, const Tuning &tu)
 {
     st.fast = st.line_plan = false;
+    st.blue = 0;
     static const int enabled = env_int("PFH_FAST", 1);
     static const int v512 = env_int("PFH_FAST512", 0);
     static const int nt_mb = env_int("PFH_NT_MB", 256);
     if (!enabled) return;
     const bool large = nt_mb > 0 && st.io_bytes > ((int64_t)nt_mb << 20);
-    if (tu.allow_line_plan && !large && choose_line_plan(st, tbytes)) return;
+    if (tu.allow_line_plan && !large && choose_line_plan(st, tbytes, true)) return;
     const bool has_mode = st.mode == M_C2C || st.mode == M_R2C || st.mode == M_C2R;
     const int m = st.m;
     int r0 = 0, r1 = 0, r2 = 0, em = 0;
@@ -444,7 +481,7 @@ static void choose_fast(Step &st, int tbytes, const Tuning &tu)
     }
     // (radix 32: the direct first pass covers radix <= 16)
     if (!has_mode || r0 == 0 || r0 == 32 || !fast_plan_available(tbytes, r0, r1, r2, em)) {
-        if (tu.allow_line_plan) choose_line_plan(st, tbytes);
+        if (tu.allow_line_plan) choose_line_plan(st, tbytes, true);
         return;
     }
     st.fast = true;
@@ -458,9 +495,10 @@ static void choose_fast(Step &st, int tbytes, const Tuning &tu)
     if (r2) st.radices.push_back(r2);
 }
 
-// Fills mode, lengths, radices and this step's tables (appended to tab).
+// Fills mode, lengths, radices and this step's tables (appended to tab; tables
+// false: none, for a look at the radix plan).
 static pfh_status fill_transform(Step &st, const StageSpec &sp, std::vector<double> &tab, int tbytes,
-                                 const Tuning &tu)
+                                 const Tuning &tu, bool tables = true)
 {
     const int64_t n = sp.n;
     st.n = (int)n;
@@ -541,7 +579,7 @@ static pfh_status fill_transform(Step &st, const StageSpec &sp, std::vector<doub
     if (st.long_only) st.radices.clear();
     if (tu.allow_fast && !st.long_only) choose_fast(st, tbytes, tu);
 
-    // tables
+    if (!tables) return PFH_OK;
     st.tw_base = (int64_t)(tab.size() / 2);
     int off = 0;
     auto here = [&]() { return off; };
@@ -744,7 +782,8 @@ static pfh_status size_line_plan(Step &st, const DeviceInfo &dev, int tbytes, co
     st.lds_bytes = lds_of(lt);
     set_tiles(st, tu);
     st.flags &= ~F_NT;
-    st.flags |= F_LINE_PLAN;
+    st.flags &= ~F_LINE_BLUE;
+    st.flags |= F_LINE_PLAN | (st.blue ? F_LINE_BLUE : 0);
     return PFH_OK;
 }
 
@@ -883,6 +922,7 @@ static bool wants_pieces(const Step &s)
 {
     if (s.long_only) return true;
     if (s.m <= 1) return false;
+    if (s.blue) return false; // Bluestein inside the stage's kernel
     const int64_t lim = long_line_max();
     if (lim > 0 && s.m > lim) return true;
     return largest_prime_factor(s.m) > bluestein_prime();
@@ -991,6 +1031,44 @@ static bool seven_smooth(int64_t v)
     return v == 1;
 }
 
+// Named tables of Bluestein's convolution for FFT length m (sign s) and
+// convolution length M: the chirp and the transformed, scaled conjugate chirp.
+static pfh_status chirp_tables(PlanImpl &P, int64_t m, int64_t M, int s, int64_t &c_off, int64_t &bh_off)
+{
+    pfh_status st = plan_table(P, "chirp:" + std::to_string(m) + ":" + std::to_string(s), c_off,
+                               [&](std::vector<double> &t) {
+                                   for (int64_t j = 0; j < m; ++j) {
+                                       const cxl c = chirp(j, m, s);
+                                       t.push_back((double)c.real());
+                                       t.push_back((double)c.imag());
+                                   }
+                               });
+    if (st) return st;
+    return plan_table(P, "blue:" + std::to_string(m) + ":" + std::to_string(M) + ":" + std::to_string(s), bh_off,
+                      [&](std::vector<double> &t) {
+                          std::vector<cxl> b((size_t)M, cxl(0, 0));
+                          for (int64_t j = 0; j < m; ++j) {
+                              const cxl v = chirp(j, m, -s);
+                              b[(size_t)j] = v;
+                              if (j > 0) b[(size_t)(M - j)] = v;
+                          }
+                          const std::vector<cxl> B = host_dft(b);
+                          for (int64_t k = 0; k < M; ++k) {
+                              t.push_back((double)(B[(size_t)k].real() / (long double)M));
+                              t.push_back((double)(B[(size_t)k].imag() / (long double)M));
+                          }
+                      });
+}
+
+// The convolution tables of a stage on k_line_blue (its FFT has the negative
+// sign; a positive one is conjugated on load and store).
+static pfh_status blue_tables(PlanImpl &P, Step &s)
+{
+    if (!s.blue) return PFH_OK;
+    s.xvalid_in = s.m;
+    return chirp_tables(P, s.m, s.blue, -1, s.xtab_in, s.xtab_out);
+}
+
 // Does a complex FFT of length m run as one generic line stage?
 static bool piece_fits(int64_t m, const DeviceInfo &dev, int tb, const Tuning &tu)
 {
@@ -1022,7 +1100,7 @@ static bool has_line_plan(int64_t m, int tb, const Tuning &tu)
     Step p;
     p.mode = M_C2C;
     p.m = (int)m;
-    return choose_line_plan(p, tb);
+    return choose_line_plan(p, tb, false);
 }
 
 // N1 (the first piece's length) of a split N1 x N2 = m whose pieces both
@@ -1178,7 +1256,7 @@ static pfh_status make_piece(PlanImpl &P, Step &p, int64_t N, std::vector<PieceD
     p.scale = x.scale;
     const int max_r = P.tuning.max_radix ? P.tuning.max_radix : (tb == 4 ? 16 : 8);
     p.big_bytes = big_bytes;
-    if (!(P.tuning.allow_fast && P.tuning.allow_line_plan && choose_line_plan(p, tb)) &&
+    if (!(P.tuning.allow_fast && P.tuning.allow_line_plan && choose_line_plan(p, tb, false)) &&
         !radix_plan((int)N, p.radices, max_r))
         return set_err(PFH_ERR_UNSUPPORTED, "long-line piece radix plan");
     int64_t base = 0;
@@ -1360,29 +1438,7 @@ static pfh_status core_pieces(PlanImpl &P, const Step &outer, int64_t m, const L
     if (M <= 0) return set_err(PFH_ERR_UNSUPPORTED, "no Bluestein length for this line");
     const int s = (conj & F_CONJ_IN) ? 1 : -1;
     int64_t c_off = 0, bh_off = 0;
-    pfh_status st = plan_table(P, "chirp:" + std::to_string(m) + ":" + std::to_string(s), c_off,
-                               [&](std::vector<double> &t) {
-                                   for (int64_t j = 0; j < m; ++j) {
-                                       const cxl c = chirp(j, m, s);
-                                       t.push_back((double)c.real());
-                                       t.push_back((double)c.imag());
-                                   }
-                               });
-    if (st) return st;
-    st = plan_table(P, "blue:" + std::to_string(m) + ":" + std::to_string(M) + ":" + std::to_string(s), bh_off,
-                    [&](std::vector<double> &t) {
-                        std::vector<cxl> b((size_t)M, cxl(0, 0));
-                        for (int64_t j = 0; j < m; ++j) {
-                            const cxl v = chirp(j, m, -s);
-                            b[(size_t)j] = v;
-                            if (j > 0) b[(size_t)(M - j)] = v;
-                        }
-                        const std::vector<cxl> B = host_dft(b);
-                        for (int64_t k = 0; k < M; ++k) {
-                            t.push_back((double)(B[(size_t)k].real() / (long double)M));
-                            t.push_back((double)(B[(size_t)k].imag() / (long double)M));
-                        }
-                    });
+    pfh_status st = chirp_tables(P, m, M, s, c_off, bh_off);
     if (st) return st;
     const LineSide rb = region_side(outer, rb_buf, M);
     xb[rb_buf - BUF_X0] = std::max(xb[rb_buf - BUF_X0], outer.nlines * M * 2 * tb);
@@ -1415,6 +1471,7 @@ static pfh_status expand_long(PlanImpl &P, Step &s, int tb, int64_t xb[3])
 {
     s.pieces.clear();
     s.fast = s.line_plan = false;
+    s.blue = 0;
     if (s.g.nd + 1 > kMaxDigits) return set_err(PFH_ERR_UNSUPPORTED, "too many line digits for a long line");
     LineSide in, out;
     in.buf = s.in_buf;
@@ -1930,7 +1987,7 @@ static pfh_status build_op(PlanImpl &P, int op, bool in_place, OpPlan &out)
         probe.big_bytes = std::max(specs[e].in_natural.bytes(), specs[e].out_natural.bytes());
         probe.io_bytes = specs[e].in_natural.bytes() + specs[e].out_natural.bytes();
         const pfh_error_info saved = g_err;
-        if (fill_transform(probe, specs[e], scratch, tb, P.tuning) == PFH_OK && !probe.long_only &&
+        if (fill_transform(probe, specs[e], scratch, tb, P.tuning, false) == PFH_OK && !probe.long_only &&
             !wants_pieces(probe))
             line_threads[e] = threads_per_line(probe, tb);
         g_err = saved;
@@ -1944,6 +2001,7 @@ static pfh_status build_op(PlanImpl &P, int op, bool in_place, OpPlan &out)
         s.big_bytes = std::max(X[e].bytes(), Y[e].bytes());
         s.io_bytes = X[e].bytes() + Y[e].bytes();
         st = fill_transform(s, specs[e], P.host_tables, tb, P.tuning);
+        if (!st) st = blue_tables(P, s);
         if (st) return st;
         s.in = X[e];
         s.out = Y[e];
@@ -2161,6 +2219,7 @@ static pfh_status build_local_op(PlanImpl &P, int op, OpPlan &out)
     std::array<int, 8> id{};
     Step s;
     pfh_status st = fill_transform(s, sp, P.host_tables, tb, P.tuning);
+    if (!st) st = blue_tables(P, s);
     if (st) return st;
     s.in = make_layout(1, id, shin, 1, (sp.in_c ? 2 : 1) * tb);
     s.out = make_layout(1, id, shout, 1, (sp.out_c ? 2 : 1) * tb);
@@ -2522,7 +2581,9 @@ static StageArgs<T> fill_args(const PlanImpl &P, const Step &s, void *const bufs
     a.n = s.n;
     a.nin = s.nin;
     a.nout = s.nout;
-    a.m = s.m;
+    if (s.line_plan && s.mode == M_R2C_ODD) a.mode = M_R2C; // k_line_plan and k_line_blue tell by n
+    if (s.line_plan && s.mode == M_C2R_ODD) a.mode = M_C2R;
+    a.m = s.blue ? s.blue : s.m;
     a.npass = (int)s.radices.size();
     int Ns = 1;
     for (int p = 0; p < a.npass; ++p) {

@@ -11,8 +11,8 @@
 //  - they are the same: rows, moved in 16-byte pieces where lengths, strides
 //    and addresses allow.
 // Both are bound by HBM. 256 x 384 x 240 complex f32, z,y,x -> x,z,y (189 MB
-// each way) on MI355X: the line kernel's copy stage, which held whole lines of
-// 8 points a lane in LDS on one wave per workgroup, took 154 us.
+// each way) on MI355X: 74 us; the line kernel's copy stage, which held whole
+// lines on one wave per workgroup in LDS, took 154 us.
 #include <hip/hip_runtime.h>
 
 #include "pfh_kernels.hpp"

@@ -105,6 +105,20 @@ PFH_LINE_DECLARE(double, 2)
 PFH_LINE_DECLARE(float, 3)
 PFH_LINE_DECLARE(double, 3)
 #undef PFH_LINE_DECLARE
+// Stages whose FFT length has no line plan (pfh_blue.hip, F_LINE_BLUE set).
+// KIND 0: C2C, 1: every real mode.
+template <typename T, int KIND>
+hipError_t launch_line_blue(const StageArgs<T> &a, int r0, int r1, int r2, int em, int threads, size_t lds_bytes,
+                            int64_t grid, hipStream_t s);
+#define PFH_BLUE_DECLARE(TT, K)                                                                                  \
+    template <>                                                                                                  \
+    hipError_t launch_line_blue<TT, K>(const StageArgs<TT> &a, int r0, int r1, int r2, int em, int threads,      \
+                                       size_t lds_bytes, int64_t grid, hipStream_t s);
+PFH_BLUE_DECLARE(float, 0)
+PFH_BLUE_DECLARE(float, 1)
+PFH_BLUE_DECLARE(double, 0)
+PFH_BLUE_DECLARE(double, 1)
+#undef PFH_BLUE_DECLARE
 bool fast_plan_available(int tbytes, int r0, int r1, int r2, int em);
 bool multi_batch_plan_available(int tbytes, int r0, int r1, int r2, int em);
 hipError_t set_fast_lds_limit(size_t bytes);

@@ -93,6 +93,7 @@ struct Step {
     int fr[3] = {0, 0, 0};
     int fem = 16;
     bool line_plan = false; // fast runs k_line_plan (radices and em of a line plan)
+    int blue = 0;           // line_plan: Bluestein inside the workgroup (k_line_blue), the plan's length
     int64_t big_bytes = 0;  // larger of the stage's arrays in bytes (0: not known when planned)
     int64_t io_bytes = 0;   // their sum
     int digit_axis[kMaxDigits] = {-1, -1, -1, -1, -1}; // logical axis of each line digit (-1: extras)

@@ -118,3 +118,85 @@ def test_pieces_of_long_lines(gpu, n, dt):
         ref = np.fft.fft(x.astype(np.complex128))
         assert rel_l2(_host(plan.forward(_tdev(x))), ref) <= tol(dt), lines
         assert rel_l2(_host(plan.inverse(_tdev(ref.astype(complex_of(dt))))), x) <= tol(dt), lines
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+def test_odd_real_lines(gpu, dt):
+    """Odd R2C / C2R lines on the line plans, both directions and adjoints'
+    weights (route operations), row and column sides."""
+    rng = np.random.default_rng(41)
+    for n in (9, 15, 35, 63, 105, 225, 343, 441, 945):
+        r = uniform_real(rng, (9, n), dt)
+        plan = pf.LocalR2cPlan(n, dtype=torch.from_numpy(r).dtype)
+        spec = plan.forward(_tdev(r))
+        assert rel_l2(_host(spec), np.fft.rfft(r.astype(np.float64))) <= tol(dt), n
+        assert rel_l2(_host(plan.inverse(spec)), r) <= 2 * tol(dt), n
+    for shape, permute in (((21, 10, 45), True), ((12, 35, 27), False)):
+        plan = pf.R2cPlan(shape, dtype=torch.from_numpy(r).dtype, permute_dims=permute)
+        x = uniform_real(rng, int(np.prod(shape)), dt)
+        spec = O.transform(O.KIND_R2C, x.astype(np.float64), O.FORWARD, shape=shape, permute_dims=permute)
+        for op in OPS:
+            fwd_like = op in (O.FORWARD, O.ADJ_INVERSE, O.ADJ_BACKWARD)
+            src = x if fwd_like else spec.astype(complex_of(dt))
+            ref = O.transform(O.KIND_R2C, src.astype(np.complex128 if np.iscomplexobj(src) else np.float64), op,
+                              shape=shape, permute_dims=permute)
+            assert rel_l2(_host(plan.execute(op, _tdev(src))), ref) <= 4 * tol(dt), (shape, op)
+
+
+BLUE = [17, 19, 22, 26, 33, 37, 51, 61, 74, 89, 97, 101, 121, 127, 131, 143, 194, 233, 251, 257, 319, 401, 461, 511]
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+def test_lengths_without_a_plan(gpu, dt):
+    """Bluestein inside the workgroup: primes and lengths with a prime factor
+    from 11 on, every complex and real mode, rows with a partial last tile.
+    The two extra transforms and three products stay within twice the bound."""
+    rng = np.random.default_rng(43)
+    cd = complex_of(dt)
+    for n in BLUE:
+        x = uniform_complex(rng, (13, n), cd)
+        plan = pf.LocalC2cPlan(n, dtype=torch.from_numpy(x).dtype)
+        assert rel_l2(_host(plan.forward(_tdev(x))), np.fft.fft(x.astype(np.complex128))) <= 2 * tol(dt), n
+        assert rel_l2(_host(plan.inverse(_tdev(x))), np.fft.ifft(x.astype(np.complex128))) <= 2 * tol(dt), n
+        for rn in (n, 2 * n):
+            r = uniform_real(rng, (13, rn), dt)
+            rplan = pf.LocalR2cPlan(rn, dtype=torch.from_numpy(r).dtype)
+            spec = rplan.forward(_tdev(r))
+            assert rel_l2(_host(spec), np.fft.rfft(r.astype(np.float64))) <= 2 * tol(dt), rn
+            assert rel_l2(_host(rplan.inverse(spec)), r) <= 4 * tol(dt), rn
+    for n in (17, 34, 97, 110, 131, 202, 233, 466):
+        x = uniform_real(rng, (11, n), dt)
+        td = torch.from_numpy(x).dtype
+        for kind in range(1, 10):
+            plan = pf.LocalDhtPlan(n, dtype=td) if kind == 9 else pf.LocalR2rPlan(n, kind, dtype=td)
+            for op, fn in ((O.FORWARD, plan.forward), (O.INVERSE, plan.inverse)):
+                ref = O.r2r_lines(x.astype(np.float64), kind, op)
+                assert rel_l2(_host(fn(_tdev(x))), ref) <= 2 * tol(dt), (n, kind, op)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("permute", [True, False])
+def test_routes_without_a_plan(gpu, permute, dt):
+    rng = np.random.default_rng(47)
+    td = torch.float32 if dt == np.float32 else torch.float64
+    cd = torch.complex64 if dt == np.float32 else torch.complex128
+    for kind, shape, r2r in ((O.KIND_C2C, (37, 22, 29), None), (O.KIND_R2C, (26, 41, 34), None),
+                             (O.KIND_R2C, (33, 17, 53), None), (O.KIND_R2R, (31, 46, 38), [2, 5, 9]),
+                             (O.KIND_R2R, (23, 58, 39), [3, 1, 8])):
+        n = int(np.prod(shape))
+        if kind == O.KIND_C2C:
+            plan = pf.C2cPlan(shape, dtype=cd, permute_dims=permute)
+        elif kind == O.KIND_R2C:
+            plan = pf.R2cPlan(shape, dtype=td, permute_dims=permute)
+        else:
+            plan = pf.R2rPlan(shape, r2r, dtype=td, permute_dims=permute)
+        x = uniform_complex(rng, n, complex_of(dt)) if kind == O.KIND_C2C else uniform_real(rng, n, dt)
+        kw = {"r2r": r2r} if r2r else {}
+        wide = x.astype(np.complex128 if kind == O.KIND_C2C else np.float64)
+        spec = O.transform(kind, wide, O.FORWARD, shape=shape, permute_dims=permute, **kw)
+        for op in OPS:
+            fwd_like = op in (O.FORWARD, O.ADJ_INVERSE, O.ADJ_BACKWARD)
+            src = x if fwd_like or kind == O.KIND_R2R else spec.astype(complex_of(dt))
+            ref = O.transform(kind, src.astype(np.complex128 if np.iscomplexobj(src) else np.float64), op, shape=shape,
+                              permute_dims=permute, **kw)
+            assert rel_l2(_host(plan.execute(op, _tdev(src))), ref) <= 6 * tol(dt), (kind, shape, op)
