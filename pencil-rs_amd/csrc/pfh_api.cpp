@@ -902,10 +902,14 @@ static int64_t largest_prime_factor(int64_t m)
 // compute bound as it is HBM bound on MI355X (157 TFLOP/s f32 against
 // 8 TB/s), while Bluestein's pieces move about five times a stage's bytes.
 // PFH_BLUESTEIN_PRIME overrides it; read at every plan creation.
-static int64_t bluestein_prime()
+static int64_t bluestein_env()
 {
     const char *e = std::getenv("PFH_BLUESTEIN_PRIME");
-    const int64_t v = e ? std::atoll(e) : 0;
+    return e ? std::atoll(e) : 0;
+}
+static int64_t bluestein_prime()
+{
+    const int64_t v = bluestein_env();
     return v > 0 ? v : 128;
 }
 
@@ -1242,6 +1246,33 @@ static pfh_status twiddle_table(PlanImpl &P, int64_t M, int64_t &off, int &bsh)
 // longer ones multiply three table entries.
 constexpr int64_t kFullTwiddles = 1 << 20;
 
+// exp(-2 pi i d k / (n1 n2)) at [k][d], k < n1, d < n2.
+static pfh_status full_twiddles(PlanImpl &P, int64_t n1, int64_t n2, int64_t &off)
+{
+    return plan_table(P, "twf:" + std::to_string(n1) + ":" + std::to_string(n2), off, [&](std::vector<double> &t) {
+        // products of two long-double tables: a trigonometric call per entry
+        // would take 0.2 s for 2^20 entries
+        const int64_t N = n1 * n2;
+        int64_t B = 1;
+        while (B * B < N) B *= 2;
+        std::vector<cxl> lo((size_t)B), hi((size_t)(N / B + 1));
+        auto root = [&](int64_t q) {
+            const long double a = -2.0L * kPiL * (long double)q / (long double)N;
+            return cxl(cosl(a), sinl(a));
+        };
+        for (int64_t q = 0; q < B; ++q) lo[(size_t)q] = root(q);
+        for (size_t h = 0; h < hi.size(); ++h) hi[h] = root((int64_t)h * B);
+        t.reserve(t.size() + 2 * (size_t)N);
+        for (int64_t k = 0; k < n1; ++k)
+            for (int64_t d = 0; d < n2; ++d) {
+                const int64_t q = k * d;
+                const cxl a = lo[(size_t)(q % B)], b = hi[(size_t)(q / B)];
+                t.push_back((double)(a.real() * b.real() - a.imag() * b.imag()));
+                t.push_back((double)(a.real() * b.imag() + a.imag() * b.real()));
+            }
+    });
+}
+
 // One C2C line stage of length N over the given digits: a line plan where the
 // length has one and every array of the piece (big_bytes the largest) is
 // below 4 GiB, else the generic kernel.
@@ -1270,28 +1301,7 @@ static pfh_status make_piece(PlanImpl &P, Step &p, int64_t N, std::vector<PieceD
         const int64_t n2 = x.tw_m / N;
         p.xtw_full = x.tw_m <= kFullTwiddles;
         if (p.xtw_full)
-            st = plan_table(P, "twf:" + std::to_string(N) + ":" + std::to_string(n2), p.xtwr,
-                            [&](std::vector<double> &t) {
-                                // products of two long-double tables: a trigonometric call per entry would take
-                                // 0.2 s for 2^20 entries
-                                int64_t B = 1;
-                                while (B * B < x.tw_m) B *= 2;
-                                std::vector<cxl> lo((size_t)B), hi((size_t)(x.tw_m / B + 1));
-                                auto root = [&](int64_t q) {
-                                    const long double a = -2.0L * kPiL * (long double)q / (long double)x.tw_m;
-                                    return cxl(cosl(a), sinl(a));
-                                };
-                                for (int64_t q = 0; q < B; ++q) lo[(size_t)q] = root(q);
-                                for (size_t h = 0; h < hi.size(); ++h) hi[h] = root((int64_t)h * B);
-                                t.reserve(t.size() + 2 * (size_t)x.tw_m);
-                                for (int64_t k = 0; k < N; ++k)
-                                    for (int64_t d = 0; d < n2; ++d) {
-                                        const int64_t q = k * d;
-                                        const cxl a = lo[(size_t)(q % B)], b = hi[(size_t)(q / B)];
-                                        t.push_back((double)(a.real() * b.real() - a.imag() * b.imag()));
-                                        t.push_back((double)(a.real() * b.imag() + a.imag() * b.real()));
-                                    }
-                            });
+            st = full_twiddles(P, N, n2, p.xtwr);
         else
             st = plan_table(P, "twr:" + std::to_string(RL) + ":" + std::to_string(n2), p.xtwr,
                             [&](std::vector<double> &t) {
@@ -1440,6 +1450,87 @@ static pfh_status core_pieces(PlanImpl &P, const Step &outer, int64_t m, const L
     int64_t c_off = 0, bh_off = 0;
     pfh_status st = chirp_tables(P, m, M, s, c_off, bh_off);
     if (st) return st;
+    // Both pieces of the split on line plans: three launches through one region.
+    // The first piece transforms n1 (n = N2 n1 + n2) as in fft_pieces; the
+    // middle launch finishes the first transform over n2 (k = k1 + N1 k2),
+    // multiplies by FFT_M(b) / M, conjugates and starts the second transform
+    // over k2 with q = q2 + N2 q1, row by row in place; the last piece
+    // transforms k1 and stores index q. 838 lines of 10007 points, f32, on
+    // MI355X, forward + inverse: 304 us, with 4 launches through two regions 470.
+    int64_t n1 = 0;
+    if (bluestein_env() <= 0 && !(piece_fits(M, P.dev, tb, P.tuning) && !split_pays(P, M, tb, n1)))
+        n1 = split_factor(P, M, tb);
+    else
+        n1 = 0;
+    const int64_t n2 = n1 > 0 ? M / n1 : 0;
+    const int64_t big = std::max(outer.big_bytes, outer.nlines * M * 2 * tb);
+    if (n1 > 0 && M <= kFullTwiddles && big < (1LL << 32) && has_line_plan(n1, tb, P.tuning) &&
+        has_line_plan(n2, tb, P.tuning)) {
+        const int nd = outer.g.nd;
+        const LineSide rs = region_side(outer, rs_buf, M);
+        xb[rs_buf - BUF_X0] = std::max(xb[rs_buf - BUF_X0], outer.nlines * M * 2 * tb);
+        int64_t bt_off = 0, tw_off = 0;
+        const size_t bh_at = (size_t)bh_off * 2;
+        st = plan_table(P, "bluet:" + std::to_string(m) + ":" + std::to_string(M) + ":" + std::to_string(s) + ":" +
+                               std::to_string(n1),
+                        bt_off, [&](std::vector<double> &t) {
+                            for (int64_t k1 = 0; k1 < n1; ++k1)
+                                for (int64_t k2 = 0; k2 < n2; ++k2) {
+                                    const size_t k = bh_at + 2 * (size_t)(k1 + n1 * k2);
+                                    const double re = t[k], im = t[k + 1];
+                                    t.push_back(re);
+                                    t.push_back(im);
+                                }
+                        });
+        if (!st) st = full_twiddles(P, n1, n2, tw_off);
+        if (st) return st;
+        {
+            std::vector<PieceDigit> digs;
+            digs.push_back({n2, in.point, 1, true});
+            for (int d = 0; d < nd; ++d) digs.push_back({outer.g.ext[d], in.dig[d], rs.dig[d], false});
+            PieceX x;
+            x.flags = F_XIN | F_XTW;
+            x.tab_in = c_off;
+            x.mul_in = (int)n2;
+            x.valid_in = (int)m;
+            st = twiddle_table(P, M, x.tw, x.tw_bsh);
+            if (st) return st;
+            x.tw_m = (int)M;
+            Step p;
+            st = make_piece(P, p, n1, digs, n2 * in.point, n2, in.buf, rs_buf, x, tb, big);
+            if (st) return st;
+            pieces.push_back(p);
+        }
+        {
+            std::vector<PieceDigit> digs;
+            digs.push_back({n1, n2, n2, true});
+            for (int d = 0; d < nd; ++d) digs.push_back({outer.g.ext[d], rs.dig[d], rs.dig[d], false});
+            PieceX x;
+            Step p;
+            st = make_piece(P, p, n2, digs, 1, 1, rs_buf, rs_buf, x, tb, big);
+            if (st) return st;
+            p.flags |= F_LINE_CONV;
+            p.xtab_out = bt_off;
+            p.xtwr = tw_off;
+            pieces.push_back(p);
+        }
+        {
+            std::vector<PieceDigit> digs;
+            digs.push_back({n2, 1, out.point, true});
+            for (int d = 0; d < nd; ++d) digs.push_back({outer.g.ext[d], rs.dig[d], out.dig[d], false});
+            PieceX x;
+            x.flags = F_CONJ_OUT | F_XOUT;
+            x.scale = scale;
+            x.tab_out = c_off;
+            x.valid_out = (int)m;
+            x.mul_out = (int)n2;
+            Step p;
+            st = make_piece(P, p, n1, digs, n2, n2 * out.point, rs_buf, out.buf, x, tb, big);
+            if (st) return st;
+            pieces.push_back(p);
+        }
+        return PFH_OK;
+    }
     const LineSide rb = region_side(outer, rb_buf, M);
     xb[rb_buf - BUF_X0] = std::max(xb[rb_buf - BUF_X0], outer.nlines * M * 2 * tb);
     {

@@ -87,7 +87,7 @@ hipError_t launch_line_fast(const StageArgs<T> &a, int r0, int r1, int r2, int e
                             int64_t grid, hipStream_t s);
 // Stages with a line plan (pfh_line.hip, F_LINE_PLAN set). KIND 0: C2C, 1:
 // R2C / C2R / DHT of even length, 2: the other real-to-real modes, 3: C2C
-// pieces of long lines.
+// pieces of long lines, 4: the middle of a split Bluestein convolution.
 // launch_line_fast dispatches to them.
 template <typename T, int KIND>
 hipError_t launch_line_plan(const StageArgs<T> &a, int r0, int r1, int r2, int em, int threads, size_t lds_bytes,
@@ -104,6 +104,8 @@ PFH_LINE_DECLARE(double, 1)
 PFH_LINE_DECLARE(double, 2)
 PFH_LINE_DECLARE(float, 3)
 PFH_LINE_DECLARE(double, 3)
+PFH_LINE_DECLARE(float, 4)
+PFH_LINE_DECLARE(double, 4)
 #undef PFH_LINE_DECLARE
 // Stages whose FFT length has no line plan (pfh_blue.hip, F_LINE_BLUE set).
 // KIND 0: C2C, 1: every real mode.

@@ -35,7 +35,10 @@ namespace pfh {
 // KIND 0: C2C lines; 1: R2C / C2R / DHT lines of even length (the half-length
 // transform of real pairs) and R2C / C2R lines of odd length n = M (the complex
 // transform of the real line, half of its outputs or inputs); 2: the other real-to-real modes; 3: C2C pieces of
-// long lines (load and store factors, zero padding, crop, split twiddles).
+// long lines (load and store factors, zero padding, crop, split twiddles); 4: the
+// middle of a split Bluestein convolution: rows k1 of N2 = M values, FFT, times
+// the transformed chirp (xtab_out, [k1][k2]), conjugate, FFT, times the split's
+// twiddles (xtwr, [k1][q2]), in place.
 // Lines past the end of the last tile repeat the last line's loads and store
 // nothing.
 template <typename T, int R0, int R1, int R2, int EM, int KIND>
@@ -85,7 +88,7 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
     // pieces of long lines: coordinates of the line digit that the factors and
     // full indexes run over (iline, oline may be relative to the tile)
     uint32_t idco = 0, odco = 0;
-    if constexpr (KIND == 3) {
+    if constexpr (KIND == 3 || KIND == 4) {
         if (a.xdig >= 0) {
             const uint32_t last = nlines - 1;
             idco = line_digit(a.g, tile0 + (uint32_t)il < nlines ? tile0 + (uint32_t)il : last, a.xdig);
@@ -131,7 +134,7 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
         }
         P::first_store(iln, it, v);
         P::mid(iln, tw1, it);
-    } else if constexpr (KIND == 0) {
+    } else if constexpr (KIND == 0 || KIND == 4) {
         constexpr int N0 = P::template rounds<R0>(), NB0 = M / R0;
         cpx<T> v[N0][R0];
         const uint32_t st = (uint32_t)a.ips * (uint32_t)(2 * sizeof(T));
@@ -286,7 +289,38 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
     }
 
     const T sc = a.scale;
-    if constexpr (KIND == 3) {
+    if constexpr (KIND == 4) {
+        constexpr int NL = P::template rounds<RL>(), NB = M / RL;
+        cpx<T> v[NL][RL];
+        P::last(iln, twl, it, v);
+        __syncthreads();
+        const V *bh = reinterpret_cast<const V *>(a.xtab_out) + idco * (uint32_t)M;
+        const V *tw = reinterpret_cast<const V *>(a.xtwr) + odco * (uint32_t)M;
+#pragma unroll
+        for (int b = 0; b < NL; ++b) {
+            const int j = it + TPL * b;
+            if (P::template has<RL>(b, j)) {
+#pragma unroll
+                for (int r = 0; r < RL; ++r) put<T>(iln + j + r * NB, conjg(cmul(v[b][r], get<T>(bh + j + r * NB))));
+            }
+        }
+        __syncthreads();
+        P::template first_lds<false>(iln, nullptr, it);
+        P::mid(iln, tw1, it);
+        P::last(oln, twl, ot, v);
+        if (!store) return;
+        const uint32_t st = (uint32_t)a.ops * (uint32_t)(2 * sizeof(T));
+        const uint32_t off = line_offset<true>(a.g, oline, 2 * sizeof(T)) + (uint32_t)ot * st;
+#pragma unroll
+        for (int b = 0; b < NL; ++b) {
+            const int j = ot + TPL * b;
+            if (P::template has<RL>(b, j)) {
+#pragma unroll
+                for (int r = 0; r < RL; ++r)
+                    gwrite<cpx<T>>(dst, off + (uint32_t)(b * TPL + r * NB) * st, cmul(v[b][r], get<T>(tw + j + r * NB)));
+            }
+        }
+    } else if constexpr (KIND == 3) {
         constexpr int NL = P::template rounds<RL>(), NB = M / RL;
         if (!store) return;
         cpx<T> v[NL][RL];

@@ -432,6 +432,8 @@ template <typename P, typename T, int MODE>
 __device__ __forceinline__ void load_mode(const StageArgs<T> &a, const void *src, typename P::V *ln,
                                           const typename P::V *tws, uint32_t off, int t)
 {
+    // (4 pairs in flight: the whole line's 16 at once took 3-6% longer, the
+    // registers cost more than the latency)
     constexpr int TPL = P::TPL, U = 4;
     const uint32_t s1 = (uint32_t)a.ips * (uint32_t)sizeof(T);
     const int np = (a.n + 1) >> 1;

@@ -89,6 +89,7 @@ enum StageFlags : int {
     F_XOUT = 16384, // points whose full index reaches xvalid_out are not stored; xtab_out factor on store
     F_XTW = 32768,  // twiddle exp(-2 pi i d k / xtw_m) on the store of point k
     F_LINE_PLAN = 65536, // the stage runs on k_line_plan (its radices and em are a line plan)
+    F_LINE_CONV = 262144, // with F_LINE_PLAN: the middle of a split Bluestein convolution (k_line_plan KIND 4)
     F_LINE_BLUE = 131072, // with F_LINE_PLAN: Bluestein inside k_line_blue (the plan's length M >= 2 m - 1)
 };
 
