@@ -35,8 +35,9 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_blue(const StageArgs<
     V *data = tws + a.twn;
     if (a.gate != nullptr && *a.gate != 0) return;
     const int tid = threadIdx.x, lt = a.lt, m = a.xvalid_in;
-    const uint32_t tile0 = (uint32_t)blockIdx.x * (uint32_t)lt;
+    const uint32_t tile0 = tile_of_block(a, blockIdx.x) * (uint32_t)lt;
     const uint32_t nlines = (uint32_t)a.nlines;
+    if (tile0 >= nlines) return;
     const int lsh = __builtin_ctz((unsigned)lt);
     const int rl = (int)((unsigned)tid / (unsigned)TPL), rt = tid - rl * TPL;
     const int cl = tid & (lt - 1), ct = tid >> lsh;

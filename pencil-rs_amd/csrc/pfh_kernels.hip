@@ -780,11 +780,8 @@ __global__ __launch_bounds__(WIDE ? kMaxThreadsWide : kMaxThreads) void k_line_s
     if (a.gate != nullptr && *a.gate != 0) return;
     const int tid = threadIdx.x;
     const int nthr = blockDim.x;
-    int64_t tile = blockIdx.x;
-    if (a.flags & F_XCD_REMAP) {
-        tile = (int64_t)(blockIdx.x % 8u) * a.xcd_per + blockIdx.x / 8u;
-        if (tile >= a.ntiles) return;
-    }
+    const int64_t tile = tile_of_block(a, blockIdx.x);
+    if (tile >= a.ntiles) return;
     for (int i = tid; i < a.twn; i += nthr) tws[i] = a.tw[i];
     // pass plan in LDS (read with a runtime pass index; indexing the argument
     // struct dynamically would force a private copy of it)
@@ -1187,11 +1184,8 @@ __global__ __launch_bounds__(512) void k_line_fast(const StageArgs<T> a)
     if (a.gate != nullptr && *a.gate != 0) return;
     const int tid = threadIdx.x;
     const int nthr = blockDim.x;
-    int64_t tile = blockIdx.x;
-    if (a.flags & F_XCD_REMAP) {
-        tile = (int64_t)(blockIdx.x % 8u) * a.xcd_per + blockIdx.x / 8u;
-        if (tile >= a.ntiles) return;
-    }
+    const int64_t tile = tile_of_block(a, blockIdx.x);
+    if (tile >= a.ntiles) return;
     for (int i = tid; i < a.twn; i += nthr) tws[i] = a.tw[i];
     fast_body<T, R0, R1, R2, EM, NT>(a, tile, tws, tws + a.twn);
 }

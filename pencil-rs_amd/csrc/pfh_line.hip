@@ -53,8 +53,9 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
     if (a.gate != nullptr && *a.gate != 0) return;
     const int tid = threadIdx.x;
     const int lt = a.lt;
-    const uint32_t tile0 = (uint32_t)blockIdx.x * (uint32_t)lt;
+    const uint32_t tile0 = tile_of_block(a, blockIdx.x) * (uint32_t)lt;
     const uint32_t nlines = (uint32_t)a.nlines;
+    if (tile0 >= nlines) return;
     // column side: consecutive lanes on consecutive lines (lt is a power of
     // two); row side: consecutive lanes along a line
     const int lsh = __builtin_ctz((unsigned)lt);

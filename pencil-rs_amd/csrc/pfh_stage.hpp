@@ -80,7 +80,7 @@ enum StageFlags : int {
     F_HERM_DOUBLE = 64, // R2C adjoint weights: x2 on interior bins, Im := 0 at DC/Nyquist
     F_HERM_HALF = 128,  // C2R adjoint weights: x1/2 on interior bins
     F_WEIGHTS = 256,    // apply pre/post edge weights (R2R adjoints)
-    F_XCD_REMAP = 512,  // map consecutive tiles onto one XCD
+    F_XCD_REMAP = 512,  // (unused) contiguous eighths of the tiles per XCD
     F_DIRECT_FIRST = 1024, // first radix pass reads global memory into registers
     F_DIRECT_LAST = 2048,  // last radix pass writes global memory from registers (C2C)
     F_NT = 4096,           // stage arrays exceed the last-level cache: non-temporal loads and stores
@@ -153,7 +153,7 @@ struct StageArgs {
     int lc;                 // lines computed at a time (lc * tpl threads; lt is a multiple of lc)
     int ls;                 // LDS stride of one line (complex units)
     int in_col, out_col;    // column (lines adjacent in memory) access on load / store
-    int xcd_per;            // tiles per XCD when F_XCD_REMAP
+    int xcd_per;            // consecutive tiles that go to one XCD (tile_of_block; 0: no grouping)
     T scale;
     T prew0, prew1, postw0, postw1;
     // Pieces of a long line (F_XIN / F_XOUT / F_XTW): a line too long for one
@@ -172,6 +172,17 @@ struct StageArgs {
     const cpx<T> *xtwr;
     int xtw_full;
 };
+
+// Tile of a workgroup: workgroup b runs on XCD b mod 8; with xcd_per = G > 0
+// each XCD takes G consecutive tiles of every 8 G (the grid is a multiple of
+// 8 G; tiles past the end do nothing).
+template <typename T>
+__host__ __device__ __forceinline__ uint32_t tile_of_block(const StageArgs<T> &a, uint32_t b)
+{
+    if (a.xcd_per <= 0) return b;
+    const uint32_t G = (uint32_t)a.xcd_per, g = b / (8u * G), r = b - g * (8u * G);
+    return (g * 8u + (r & 7u)) * G + (r >> 3);
+}
 
 // Pre- and post-processing of a long real line (k_long_prep / k_long_post,
 // pfh_long.hip): the transform runs as a complex FFT of length m of the

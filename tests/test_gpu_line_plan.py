@@ -200,3 +200,17 @@ def test_routes_without_a_plan(gpu, permute, dt):
             ref = O.transform(kind, src.astype(np.complex128 if np.iscomplexobj(src) else np.float64), op, shape=shape,
                               permute_dims=permute, **kw)
             assert rel_l2(_host(plan.execute(op, _tdev(src))), ref) <= 6 * tol(dt), (kind, shape, op)
+
+
+@pytest.mark.parametrize("tiles", [63, 64, 127, 128, 129, 257, 1023, 1024, 1025, 1300])
+def test_tile_runs_cover_every_line(gpu, tiles):
+    """Runs of tiles per XCD: tile counts around the multiples of a round of
+    runs, on k_line_plan (15), k_line_blue (17) and the generic kernel (11)."""
+    rng = np.random.default_rng(tiles)
+    for n, per in ((15, 256 // 3), (17, 256 // 9), (11, 128)):
+        lines = tiles * per - 1
+        x = uniform_complex(rng, (lines, n), np.complex64)
+        got = _host(pf.LocalC2cPlan(n, dtype=torch.complex64).forward(_tdev(x)))
+        ref = np.fft.fft(x.astype(np.complex128))
+        per_line = np.linalg.norm(got - ref, axis=1) / np.linalg.norm(ref, axis=1)
+        assert per_line.max() <= 4 * tol(np.float32), (n, int(per_line.argmax()))
