@@ -2663,11 +2663,11 @@ static pfh_status view_workspace(const PlanImpl &P, const OpPlan &o, void *ws, s
 }
 
 template <typename T>
-static StageArgs<T> fill_args(const PlanImpl &P, const Step &s, void *const bufs[BUF_COUNT], const int *gate)
+static StageArgs<T> fill_args(const PlanImpl &P, const Step &s, const void *in, void *out, const int *gate)
 {
     StageArgs<T> a{};
-    a.src = bufs[s.in_buf];
-    a.dst = bufs[s.out_buf];
+    a.src = in;
+    a.dst = out;
     a.tw = reinterpret_cast<const cpx<T> *>(P.dev_tables) + s.tw_base;
     a.gate = gate;
     a.nlines = s.nlines;
@@ -2788,12 +2788,8 @@ static pfh_status launch_step_ptrs(const PlanImpl &P, const Step &s, const void 
         PFH_HIP_CHECK(launch_local_endpoint_check<T>(in, s.nlines, s.nin, (s.n % 2 == 0) ? 1 : 0, wv.first_code,
                                                      wv.gate, wv.status, stream));
     }
-    void *io[BUF_COUNT] = {const_cast<void *>(in), out};
-    Step sp = s;
-    sp.in_buf = 0;
-    sp.out_buf = 1;
     const bool gated = s.endpoint_check || s.local_endpoint_check || s.gated || wv.gate_all;
-    const StageArgs<T> a = fill_args<T>(P, sp, io, gated ? wv.gate : nullptr);
+    const StageArgs<T> a = fill_args<T>(P, s, in, out, gated ? wv.gate : nullptr);
     if (s.fast) {
         PFH_HIP_CHECK(launch_line_fast<T>(a, s.fr[0], s.fr[1], s.fr[2], s.fem, s.threads, s.lds_bytes, s.grid, stream));
         return PFH_OK;
@@ -2836,11 +2832,7 @@ static pfh_status launch_pieces(const PlanImpl &P, const Step &s, void *const bu
         } else if (pc.launch == 2) {
             PFH_HIP_CHECK(launch_long_post<T>(fill_long_args<T>(P, pc, pin, pout, gate), stream));
         } else {
-            void *io[BUF_COUNT] = {const_cast<void *>(pin), pout};
-            Step sp = pc;
-            sp.in_buf = 0;
-            sp.out_buf = 1;
-            const StageArgs<T> a = fill_args<T>(P, sp, io, gate);
+            const StageArgs<T> a = fill_args<T>(P, pc, pin, pout, gate);
             if (pc.fast) {
                 PFH_HIP_CHECK(launch_line_fast<T>(a, pc.fr[0], pc.fr[1], pc.fr[2], pc.fem, pc.threads, pc.lds_bytes,
                                                   pc.grid, stream));
@@ -4014,7 +4006,7 @@ static pfh_status batch_upload(pfh_batch_s &B, int op, const void *const *srcs, 
             pfh_status e = view_workspace(P, o, static_cast<char *>(ws) + off[i], (size_t)(B.ws_bytes), wv);
             if (e) return e;
             void *bufs[4] = {const_cast<void *>(srcs[i]), dsts[i], wv.w[0], wv.w[1]};
-            g->items.push_back(fill_args<T>(P, st, bufs, nullptr));
+            g->items.push_back(fill_args<T>(P, st, bufs[st.in_buf], bufs[st.out_buf], nullptr));
             g->prefix.push_back(g->prefix.back() + st.tiles);
             g->bs.lds = std::max(g->bs.lds, st.lds_bytes);
             g->bs.threads = std::max(g->bs.threads, st.threads);

@@ -262,7 +262,14 @@ def _require_gpu():
         raise RuntimeError("pencil_fft_hip needs a ROCm GPU; there is no CPU fallback")
 
 
+# torch.cuda.current_stream() builds a Stream object on every call (2.8 us of
+# the 15 us a three-launch call takes); the raw handle needs none.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream():
+    if _raw_stream is not None:
+        return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
@@ -525,8 +532,8 @@ class _RoutePlan(_Plan):
         return torch.empty(elems, dtype=dt, device=device)
 
     def execute(self, op, src, dst=None, workspace=None, flags=0):
-        (_, _), (oe, ob) = self._in_out(op)
         if dst is None:
+            (_, _), (oe, ob) = self._in_out(op)
             dst = self._alloc(oe, ob, src.device)
         w = self._workspace(workspace)
         _check(_lib.pfh_execute(self._h, op, _ptr(src), src.numel(), _ptr(dst), dst.numel(), _ptr(w), w.numel(),
