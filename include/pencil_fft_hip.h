@@ -315,6 +315,19 @@ pfh_status pfh_local_execute(pfh_plan plan, int op, const void *src, size_t src_
 pfh_status pfh_local_execute_in_place(pfh_plan plan, int op, void *data, size_t elems, size_t capacity_bytes,
                                       void *workspace, size_t workspace_bytes, pfh_stream_t stream, int flags);
 
+/* An operation and the pointwise step that follows it, in the operation's last
+ * pass where that stage can carry it, as two steps otherwise (the same results).
+ * pfh_execute_scaled: pfh_execute, then pfh_pointwise_scale_axes of dst by real
+ * per-axis factors (the complex side of the plan: FORWARD, ADJOINT_INVERSE and
+ * ADJOINT_BACKWARD). pfh_execute_quadratic: pfh_execute into a real dst, then
+ * dst = y + a y^2 (pfh_pointwise_quadratic); with PFH_EXEC_DEFER_STATUS a
+ * rejected spectrum leaves dst's contents unspecified. */
+pfh_status pfh_execute_scaled(pfh_plan plan, int op, const void *src, size_t src_elems, void *dst, size_t dst_elems,
+                              const void *factors, void *workspace, size_t workspace_bytes, pfh_stream_t stream,
+                              int flags);
+pfh_status pfh_execute_quadratic(pfh_plan plan, int op, const void *src, size_t src_elems, void *dst, size_t dst_elems,
+                                 double a, void *workspace, size_t workspace_bytes, pfh_stream_t stream, int flags);
+
 /* *_with_timing (distributed.rs:290-325, 3796-3867): same as pfh_execute,
  * synchronous, with per-step device times from HIP events. */
 pfh_status pfh_execute_with_timing(pfh_plan plan, int op, const void *src, size_t src_elems, void *dst,

@@ -780,7 +780,8 @@ static pfh_status size_line_plan(Step &st, const DeviceInfo &dev, int tbytes, co
                                    st.out_col ? (st.out_cplx ? 128 / cb : 64 / tbytes) : 1);
         while (lt / 2 >= least && lds_of(lt) > dev.lds_limit / 2) lt /= 2;
     } else {
-        lt = (int)std::max<int64_t>(1, std::min<int64_t>(256 / tpl, st.nlines));
+        static const int row_threads = env_int("PFH_ROW_THREADS", 256);
+        lt = (int)std::max<int64_t>(1, std::min<int64_t>(row_threads / tpl, st.nlines));
     }
     while (lt > 1 && lds_of(lt) > dev.lds_limit) lt /= 2;
     if (lds_of(lt) > dev.lds_limit) return set_err(PFH_ERR_UNSUPPORTED, "line does not fit in LDS");
@@ -2531,6 +2532,11 @@ static pfh_status create_impl(const pfh_desc *d, PlanImpl &P)
 // ---------------------------------------------------------------------------
 
 struct WsView {
+    // a pointwise step that the call's last stage applies at its store
+    const Step *last = nullptr;       // that stage (null: none)
+    const void *factors = nullptr;    // per-axis factors, or
+    double quad = 0.0;                // the quadratic step's coefficient
+    int foff[8] = {0};                // factor offset of every logical axis
     int *status = nullptr;
     int *gate = nullptr;
     unsigned long long *first_code = nullptr;
@@ -2789,7 +2795,18 @@ static pfh_status launch_step_ptrs(const PlanImpl &P, const Step &s, const void 
                                                      wv.gate, wv.status, stream));
     }
     const bool gated = s.endpoint_check || s.local_endpoint_check || s.gated || wv.gate_all;
-    const StageArgs<T> a = fill_args<T>(P, s, in, out, gated ? wv.gate : nullptr);
+    StageArgs<T> a = fill_args<T>(P, s, in, out, gated ? wv.gate : nullptr);
+    if (wv.last == &s) {
+        if (wv.factors) {
+            a.flags |= F_AXIS_SCALE;
+            a.sfac = static_cast<const T *>(wv.factors);
+            a.sfac_pt = wv.foff[s.axis];
+            for (int d = 0; d < kMaxDigits; ++d) a.sfac_dig[d] = s.digit_axis[d] >= 0 ? wv.foff[s.digit_axis[d]] : -1;
+        } else {
+            a.flags |= F_QUADRATIC;
+            a.quad = (T)wv.quad;
+        }
+    }
     if (s.fast) {
         PFH_HIP_CHECK(launch_line_fast<T>(a, s.fr[0], s.fr[1], s.fr[2], s.fem, s.threads, s.lds_bytes, s.grid, stream));
         return PFH_OK;
@@ -3019,9 +3036,25 @@ static pfh_status collect_status(const PlanImpl &P, const WsView &wv, hipStream_
     return ok();
 }
 
+// A pointwise step after an operation: per-axis factors (factors set) or the
+// quadratic step with coefficient quad.
+struct PostStep {
+    const void *factors;
+    double quad;
+};
+
+// Can the operation's last stage apply the step at its store?
+static bool can_fuse(const OpPlan &o, const PostStep &post)
+{
+    if (o.steps.empty() || !o.pairs.empty()) return false;
+    const Step &s = o.steps.back();
+    if (!s.line_plan || s.blue || !s.pieces.empty()) return false;
+    return post.factors ? s.mode == M_C2C : (s.mode == M_C2R || s.mode == M_C2R_ODD);
+}
+
 static pfh_status execute_impl(PlanImpl &P, int op, const void *src, size_t src_elems, void *dst, size_t dst_elems,
                                void *ws, size_t ws_bytes, hipStream_t stream, int flags, pfh_transform_timing *timing,
-                               bool bind = true)
+                               bool bind = true, const PostStep *post = nullptr, bool *fused = nullptr)
 {
     if (op < 0 || op > 5) return set_err(PFH_ERR_INVALID_ARGUMENT, "op");
     const bool is_tr = (P.kind == PFH_LOCAL_TRANSPOSE || P.kind == PFH_ALLTOALLV_TRANSPOSE);
@@ -3090,6 +3123,17 @@ static pfh_status execute_impl(PlanImpl &P, int op, const void *src, size_t src_
             pfh_status st = bind_workspace(P, ws, stream);
             if (st) return st;
         }
+    }
+    if (post && can_fuse(o, *post)) {
+        wv.last = &o.steps.back();
+        wv.factors = post->factors;
+        wv.quad = post->quad;
+        int off = 0;
+        for (int a = 0; a < o.out.N; ++a) {
+            wv.foff[a] = off;
+            off += (int)o.out.shape[a];
+        }
+        *fused = true;
     }
     void *bufs[4] = {const_cast<void *>(src), dst, wv.w[0], wv.w[1]};
     TimingTrace tr;
@@ -4454,6 +4498,39 @@ pfh_status pfh_pointwise_quadratic(int precision, const void *w, void *u, size_t
     PFH_HIP_CHECK(precision == PFH_F32 ? launch_quadratic<float>(w, u, (int64_t)n, a, s)
                                        : launch_quadratic<double>(w, u, (int64_t)n, a, s));
     return ok();
+}
+
+pfh_status pfh_execute_scaled(pfh_plan plan, int op, const void *src, size_t src_elems, void *dst, size_t dst_elems,
+                              const void *factors, void *workspace, size_t workspace_bytes, pfh_stream_t stream,
+                              int flags)
+{
+    if (!plan || !factors) return set_err(PFH_ERR_INVALID_ARGUMENT, "null argument");
+    PlanImpl &P = plan->impl;
+    if (!(P.kind == PFH_C2C || P.kind == PFH_R2C || P.kind == PFH_MIXED_C2C || P.kind == PFH_MIXED_R2C) ||
+        !(op == PFH_FORWARD || op == PFH_ADJOINT_INVERSE || op == PFH_ADJOINT_BACKWARD))
+        return set_err(PFH_ERR_INVALID_ARGUMENT, "needs an operation onto the complex output side of a plan");
+    const PostStep post{factors, 0.0};
+    bool fused = false;
+    pfh_status st = execute_impl(P, op, src, src_elems, dst, dst_elems, workspace, workspace_bytes,
+                                 reinterpret_cast<hipStream_t>(stream), flags, nullptr, true, &post, &fused);
+    if (st || fused || dst_elems == 0) return st;
+    return scale_axes_impl(plan, 1, dst, dst_elems, factors, false, stream);
+}
+
+pfh_status pfh_execute_quadratic(pfh_plan plan, int op, const void *src, size_t src_elems, void *dst, size_t dst_elems,
+                                 double a, void *workspace, size_t workspace_bytes, pfh_stream_t stream, int flags)
+{
+    if (!plan) return set_err(PFH_ERR_INVALID_ARGUMENT, "null argument");
+    PlanImpl &P = plan->impl;
+    if (!(P.kind == PFH_R2C || P.kind == PFH_MIXED_R2C) ||
+        !(op == PFH_INVERSE || op == PFH_BACKWARD || op == PFH_ADJOINT_FORWARD))
+        return set_err(PFH_ERR_INVALID_ARGUMENT, "needs an operation onto the real side of a plan");
+    const PostStep post{nullptr, a};
+    bool fused = false;
+    pfh_status st = execute_impl(P, op, src, src_elems, dst, dst_elems, workspace, workspace_bytes,
+                                 reinterpret_cast<hipStream_t>(stream), flags, nullptr, true, &post, &fused);
+    if (st || fused || dst_elems == 0) return st;
+    return pfh_pointwise_quadratic(P.precision, dst, dst, dst_elems, a, stream);
 }
 
 pfh_status pfh_pointwise_quadratic_adjoint(int precision, const void *w, const void *g, void *out, size_t n,

@@ -1273,6 +1273,8 @@ hipError_t launch_line_fast(const StageArgs<T> &a, int r0, int r1, int r2, int e
         if (a.mode == M_C2C) return launch_line_blue<T, 0>(a, r0, r1, r2, em, threads, lds_bytes, grid, s);
         return launch_line_blue<T, 1>(a, r0, r1, r2, em, threads, lds_bytes, grid, s);
     }
+    if (a.flags & F_AXIS_SCALE) return launch_line_plan<T, 5>(a, r0, r1, r2, em, threads, lds_bytes, grid, s);
+    if (a.flags & F_QUADRATIC) return launch_line_plan<T, 6>(a, r0, r1, r2, em, threads, lds_bytes, grid, s);
     if (a.flags & F_LINE_CONV) return launch_line_plan<T, 4>(a, r0, r1, r2, em, threads, lds_bytes, grid, s);
     if (a.flags & F_LINE_PLAN) {
         if (a.mode == M_C2C && (a.flags & (F_XIN | F_XOUT | F_XTW)))

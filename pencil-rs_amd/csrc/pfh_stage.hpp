@@ -89,6 +89,8 @@ enum StageFlags : int {
     F_XOUT = 16384, // points whose full index reaches xvalid_out are not stored; xtab_out factor on store
     F_XTW = 32768,  // twiddle exp(-2 pi i d k / xtw_m) on the store of point k
     F_LINE_PLAN = 65536, // the stage runs on k_line_plan (its radices and em are a line plan)
+    F_AXIS_SCALE = 524288, // outputs times the per-axis factors sfac
+    F_QUADRATIC = 1048576, // real outputs y as y + quad y^2
     F_LINE_CONV = 262144, // with F_LINE_PLAN: the middle of a split Bluestein convolution (k_line_plan KIND 4)
     F_LINE_BLUE = 131072, // with F_LINE_PLAN: Bluestein inside k_line_blue (the plan's length M >= 2 m - 1)
 };
@@ -171,6 +173,10 @@ struct StageArgs {
     // at [r][d], exp(-2 pi i d r / (RL n2)), r < RL (the last radix), a factor of the two-level table's
     const cpx<T> *xtwr;
     int xtw_full;
+    // Pointwise steps in the last stage's store (k_line_plan KIND 5 and 6).
+    const T *sfac;          // per-axis factors (F_AXIS_SCALE): point k's at sfac_pt + k, digit d's at sfac_dig[d] + coordinate
+    int sfac_pt, sfac_dig[kMaxDigits]; // (sfac_dig < 0: no factor)
+    T quad;                 // y + quad y^2 (F_QUADRATIC)
 };
 
 // Tile of a workgroup: workgroup b runs on XCD b mod 8; with xcd_per = G > 0

@@ -183,7 +183,8 @@ _lib = None
 EXPORTED_SYMBOLS = (
     "pfh_version", "pfh_last_error", "pfh_status_string", "pfh_plan_create", "pfh_plan_destroy",
     "pfh_plan_workspace_bytes", "pfh_plan_layout", "pfh_execute", "pfh_execute_in_place", "pfh_local_execute",
-    "pfh_local_execute_in_place", "pfh_execute_with_timing", "pfh_workspace_take_status", "pfh_workspace_init", "pfh_execute_noalloc", "pfh_batch_create",
+    "pfh_local_execute_in_place", "pfh_execute_with_timing", "pfh_workspace_take_status", "pfh_workspace_init", "pfh_execute_noalloc", "pfh_execute_scaled",
+    "pfh_execute_quadratic", "pfh_batch_create",
     "pfh_batch_destroy", "pfh_batch_workspace_bytes", "pfh_batch_execute", "pfh_batch_tuning",
     "pfh_batch_tuning_source", "pfh_batch_tuning_cache_clear",
     "pfh_pointwise_scale_axes", "pfh_pointwise_scale_axes_complex", "pfh_pointwise_quadratic", "pfh_pointwise_quadratic_adjoint", "pfh_sum_squares",
@@ -220,6 +221,8 @@ def load_library(path: str = LIB_PATH):
     lib.pfh_workspace_take_status.argtypes = [vp, vp, vp]
     lib.pfh_workspace_init.argtypes = [vp, vp, sz, vp]
     lib.pfh_execute_noalloc.argtypes = [vp, i, vp, sz, vp, sz, vp, i]
+    lib.pfh_execute_scaled.argtypes = [vp, i, vp, sz, vp, sz, vp, vp, sz, vp, i]
+    lib.pfh_execute_quadratic.argtypes = [vp, i, vp, sz, vp, sz, ctypes.c_double, vp, sz, vp, i]
     lib.pfh_batch_create.argtypes = [ctypes.POINTER(_Desc), i, i, ctypes.POINTER(vp)]
     lib.pfh_batch_destroy.argtypes = [vp]
     lib.pfh_batch_workspace_bytes.argtypes = [vp, ctypes.POINTER(sz)]
@@ -538,6 +541,21 @@ class _RoutePlan(_Plan):
         w = self._workspace(workspace)
         _check(_lib.pfh_execute(self._h, op, _ptr(src), src.numel(), _ptr(dst), dst.numel(), _ptr(w), w.numel(),
                                 _stream(), flags))
+        return dst
+
+    def execute_scaled(self, op, src, dst, factors, workspace=None, flags=0):
+        """execute, then scale_axes(self, 1, dst, factors) with real factors:
+        one pass less where the last stage applies them at its store."""
+        w = self._workspace(workspace)
+        _check(_lib.pfh_execute_scaled(self._h, op, _ptr(src), src.numel(), _ptr(dst), dst.numel(), _ptr(factors),
+                                       _ptr(w), w.numel(), _stream(), flags))
+        return dst
+
+    def execute_quadratic(self, op, src, dst, a, workspace=None, flags=0):
+        """execute onto the real side, then dst = y + a y^2, likewise."""
+        w = self._workspace(workspace)
+        _check(_lib.pfh_execute_quadratic(self._h, op, _ptr(src), src.numel(), _ptr(dst), dst.numel(), float(a),
+                                          _ptr(w), w.numel(), _stream(), flags))
         return dst
 
     def execute_with_timing(self, op, src, dst=None, workspace=None) -> tuple:

@@ -65,14 +65,18 @@ class PseudoSpectralModel:
 
     def _filtered(self, u: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
         """out = C2R(E * R2C(u))."""
-        self.plan.forward(u, self.spec, self.ws)
-        pf.scale_axes(self.plan, 1, self.spec, self.decay)
+        self.plan.execute_scaled(pf.FORWARD, u, self.spec, self.decay, self.ws)
         self.plan.inverse(self.spec, out, self.ws, flags=pf.EXEC_DEFER_STATUS)
         return out
 
     def step(self, u: torch.Tensor, w: torch.Tensor, u_next: torch.Tensor):
         self._filtered(u, w)
         pf.quadratic(w, self.gamma, out=u_next)
+
+    def advance(self, u: torch.Tensor, u_next: torch.Tensor):
+        """step without w: the quadratic update in the C2R's last pass."""
+        self.plan.execute_scaled(pf.FORWARD, u, self.spec, self.decay, self.ws)
+        self.plan.execute_quadratic(pf.INVERSE, self.spec, u_next, self.gamma, self.ws, flags=pf.EXEC_DEFER_STATUS)
 
     def loss(self, u: torch.Tensor) -> torch.Tensor:
         return pf.sum_squares(u, self.sq_ws)
@@ -95,13 +99,12 @@ class PseudoSpectralModel:
     def forward(self, u0: torch.Tensor) -> Tuple[float, torch.Tensor, List[torch.Tensor]]:
         """Runs the N steps; returns (loss, u_N, checkpoints u_0, u_e, u_2e, ...)."""
         u = u0.clone()
-        w = torch.empty_like(u0)
         nxt = torch.empty_like(u0)
         ckpt = []
         for j in range(self.steps):
             if j % self.every == 0:
                 ckpt.append(u.clone())
-            self.step(u, w, nxt)
+            self.advance(u, nxt)
             u, nxt = nxt, u
         self.plan.take_status(self.ws)
         return float(self.loss(u).item()), u, ckpt
@@ -119,15 +122,17 @@ class PseudoSpectralModel:
             ws_seg = []
             u = ckpt[s].clone()
             nxt = torch.empty_like(u)
-            for _ in range(j0, j1):
+            for j in range(j0, j1):
                 w = torch.empty_like(u)
-                self.step(u, w, nxt)
+                if j + 1 < j1:
+                    self.step(u, w, nxt)
+                else:  # the reverse sweep needs the last w only
+                    self._filtered(u, w)
                 ws_seg.append(w)
                 u, nxt = nxt, u
             for j in range(j1 - 1, j0 - 1, -1):
                 pf.quadratic_adjoint(ws_seg[j - j0], g, self.gamma, out=gw)
-                self.plan.adjoint_inverse(gw, spec, self.ws)
-                pf.scale_axes(self.plan, 1, spec, self.decay)
+                self.plan.execute_scaled(pf.ADJOINT_INVERSE, gw, spec, self.decay, self.ws)
                 self.plan.adjoint_forward(spec, g, self.ws)
         self.plan.take_status(self.ws)
         return g

@@ -50,3 +50,29 @@ def test_scale_axes_rows(gpu, shape, dt):
             ref = ref * v.reshape([1] + [-1 if q == pos else 1 for q in range(3)])
         # three products, each within one rounding per component (complex: three)
         assert rel_l2(got, ref) <= 16 * np.finfo(dt).eps, (side, cf)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float64])
+@pytest.mark.parametrize("permute", [True, False])
+@pytest.mark.parametrize("shape,extra", [((45, 20, 24), ()), ((30, 35, 50), (2,)), ((17, 12, 21), ()), ((11, 9, 16), (3,))])
+def test_steps_folded_into_the_last_stage(gpu, shape, extra, permute, dt):
+    """execute_scaled / execute_quadratic against the two separate calls:
+    last axes with a line plan (folded), on Bluestein and on the generic
+    kernel (two steps). The factors are multiplied in the same order with
+    permuted output and to within a rounding or two otherwise."""
+    plan = pf.R2cPlan(shape, dtype=dt, extra_shape=extra, permute_dims=permute)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(shape[0])
+    x = torch.randn(plan.input_elements(), generator=g, device="cuda", dtype=dt)
+    f = torch.rand(shape[0] + shape[1] + shape[2] // 2 + 1, generator=g, device="cuda", dtype=dt) + 0.5
+    eps = torch.finfo(dt).eps
+    for op in (pf.FORWARD, pf.ADJOINT_INVERSE, pf.ADJOINT_BACKWARD):
+        ref = pf.scale_axes(plan, 1, plan.execute(op, x), f)
+        got = plan.execute_scaled(op, x, torch.empty_like(ref), f)
+        assert torch.linalg.norm(got - ref) <= (0 if permute else 4 * eps) * torch.linalg.norm(ref), op
+    spec = plan.forward(x)
+    for op in (pf.INVERSE, pf.BACKWARD, pf.ADJOINT_FORWARD):
+        ref = pf.quadratic(plan.execute(op, spec), 0.25)
+        got = plan.execute_quadratic(op, spec, torch.empty_like(ref), 0.25)
+        # a y y as one fused multiply-add or as two roundings
+        assert torch.linalg.norm(got - ref) <= 2 * eps * torch.linalg.norm(ref), op
