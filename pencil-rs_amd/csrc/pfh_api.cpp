@@ -340,21 +340,24 @@ static int env_int(const char *name, int dflt)
 }
 
 // The line plan (k_line_plan) of an FFT length; radices 0 if there is none.
-static void find_line_plan(int m, int tbytes, int r[3], int &em)
+static void find_line_plan(int m, int tbytes, int r[3], int &em, bool real_modes = false)
 {
     using Entry = std::array<int, 4>;
-    static const std::map<int, Entry> plans[2] = {
-#define PFH_LINE_F32(TT, A, B, C, E) {sizeof(TT) == 4 ? (A) * (B) * ((C) ? (C) : 1) : 0, {A, B, C, E}},
-#define PFH_LINE_F64(TT, A, B, C, E) {sizeof(TT) == 8 ? (A) * (B) * ((C) ? (C) : 1) : 0, {A, B, C, E}},
-        {PFH_FAST_ROUTE_PLANS(PFH_LINE_F32)},
-        {PFH_FAST_ROUTE_PLANS(PFH_LINE_F64)},
-#undef PFH_LINE_F32
-#undef PFH_LINE_F64
-    };
+    using Table = std::map<int, Entry>;
+    // [precision][0: every kind, 1: the real-to-real modes' own variants]
+    static const std::array<std::array<Table, 2>, 2> plans = [] {
+        std::array<std::array<Table, 2>, 2> t;
+#define PFH_LINE_ADD(TT, A, B, C, E) \
+    t[sizeof(TT) == 4 ? 0 : 1][line_plan_real_only(A, B, C, E) ? 1 : 0][(A) * (B) * ((C) ? (C) : 1)] = {A, B, C, E};
+        PFH_FAST_ROUTE_PLANS(PFH_LINE_ADD)
+#undef PFH_LINE_ADD
+        return t;
+    }();
     r[0] = 0;
-    const std::map<int, Entry> &t = plans[tbytes == 4 ? 0 : 1];
+    const std::array<Table, 2> &own = plans[tbytes == 4 ? 0 : 1];
+    const Table &t = real_modes && own[1].count(m) ? own[1] : own[0];
     const auto it = t.find(m);
-    if (m < 2 || it == t.end()) return;
+    if (it == t.end()) return;
     for (int i = 0; i < 3; ++i) r[i] = it->second[i];
     em = it->second[3];
 }
@@ -396,7 +399,7 @@ static bool choose_line_plan(Step &st, int tbytes, bool in_stage)
     const bool odd = st.mode == M_R2C_ODD || st.mode == M_C2R_ODD;
     if (!(st.mode == M_C2C || st.mode == M_R2C || st.mode == M_C2R || odd || dht || r2r)) return false;
     int r[3], em = 0;
-    find_line_plan(st.m, tbytes, r, em);
+    find_line_plan(st.m, tbytes, r, em, r2r);
     if (r2r && st.m > kLinePlanRealMax) r[0] = 0;
     st.blue = 0;
     // a length without a plan: Bluestein in the workgroup. Below 16 points the
@@ -780,8 +783,7 @@ static pfh_status size_line_plan(Step &st, const DeviceInfo &dev, int tbytes, co
                                    st.out_col ? (st.out_cplx ? 128 / cb : 64 / tbytes) : 1);
         while (lt / 2 >= least && lds_of(lt) > dev.lds_limit / 2) lt /= 2;
     } else {
-        static const int row_threads = env_int("PFH_ROW_THREADS", 256);
-        lt = (int)std::max<int64_t>(1, std::min<int64_t>(row_threads / tpl, st.nlines));
+        lt = (int)std::max<int64_t>(1, std::min<int64_t>(256 / tpl, st.nlines));
     }
     while (lt > 1 && lds_of(lt) > dev.lds_limit) lt /= 2;
     if (lds_of(lt) > dev.lds_limit) return set_err(PFH_ERR_UNSUPPORTED, "line does not fit in LDS");

@@ -282,7 +282,8 @@ hipError_t launch_line_blue<LineT, PFH_LINE_KIND>(const StageArgs<LineT> &a, int
                                                   size_t lds_bytes, int64_t grid, hipStream_t s)
 {
 #define PFH_BLUE_CASE(TT, A, B, C, E)                                                                      \
-    if constexpr (sizeof(TT) == sizeof(LineT) && blue_length((A) * (B) * ((C) ? (C) : 1)))                 \
+    if constexpr (sizeof(TT) == sizeof(LineT) && blue_length((A) * (B) * ((C) ? (C) : 1)) &&               \
+                  !line_plan_real_only(A, B, C, E))                                                        \
         if (r0 == A && r1 == B && r2 == C && em == E)                                                      \
             return launch_blue<LineT, A, B, C, E, PFH_LINE_KIND>(a, threads, lds_bytes, grid, s);
     PFH_FAST_ROUTE_PLANS(PFH_BLUE_CASE)

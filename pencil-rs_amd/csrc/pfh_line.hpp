@@ -27,6 +27,13 @@ __host__ __device__ constexpr int line_plan_tpl(int r0, int r1, int r2, int em)
     return t;
 }
 
+// A plan whose values per thread are below its largest radix is a variant for
+// the real-to-real modes (k_line_plan KIND 2): twice the threads per line.
+__host__ __device__ constexpr bool line_plan_real_only(int r0, int r1, int r2, int em)
+{
+    return em < r0 || em < r1 || em < r2;
+}
+
 // LDS stride of a line (complex values, odd): between passes the line is kept
 // as m / r0 rows of r0 values at the odd row stride r0 | 1, before the first
 // and after the last pass as m (+ 1) values in natural order.

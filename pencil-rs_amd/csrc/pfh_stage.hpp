@@ -515,7 +515,27 @@ struct PlaneArgs {
     X(double, 5, 14, 14, 15)   \
     X(double, 10, 10, 10, 10)  \
     X(double, 7, 12, 12, 14)   \
-    X(double, 8, 8, 16, 16)
+    X(double, 8, 8, 16, 16)      \
+    X(float, 6, 12, 0, 6)        \
+    X(float, 5, 14, 0, 5)        \
+    X(float, 5, 15, 0, 5)        \
+    X(float, 7, 12, 0, 7)        \
+    X(float, 8, 12, 0, 8)        \
+    X(float, 7, 14, 0, 7)        \
+    X(float, 7, 15, 0, 7)        \
+    X(float, 8, 14, 0, 8)        \
+    X(float, 8, 15, 0, 8)        \
+    X(float, 8, 16, 0, 8)        \
+    X(double, 6, 12, 0, 6)       \
+    X(double, 5, 14, 0, 5)       \
+    X(double, 5, 15, 0, 5)       \
+    X(double, 7, 12, 0, 7)       \
+    X(double, 8, 12, 0, 8)       \
+    X(double, 7, 14, 0, 7)       \
+    X(double, 7, 15, 0, 7)       \
+    X(double, 8, 14, 0, 8)       \
+    X(double, 8, 15, 0, 8)       \
+    X(double, 8, 16, 0, 8)
 
 // Plans of k_line_fast and the batched kernels: {R0, R1, R2, EM}.
 #define PFH_FAST_PLANS(X)      \
