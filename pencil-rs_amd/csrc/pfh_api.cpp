@@ -399,7 +399,9 @@ static bool choose_line_plan(Step &st, int tbytes, bool in_stage)
     const bool odd = st.mode == M_R2C_ODD || st.mode == M_C2R_ODD;
     if (!(st.mode == M_C2C || st.mode == M_R2C || st.mode == M_C2R || odd || dht || r2r)) return false;
     int r[3], em = 0;
-    find_line_plan(st.m, tbytes, r, em, r2r);
+    // (f64 half-complex stages take the variants too: 256 x 384 x 240 f64 DHT
+    // forward + inverse 444 -> 415 us on MI355X; f32 ones gain nothing)
+    find_line_plan(st.m, tbytes, r, em, r2r || (tbytes == 8 && st.mode != M_C2C));
     if (r2r && st.m > kLinePlanRealMax) r[0] = 0;
     st.blue = 0;
     // a length without a plan: Bluestein in the workgroup. Below 16 points the

@@ -559,8 +559,9 @@ hipError_t launch_line_plan<LineT, PFH_LINE_KIND>(const StageArgs<LineT> &a, int
 {
 #define PFH_LINE_CASE(TT, A, B, C, E)                                                                      \
     if constexpr (sizeof(TT) == sizeof(LineT) &&                                                           \
-                  (PFH_LINE_KIND == 2 ? (A) * (B) * ((C) ? (C) : 1) <= kLinePlanRealMax                   \
-                                      : !line_plan_real_only(A, B, C, E)))                              \
+                  (PFH_LINE_KIND == 2   ? (A) * (B) * ((C) ? (C) : 1) <= kLinePlanRealMax                 \
+                   : (PFH_LINE_KIND == 1 || PFH_LINE_KIND == 6) && sizeof(TT) == 8 ? true                \
+                                        : !line_plan_real_only(A, B, C, E)))                            \
         if (r0 == A && r1 == B && r2 == C && em == E)                                                      \
             return launch_one<LineT, A, B, C, E, PFH_LINE_KIND>(a, threads, lds_bytes, grid, s);
     PFH_FAST_ROUTE_PLANS(PFH_LINE_CASE)
