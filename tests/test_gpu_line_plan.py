@@ -71,6 +71,22 @@ def test_real_kinds_on_row_lines(gpu, kind, dt):
 
 
 @pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("kind", [4, 8])
+@pytest.mark.parametrize("m", [70, 72, 75, 84, 96, 98, 105, 112, 120, 128])
+def test_type_four_lines_on_either_plan(gpu, m, kind, dt):
+    """DCT-IV / DST-IV lines of 2m points: the plan that every kind shares where
+    12 divides m, the one with twice the threads elsewhere; one partial tile
+    and several."""
+    rng = np.random.default_rng(m)
+    for lines in (3, 67):
+        x = uniform_real(rng, (lines, 2 * m), dt)
+        plan = pf.LocalR2rPlan(2 * m, kind, dtype=torch.from_numpy(x).dtype)
+        for op, fn in ((O.FORWARD, plan.forward), (O.INVERSE, plan.inverse)):
+            ref = O.r2r_lines(x.astype(np.float64), kind, op)
+            assert rel_l2(_host(fn(_tdev(x))), ref) <= tol(dt), (lines, op)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("permute", [True, False])
 @pytest.mark.parametrize("kinds", [(1, 2, 3), (4, 5, 6), (7, 8, 9), (9, 1, 5)])
 def test_real_kinds_on_column_sides(gpu, kinds, permute, dt):
