@@ -3055,10 +3055,14 @@ struct PostStep {
     double quad;
 };
 
-// Can the operation's last stage apply the step at its store?
+// Can the operation's last stage apply the step at its store? Its factors are
+// the point's and one per line digit; an axis of extent 1 is no digit
+// (step_geometry), so arrays with one take the separate pass.
 static bool can_fuse(const OpPlan &o, const PostStep &post)
 {
     if (o.steps.empty() || !o.pairs.empty()) return false;
+    for (int a = 0; post.factors && a < o.out.N; ++a)
+        if (o.out.shape[a] == 1) return false;
     const Step &s = o.steps.back();
     if (!s.line_plan || s.blue || !s.pieces.empty()) return false;
     return post.factors ? s.mode == M_C2C : (s.mode == M_C2R || s.mode == M_C2R_ODD);

@@ -426,6 +426,25 @@ static void emulate_math(const char *what, const StageArgs<T> &a)
     }
 }
 
+// Factor of point k of a line in a stage that folds per-axis factors into its
+// store (k_line_plan KIND 5): the point's, then each line digit's.
+template <typename T>
+static T axis_factor(const char *what, const StageArgs<T> &a, int64_t line, int k)
+{
+    const T *p = a.sfac + a.sfac_pt + k;
+    if (!check_read("axis factors", p, sizeof(T))) return (T)0;
+    T f = *p;
+    for (int d = 0; d < a.g.nd; ++d) {
+        const int64_t c = line % a.g.ext[d];
+        line /= a.g.ext[d];
+        if (a.sfac_dig[d] < 0) continue;
+        p = a.sfac + a.sfac_dig[d] + c;
+        if (!check_read(what, p, sizeof(T))) return (T)0;
+        f *= *p;
+    }
+    return f;
+}
+
 // identity-on-points emulation of one line stage
 template <typename T>
 static void emulate(const char *what, const StageArgs<T> &a)
@@ -453,7 +472,13 @@ static void emulate(const char *what, const StageArgs<T> &a)
             char *p = static_cast<char *>(a.dst) + (oo + (int64_t)k * a.ops) * (int64_t)eo;
             if (!check_write(what, p, eo)) return;
             T *v = reinterpret_cast<T *>(p);
-            const T r = k < a.nin ? re[k] : (T)0, i = k < a.nin ? im[k] : (T)0;
+            T r = k < a.nin ? re[k] : (T)0, i = k < a.nin ? im[k] : (T)0;
+            if (a.flags & F_AXIS_SCALE) {
+                const T f = axis_factor(what, a, line, k);
+                r *= f;
+                i *= f;
+            }
+            if (a.flags & F_QUADRATIC) r = r + a.quad * r * r;
             v[0] = r;
             if (co) v[1] = (a.mode == M_R2C || a.mode == M_R2C_ODD) ? (T)0 : i;
         }
@@ -1992,6 +2017,81 @@ void route_long_case(std::vector<size_t> shape, size_t extra, int op, double tol
     pfh_plan_destroy(p);
 }
 
+// pfh_execute_scaled / pfh_execute_quadratic against the operation followed by
+// the pointwise call, bit for bit: permuted outputs, extras, and axes of extent
+// 1 (which no line digit stands for) in each position.
+template <typename T>
+void fold_case(int kind, std::vector<size_t> shape, size_t extra, bool permute)
+{
+    const int nd = (int)shape.size();
+    char name[112];
+    std::snprintf(name, sizeof name, "fold kind %d %zux%zux%zu%s extra %zu %s %s", kind, shape[0], shape[1], shape[2],
+                  nd > 3 ? " 4d" : "", extra, sizeof(T) == 4 ? "f32" : "f64", permute ? "permuted" : "strided");
+    const int before = g_fail;
+    pfh_desc d = route_desc(kind, sizeof(T) == 4 ? PFH_F32 : PFH_F64, shape,
+                            extra > 1 ? std::vector<size_t>{extra} : std::vector<size_t>{});
+    d.permute_dims = permute ? 1 : 0;
+    pfh_plan p = nullptr;
+    if (pfh_plan_create(&d, &p) != PFH_OK) {
+        fail("%s: plan creation", name);
+        return;
+    }
+    const Arr side[2] = {layout(p, 0, nd), layout(p, 1, nd)};
+    const bool r2c = kind == PFH_R2C;
+    int64_t nf = 0;
+    for (int64_t v : side[1].shape) nf += v;
+    T *f = static_cast<T *>(dmalloc((size_t)nf * sizeof(T)));
+    for (int64_t i = 0; i < nf; ++i) f[i] = (T)(1.25 + 0.5 * urand());
+    auto run = [&](int op, bool folded, bool quad) {
+        const bool fwd = op == PFH_FORWARD || op == PFH_ADJOINT_INVERSE || op == PFH_ADJOINT_BACKWARD;
+        const Arr &in = side[fwd ? 0 : 1], &out = side[fwd ? 1 : 0];
+        char *src = static_cast<char *>(dmalloc((size_t)(in.elems * in.eb)));
+        char *dst = static_cast<char *>(dmalloc((size_t)(out.elems * out.eb)));
+        for (int64_t i = 0; i < in.elems * in.eb / (int64_t)sizeof(T); ++i)
+            reinterpret_cast<T *>(src)[i] = (T)((i * 7919) % 1009) / (T)512 - (T)1;
+        size_t wsb = 0;
+        pfh_plan_workspace_bytes(p, op, &wsb);
+        void *ws = dmalloc(wsb ? wsb : 1, true);
+        pfh_status st;
+        if (folded && quad) {
+            st = pfh_execute_quadratic(p, op, src, in.elems, dst, out.elems, 0.25, ws, wsb, nullptr, 0);
+        } else if (folded) {
+            st = pfh_execute_scaled(p, op, src, in.elems, dst, out.elems, f, ws, wsb, nullptr, 0);
+        } else {
+            st = pfh_execute(p, op, src, in.elems, dst, out.elems, ws, wsb, nullptr, 0);
+            if (!st && quad) st = pfh_pointwise_quadratic(d.precision, dst, dst, out.elems, 0.25, nullptr);
+            if (!st && !quad) st = pfh_pointwise_scale_axes(p, 1, dst, out.elems, f, nullptr);
+        }
+        if (st) fail("%s op %d: status %d", name, op, (int)st);
+        std::vector<char> got(dst, dst + out.elems * out.eb);
+        for (void *q : {(void *)src, (void *)dst, ws}) (void)hipFree(q);
+        return got;
+    };
+    for (int op : {PFH_FORWARD, PFH_ADJOINT_INVERSE, PFH_ADJOINT_BACKWARD})
+        if (run(op, true, false) != run(op, false, false)) fail("%s op %d: factors differ from two calls", name, op);
+    if (r2c)
+        for (int op : {PFH_INVERSE, PFH_BACKWARD, PFH_ADJOINT_FORWARD})
+            if (run(op, true, true) != run(op, false, true)) fail("%s op %d: quadratic step differs", name, op);
+    (void)hipFree(f);
+    pfh_plan_destroy(p);
+    std::printf("%s: %s\n", name, g_fail == before ? "ok" : "FAILED");
+}
+
+void fold_cases()
+{
+    for (int kind : {PFH_C2C, PFH_R2C})
+        for (bool permute : {true})
+            for (size_t extra : {1, 3}) {
+                for (const std::vector<size_t> &s : std::vector<std::vector<size_t>>{
+                         {16, 12, 20}, {16, 1, 32}, {16, 20, 1}, {1, 16, 24}, {64, 1, 48}, {1, 1, 18}, {11, 9, 16}}) {
+                    if (kind == PFH_R2C && s[2] == 1) continue; // no half-complex axis
+                    fold_case<double>(kind, s, extra, permute);
+                    fold_case<float>(kind, s, extra, permute);
+                }
+                fold_case<double>(kind, {8, 6, 5, 10}, extra, permute);
+            }
+}
+
 void long_cases()
 {
     const int before = g_fail;
@@ -2146,6 +2246,11 @@ int main(int argc, char **argv)
 {
     if (argc == 2 && std::strcmp(argv[1], "long") == 0) {
         long_cases();
+        std::printf("launches %d, failures %d\n", pfh::g_launches, g_fail);
+        return g_fail ? 1 : 0;
+    }
+    if (argc == 2 && std::strcmp(argv[1], "fold") == 0) {
+        fold_cases();
         std::printf("launches %d, failures %d\n", pfh::g_launches, g_fail);
         return g_fail ? 1 : 0;
     }

@@ -72,3 +72,13 @@ def test_long_lines_against_naive_sums(emu):
     r = subprocess.run([emu, "long"], capture_output=True, text=True, timeout=900)
     assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-2000:]
     assert "long lines: ok" in r.stdout
+
+
+def test_folded_steps_equal_two_calls(emu):
+    """execute_scaled / execute_quadratic, folded into the last stage or not,
+    against the operation followed by the pointwise call, bit for bit: extras
+    and axes of extent 1 in every position, whose factors count too."""
+    r = subprocess.run([emu, "fold"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-2000:]
+    lines = [l for l in r.stdout.splitlines() if l.endswith(": ok") or l.endswith(": FAILED")]
+    assert len(lines) > 20 and all(l.endswith(": ok") for l in lines)
