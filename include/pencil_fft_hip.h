@@ -316,7 +316,7 @@ pfh_status pfh_local_execute_in_place(pfh_plan plan, int op, void *data, size_t 
                                       void *workspace, size_t workspace_bytes, pfh_stream_t stream, int flags);
 
 /* An operation and the pointwise step that follows it, in the operation's last
- * pass where that stage can carry it, as two steps otherwise (the same results).
+ * pass where that stage can carry it, as two steps otherwise (the same bits).
  * pfh_execute_scaled: pfh_execute, then pfh_pointwise_scale_axes of dst by real
  * per-axis factors (the complex side of the plan: FORWARD, ADJOINT_INVERSE and
  * ADJOINT_BACKWARD). pfh_execute_quadratic: pfh_execute into a real dst, then

@@ -2813,7 +2813,13 @@ static pfh_status launch_step_ptrs(const PlanImpl &P, const Step &s, const void 
             a.flags |= F_AXIS_SCALE;
             a.sfac = static_cast<const T *>(wv.factors);
             a.sfac_pt = wv.foff[s.axis];
-            for (int d = 0; d < kMaxDigits; ++d) a.sfac_dig[d] = s.digit_axis[d] >= 0 ? wv.foff[s.digit_axis[d]] : -1;
+            for (int d = 0; d < kMaxDigits; ++d) {
+                a.sfac_dig[d] = s.digit_axis[d] >= 0 ? wv.foff[s.digit_axis[d]] : -1;
+                if (a.sfac_dig[d] < 0) continue;
+                a.sfac_pre += s.g.os[d] < s.ops ? 1 : 0;
+                for (int e = 0; e < s.g.nd; ++e)
+                    if (s.digit_axis[e] >= 0 && s.g.os[e] < s.g.os[d]) ++a.sfac_rank[d];
+            }
         } else {
             a.flags |= F_QUADRATIC;
             a.quad = (T)wv.quad;

@@ -376,21 +376,36 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
             }
         }
     } else if constexpr (KIND == 5) {
-        // the product of factors in scale_axes' order: the stage's axis, then
-        // the line digits (ascending strides)
+        // the factors multiplied as scale_axes does, in the order of the
+        // output's strides (q: the digits' by rank, the first sfac_pre of them
+        // before the point's), so that both give the same bits
         constexpr int NL = P::template rounds<RL>(), NB = M / RL;
         if (!store) return;
         cpx<T> v[NL][RL];
         P::last(oln, twl, ot, v);
-        T fd[kMaxDigits];
+        T q[kMaxDigits];
+#pragma unroll
+        for (int r = 0; r < kMaxDigits; ++r) q[r] = (T)1;
         uint32_t x = tile0 + (uint32_t)ol;
 #pragma unroll
         for (int d = 0; d < kMaxDigits; ++d) {
-            fd[d] = (T)1;
             if (d < a.g.nd) {
-                const uint32_t q = fastdiv(x, a.g.dmag[d], a.g.dsh[d]);
-                if (a.sfac_dig[d] >= 0) fd[d] = a.sfac[(uint32_t)a.sfac_dig[d] + x - q * (uint32_t)a.g.ext[d]];
-                x = q;
+                const uint32_t y = fastdiv(x, a.g.dmag[d], a.g.dsh[d]);
+                if (a.sfac_dig[d] >= 0) {
+                    const T f = a.sfac[(uint32_t)a.sfac_dig[d] + x - y * (uint32_t)a.g.ext[d]];
+#pragma unroll
+                    for (int r = 0; r < kMaxDigits; ++r)
+                        if (a.sfac_rank[d] == r) q[r] = f;
+                }
+                x = y;
+            }
+        }
+        T pre = (T)1;
+#pragma unroll
+        for (int r = 0; r < kMaxDigits; ++r) {
+            if (r < a.sfac_pre) {
+                pre *= q[r];
+                q[r] = (T)1;
             }
         }
         const uint32_t st = (uint32_t)a.ops * (uint32_t)(2 * sizeof(T));
@@ -402,10 +417,10 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
             if (P::template has<RL>(b, ot + TPL * b)) {
 #pragma unroll
                 for (int r = 0; r < RL; ++r) {
-                    T f = fp[b * TPL + r * NB];
+                    T f = pre * fp[b * TPL + r * NB];
 #pragma unroll
                     for (int d = 0; d < kMaxDigits; ++d)
-                        if (d < a.g.nd) f *= fd[d];
+                        if (d < a.g.nd) f *= q[d];
                     gwrite<cpx<T>>(dst, off + (uint32_t)(b * TPL + r * NB) * st, mk(v[b][r].x * sc * f, v[b][r].y * sy * f));
                 }
             }
@@ -429,7 +444,8 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
     } else if constexpr (KIND == 1 || KIND == 6) {
         auto fin = [&](T y) {
             y = y * sc;
-            if constexpr (KIND == 6) y = y + a.quad * y * y;
+            // (one fused multiply-add of the rounded y, as k_quadratic computes it)
+            if constexpr (KIND == 6) y = fma(a.quad * y, y, y);
             return y;
         };
         if ((M & 1) && a.n == M) {

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kBlock) void k_quadratic(const T *w, T *u, int64_t 
         if (b + k * kBlock < n) v[k] = w[b + k * kBlock];
 #pragma unroll
     for (int k = 0; k < kUnroll; ++k)
-        if (b + k * kBlock < n) u[b + k * kBlock] = v[k] + a * v[k] * v[k];
+        if (b + k * kBlock < n) u[b + k * kBlock] = fma(a * v[k], v[k], v[k]);
 }
 
 // out = g (1 + 2 a w): the transpose of the quadratic step's derivative

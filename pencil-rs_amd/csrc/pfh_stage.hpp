@@ -176,6 +176,9 @@ struct StageArgs {
     // Pointwise steps in the last stage's store (k_line_plan KIND 5 and 6).
     const T *sfac;          // per-axis factors (F_AXIS_SCALE): point k's at sfac_pt + k, digit d's at sfac_dig[d] + coordinate
     int sfac_pt, sfac_dig[kMaxDigits]; // (sfac_dig < 0: no factor)
+    // the order of the products is launch_scale_axes': ascending output strides. Rank of each digit among the
+    // digits, and how many of them come before the point
+    int sfac_rank[kMaxDigits], sfac_pre;
     T quad;                 // y + quad y^2 (F_QUADRATIC)
 };
 

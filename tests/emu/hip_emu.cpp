@@ -427,21 +427,28 @@ static void emulate_math(const char *what, const StageArgs<T> &a)
 }
 
 // Factor of point k of a line in a stage that folds per-axis factors into its
-// store (k_line_plan KIND 5): the point's, then each line digit's.
+// store (k_line_plan KIND 5): the point's and each line digit's, multiplied in
+// the order of the output's strides as launch_scale_axes multiplies them.
 template <typename T>
 static T axis_factor(const char *what, const StageArgs<T> &a, int64_t line, int k)
 {
+    T q[kMaxDigits], pre = (T)1, f;
+    for (int d = 0; d < kMaxDigits; ++d) q[d] = (T)1;
+    int64_t x = line;
+    for (int d = 0; d < a.g.nd; ++d) {
+        const int64_t c = x % a.g.ext[d];
+        x /= a.g.ext[d];
+        if (a.sfac_dig[d] < 0) continue;
+        if (a.sfac_rank[d] < 0 || a.sfac_rank[d] >= a.g.nd) fail("%s: rank %d of digit %d", what, a.sfac_rank[d], d);
+        const T *p = a.sfac + a.sfac_dig[d] + c;
+        if (!check_read("axis factors", p, sizeof(T))) return (T)0;
+        q[a.sfac_rank[d]] = *p;
+    }
     const T *p = a.sfac + a.sfac_pt + k;
     if (!check_read("axis factors", p, sizeof(T))) return (T)0;
-    T f = *p;
-    for (int d = 0; d < a.g.nd; ++d) {
-        const int64_t c = line % a.g.ext[d];
-        line /= a.g.ext[d];
-        if (a.sfac_dig[d] < 0) continue;
-        p = a.sfac + a.sfac_dig[d] + c;
-        if (!check_read(what, p, sizeof(T))) return (T)0;
-        f *= *p;
-    }
+    for (int r = 0; r < a.sfac_pre; ++r) pre = r == 0 ? q[r] : pre * q[r];
+    f = a.sfac_pre > 0 ? pre * *p : *p;
+    for (int r = a.sfac_pre; r < kMaxDigits; ++r) f *= q[r];
     return f;
 }
 
@@ -478,7 +485,7 @@ static void emulate(const char *what, const StageArgs<T> &a)
                 r *= f;
                 i *= f;
             }
-            if (a.flags & F_QUADRATIC) r = r + a.quad * r * r;
+            if (a.flags & F_QUADRATIC) r = std::fma(a.quad * r, r, r);
             v[0] = r;
             if (co) v[1] = (a.mode == M_R2C || a.mode == M_R2C_ODD) ? (T)0 : i;
         }
@@ -1085,7 +1092,7 @@ hipError_t launch_quadratic(const void *w, void *u, int64_t n, double a, hipStre
     check_read("quadratic out", u, n * sizeof(T));
     for (int64_t i = 0; i < n; ++i) {
         const T v = static_cast<const T *>(w)[i];
-        static_cast<T *>(u)[i] = v + (T)a * v * v;
+        static_cast<T *>(u)[i] = std::fma((T)a * v, v, v);
     }
     return hipSuccess;
 }
@@ -2018,7 +2025,7 @@ void route_long_case(std::vector<size_t> shape, size_t extra, int op, double tol
 }
 
 // pfh_execute_scaled / pfh_execute_quadratic against the operation followed by
-// the pointwise call, bit for bit: permuted outputs, extras, and axes of extent
+// the pointwise call, bit for bit: every axis order, extras, and axes of extent
 // 1 (which no line digit stands for) in each position.
 template <typename T>
 void fold_case(int kind, std::vector<size_t> shape, size_t extra, bool permute)
@@ -2080,7 +2087,7 @@ void fold_case(int kind, std::vector<size_t> shape, size_t extra, bool permute)
 void fold_cases()
 {
     for (int kind : {PFH_C2C, PFH_R2C})
-        for (bool permute : {true})
+        for (bool permute : {true, false})
             for (size_t extra : {1, 3}) {
                 for (const std::vector<size_t> &s : std::vector<std::vector<size_t>>{
                          {16, 12, 20}, {16, 1, 32}, {16, 20, 1}, {1, 16, 24}, {64, 1, 48}, {1, 1, 18}, {11, 9, 16}}) {
