@@ -522,6 +522,8 @@ class LocalDhtPlan(LocalR2rPlan):
 class _RoutePlan(_Plan):
     """Common execution of the one-rank distributed plans."""
 
+    _axis_points = None  # points of all output axes together (execute_scaled)
+
     def _in_out(self, op):
         fwd_like = op in (FORWARD, ADJOINT_INVERSE, ADJOINT_BACKWARD)
         _, _, in_el, in_b = self.layout(0)
@@ -544,8 +546,21 @@ class _RoutePlan(_Plan):
         return dst
 
     def execute_scaled(self, op, src, dst, factors, workspace=None, flags=0):
-        """execute, then scale_axes(self, 1, dst, factors) with real factors:
-        one pass less where the last stage applies them at its store."""
+        """execute onto the complex side, then scale_axes(self, 1, dst,
+        factors): real factors in one pass less where the last stage applies
+        them at its store, complex ones as the two calls. Factors of another
+        precision or number than the output's axes need are refused."""
+        want = _complex_dtype(self.precision) if factors.is_complex() else _real_dtype(self.precision)
+        if factors.dtype != want:
+            raise TypeError(f"factors of dtype {factors.dtype}, the plan needs {want}")
+        if self._axis_points is None:
+            self._axis_points = sum(self.layout(1)[1])
+        if factors.numel() != self._axis_points:
+            raise ValueError(f"{factors.numel()} factors, the output's axes have {self._axis_points} points")
+        if factors.is_complex():
+            if op not in (FORWARD, ADJOINT_INVERSE, ADJOINT_BACKWARD):
+                raise ValueError("needs an operation onto the complex output side of a plan")
+            return scale_axes(self, 1, self.execute(op, src, dst, workspace, flags), factors)
         w = self._workspace(workspace)
         _check(_lib.pfh_execute_scaled(self._h, op, _ptr(src), src.numel(), _ptr(dst), dst.numel(), _ptr(factors),
                                        _ptr(w), w.numel(), _stream(), flags))

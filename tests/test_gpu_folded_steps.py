@@ -47,3 +47,26 @@ def test_folded_steps_give_the_bits_of_two_calls(gpu, kind, extra, permute, dt):
             ref = pf.quadratic(plan.execute(op, spec), 0.25)
             got = plan.execute_quadratic(op, spec, torch.empty_like(ref), 0.25)
             assert torch.equal(got, ref), (shape, op)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float64])
+def test_factors_the_plan_cannot_take(gpu, dt):
+    """Refused before any launch: another precision, too few or too many
+    factors. Complex factors are the two calls."""
+    other = torch.float64 if dt == torch.float32 else torch.float32
+    plan = pf.C2cPlan((16, 12, 20), dtype=COMPLEX[dt])
+    x = torch.randn(plan.input_elements(), device="cuda", dtype=COMPLEX[dt])
+    dst = torch.zeros_like(x)
+    for bad, error in ((torch.ones(48, device="cuda", dtype=other), TypeError),
+                       (torch.ones(48, device="cuda", dtype=COMPLEX[other]), TypeError),
+                       (torch.ones(47, device="cuda", dtype=dt), ValueError),
+                       (torch.ones(49, device="cuda", dtype=dt), ValueError),
+                       (torch.ones(47, device="cuda", dtype=COMPLEX[dt]), ValueError)):
+        with pytest.raises(error):
+            plan.execute_scaled(pf.FORWARD, x, dst, bad)
+    with pytest.raises(ValueError):
+        plan.execute_scaled(pf.INVERSE, x, dst, torch.ones(48, device="cuda", dtype=COMPLEX[dt]))
+    assert not dst.any()
+    f = torch.randn(48, device="cuda", dtype=COMPLEX[dt])
+    got = plan.execute_scaled(pf.FORWARD, x, dst, f)
+    assert torch.equal(torch.view_as_real(got), torch.view_as_real(pf.scale_axes(plan, 1, plan.forward(x), f)))
