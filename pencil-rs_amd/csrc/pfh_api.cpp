@@ -370,24 +370,30 @@ static void find_line_plan(int m, int tbytes, int r[3], int &em, bool real_modes
     em = e[3];
 }
 
-// Does k_line_blue beat the generic kernel for an FFT length without a line
-// plan? Always for a prime factor of 17 and more, whose generic pass is O(p^2)
-// (MI355X, 2^21 points of C2C lines, f32 / f64 us: n = 97 192 / 215 generic, 18 /
-// 30 Bluestein; 209 73 / 78, 26 / 52). With 11 and 13 the generic kernel has
-// direct butterflies: it keeps products of two of them (143: 18 / 28 against 22 /
-// 35 us) and f64 lengths above 350 (462: 47 against 55 us; 330: 42 against 39).
-static bool blue_pays(int m, int tbytes)
+static int64_t largest_prime_factor(int64_t m);
+
+// Does a stage whose FFT length has no line plan run on k_line_blue? Where its
+// error against 64 bits is no larger than that of the kernels it replaces.
+//  - A prime factor p up to 127 is a direct sum on the generic kernel, whose
+//    rounding grows as sqrt(p); the chirp convolution rounds about as two FFTs of
+//    2m points at any length. Relative L2 error of k_line_blue over the generic
+//    kernel's, mean (largest) of every FFT length 16..512 and every mode, f32 /
+//    f64: p = 11 1.43 (1.75) / 1.43 (1.91), 17 1.29 (1.45) / 1.38 (1.73), 31 1.17
+//    (1.29) / 1.20 (1.37), 47 1.05 (1.12) / 1.11 (1.21), 67 0.91 (1.02) / 0.98
+//    (1.09), 73 0.90 (1.04) / 0.95 (1.12), 79..127 0.82 (0.98) / 0.87 (1.02). So
+//    from 79 on; shorter factors stay on the generic kernel (209 = 11 x 19: 73 / 78
+//    us for 2^21 points on MI355X, Bluestein 26 / 52; n = 97: 192 / 215 generic, 18 /
+//    30 Bluestein).
+//  - Larger ones run as the pieces of a Bluestein line otherwise, with the same
+//    error on average (1.00 / 1.00; symmetric lines, odd C2R, DCT-I and DST-I,
+//    scatter by up to 25% with the convolution length on either side, mean 1.01 /
+//    1.00) except for C2R of even length, 1.29 (1.55) / 1.32 (1.48): those stay
+//    pieces.
+constexpr int kBluePrime = 79;
+static bool blue_pays(int m, int mode)
 {
-    int wide = 0, rest = m;
-    for (int p : {11, 13})
-        while (rest % p == 0) {
-            rest /= p;
-            ++wide;
-        }
-    for (int p : {2, 3, 5, 7})
-        while (rest % p == 0) rest /= p;
-    if (rest > 1) return true;
-    return wide < 2 && (tbytes == 4 || m <= 350);
+    const int64_t p = largest_prime_factor(m);
+    return p >= kBluePrime && (p < 128 || mode != M_C2R);
 }
 
 // k_line_plan for a stage whose mode and FFT length it has: radices, values
@@ -412,12 +418,11 @@ static bool choose_line_plan(Step &st, int tbytes, bool in_stage)
     find_line_plan(st.m, tbytes, r, em, r2r || (tbytes == 8 && st.mode != M_C2C), st.mode == M_DCT4);
     if (r2r && st.m > kLinePlanRealMax) r[0] = 0;
     st.blue = 0;
-    // a length without a plan: Bluestein in the workgroup. Below 16 points the
-    // generic kernel's single pass stays. (PFH_BLUESTEIN_PRIME, a request for
-    // the pieces of long lines, turns it off.)
+    // a length without a plan: Bluestein in the workgroup. (PFH_BLUESTEIN_PRIME,
+    // a request for the pieces of long lines, turns it off.)
     static const int blue = env_int("PFH_LINE_BLUE", 1);
-    if (r[0] == 0 && blue && in_stage && std::getenv("PFH_BLUESTEIN_PRIME") == nullptr && st.m >= 16 && st.m <= kBlueMax &&
-        blue_pays(st.m, tbytes)) {
+    if (r[0] == 0 && blue && in_stage && std::getenv("PFH_BLUESTEIN_PRIME") == nullptr && st.m <= kBlueMax &&
+        blue_pays(st.m, st.mode)) {
         for (int M = 2 * st.m - 1; M <= 1024 && r[0] == 0; ++M)
             if (blue_length(M)) {
                 find_line_plan(M, tbytes, r, em);

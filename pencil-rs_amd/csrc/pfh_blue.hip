@@ -1,5 +1,6 @@
-// k_line_blue: stages whose FFT length m has no line plan (a prime factor of
-// 11 and more), as Bluestein's chirp convolution inside one workgroup.
+// k_line_blue: stages whose FFT length m has no line plan and a prime factor of
+// 79 and more (blue_pays in pfh_api.cpp), as Bluestein's chirp convolution inside
+// one workgroup.
 //
 // With c_j = exp(-i pi j^2 / m) and b_t = exp(+i pi t^2 / m),
 //   Z_k = c_k sum_j (x_j c_j) b_{k-j},
@@ -9,8 +10,7 @@
 // memory once. It costs two FFTs of about 2.1 m points, some 270 lane
 // instructions per complex value in f32; the generic kernel's O(p^2) pass for
 // a prime factor p costs 8 p and its own index arithmetic. MI355X, 2^21 points
-// of f32 / f64 C2C lines, before and after: n = 97 192 / 215 -> 18 / 30 us, 209
-// 73 / 78 -> 26 / 52 us, 319 102 / 111 -> 24 / 40 us.
+// of f32 / f64 C2C lines, generic and here: n = 97 192 / 215 -> 18 / 30 us.
 // Every mode of the line kernels runs here, its pre-processing placing the
 // length-m FFT input in natural order in LDS.
 // Compiled once per precision and kind (PFH_LINE_F64, PFH_LINE_KIND).

@@ -52,13 +52,11 @@ __host__ __device__ constexpr int line_plan_stride(int r0, int r1, int r2)
 constexpr int kLinePlanRealMax = 512;
 
 // Convolution lengths of k_line_blue, among the line plans' lengths: steps of
-// at most 20%, FFT lengths m up to kBlueMax.
+// at most 20% from 160 on (its FFT lengths m are 79 to kBlueMax).
 __host__ __device__ constexpr bool blue_length(int M)
 {
-    return M == 32 || M == 36 || M == 40 || M == 48 || M == 56 || M == 64 || M == 72 || M == 80 || M == 90 || M == 100 ||
-           M == 112 || M == 128 || M == 144 || M == 160 || M == 180 || M == 196 || M == 210 || M == 225 || M == 240 ||
-           M == 256 || M == 288 || M == 320 || M == 360 || M == 400 || M == 450 || M == 512 || M == 600 || M == 700 ||
-           M == 800 || M == 900 || M == 1024;
+    return M == 160 || M == 180 || M == 196 || M == 210 || M == 225 || M == 240 || M == 256 || M == 288 || M == 320 ||
+           M == 360 || M == 400 || M == 450 || M == 512 || M == 600 || M == 700 || M == 800 || M == 900 || M == 1024;
 }
 constexpr int kBlueMax = 512;
 

@@ -503,6 +503,7 @@ static void check_grid(const char *what, const StageArgs<T> &a, int64_t grid)
 }
 
 int g_launches = 0;
+int g_blue_launches = 0;         // stages on k_line_blue
 int g_all_launches = 0;         // every device launch, fills included
 bool g_reject_endpoints = false; // the emulated C2R boundary check rejects every spectrum
 static const bool g_trace = std::getenv("PFH_EMU_TRACE") != nullptr;
@@ -703,6 +704,7 @@ hipError_t launch_line_fast(const StageArgs<T> &a, int r0, int r1, int r2, int e
     ++g_launches;
     ++g_all_launches;
     begin_launch();
+    if (a.flags & F_LINE_BLUE) ++g_blue_launches;
     if (threads > 512) fail("line_fast: %d threads", threads);
     if (!fast_plan_available((int)sizeof(T), r0, r1, r2, em)) fail("line_fast: plan not instantiated");
     if (a.radix[0] != r0 || a.radix[1] != r1 || (r2 && a.radix[2] != r2)) fail("line_fast: radices differ");
@@ -2099,6 +2101,77 @@ void fold_cases()
             }
 }
 
+// Which kernel a line without a plan takes: the generic one for prime factors
+// up to 73, k_line_blue from 79 on, the pieces of a long line for C2R lines of
+// even length with a factor above 127. Identity arithmetic.
+template <typename T>
+void blue_route(int kind, int r2r, int64_t n, int op, int64_t m, int want)
+{
+    pfh_desc d;
+    std::memset(&d, 0, sizeof d);
+    d.kind = kind;
+    d.precision = sizeof(T) == 4 ? PFH_F32 : PFH_F64;
+    d.line_len = (size_t)n;
+    d.r2r_kind = r2r;
+    pfh_plan p = nullptr;
+    if (pfh_plan_create(&d, &p) != PFH_OK) {
+        fail("blue route: plan of %" PRId64 " points", n);
+        return;
+    }
+    const bool r2c = kind == PFH_LOCAL_R2C, c2r = r2c && op == PFH_INVERSE, cplx = kind == PFH_LOCAL_C2C;
+    const int64_t lin = c2r ? n / 2 + 1 : n, lout = (r2c && !c2r) ? n / 2 + 1 : n, batch = 3;
+    size_t wsb = 0;
+    pfh_plan_workspace_bytes(p, op, &wsb);
+    void *src = dmalloc((size_t)(batch * lin) * (cplx || c2r ? 2 : 1) * sizeof(T), true);
+    void *dst = dmalloc((size_t)(batch * lout) * (cplx || (r2c && !c2r) ? 2 : 1) * sizeof(T));
+    void *ws = dmalloc(wsb ? wsb : 1, true);
+    const int l0 = pfh::g_launches, b0 = pfh::g_blue_launches;
+    const pfh_status st = pfh_local_execute(p, op, src, (size_t)(batch * lin), dst, (size_t)(batch * lout), ws, wsb,
+                                            nullptr, 0);
+    const int blue = pfh::g_blue_launches - b0, lines = pfh::g_launches - l0 - (c2r ? 1 : 0); // (the endpoint check)
+    const int got = blue == 1 && lines == 1 ? 1 : lines > 1 && blue == 0 ? 2 : blue == 0 ? 0 : -1;
+    if (st != PFH_OK || got != want)
+        fail("blue route: kind %d r2r %d n %" PRId64 " op %d (m %" PRId64 "): %d (status %d), expected %d", kind, r2r, n, op,
+             m, got, (int)st, want);
+    for (void *q : {src, dst, ws}) (void)hipFree(q);
+    pfh_plan_destroy(p);
+}
+
+void blue_routes()
+{
+    const int before = g_fail;
+    pfh::g_math_dft = false; // pieces of long lines (g_math): bounds and shapes only
+    for (int64_t m : {22, 26, 88, 121, 17, 34, 209, 53, 106, 146, 438, 79, 158, 474, 127, 254, 131, 393, 223, 509}) {
+        int64_t pm = 1, r = m;
+        for (int64_t q = 2; q <= r; ++q)
+            while (r % q == 0) {
+                pm = q;
+                r /= q;
+            }
+        const int want = pm < 79 ? 0 : 1;
+        for (int op : {PFH_FORWARD, PFH_INVERSE}) {
+            blue_route<float>(PFH_LOCAL_C2C, 0, m, op, m, want);
+            blue_route<double>(PFH_LOCAL_C2C, 0, m, op, m, want);
+        }
+        for (int64_t n : {m, 2 * m}) {
+            const int64_t fm = n % 2 ? n : n / 2; // FFT length of a half-complex line
+            if (fm != m) continue;
+            blue_route<float>(PFH_LOCAL_R2C, 0, n, PFH_FORWARD, m, want);
+            blue_route<double>(PFH_LOCAL_R2C, 0, n, PFH_FORWARD, m, want);
+            blue_route<float>(PFH_LOCAL_R2R, PFH_DCT2, n, PFH_FORWARD, m, want);
+            const bool pieces = pm > 127 && n % 2 == 0;
+            pfh::g_math = pieces;
+            blue_route<float>(PFH_LOCAL_R2C, 0, n, PFH_INVERSE, m, pieces ? 2 : want);
+            blue_route<double>(PFH_LOCAL_R2C, 0, n, PFH_INVERSE, m, pieces ? 2 : want);
+            pfh::g_math = false;
+        }
+        blue_route<float>(PFH_LOCAL_R2R, PFH_DCT1, m + 1, PFH_FORWARD, m, want);
+        blue_route<double>(PFH_LOCAL_R2R, PFH_DST1, m - 1, PFH_FORWARD, m, want);
+    }
+    pfh::g_math_dft = true;
+    std::printf("lines without a plan: %s\n", g_fail == before ? "ok" : "FAILED");
+}
+
 void long_cases()
 {
     const int before = g_fail;
@@ -2253,6 +2326,11 @@ int main(int argc, char **argv)
 {
     if (argc == 2 && std::strcmp(argv[1], "long") == 0) {
         long_cases();
+        std::printf("launches %d, failures %d\n", pfh::g_launches, g_fail);
+        return g_fail ? 1 : 0;
+    }
+    if (argc == 2 && std::strcmp(argv[1], "blue") == 0) {
+        blue_routes();
         std::printf("launches %d, failures %d\n", pfh::g_launches, g_fail);
         return g_fail ? 1 : 0;
     }

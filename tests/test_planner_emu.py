@@ -82,3 +82,12 @@ def test_folded_steps_equal_two_calls(emu):
     assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-2000:]
     lines = [l for l in r.stdout.splitlines() if l.endswith(": ok") or l.endswith(": FAILED")]
     assert len(lines) > 20 and all(l.endswith(": ok") for l in lines)
+
+
+def test_lines_without_a_plan_keep_their_accuracy(emu):
+    """The in-workgroup Bluestein is taken only where its error is no larger
+    than that of the kernel it replaces: prime factors from 79 on, above 127
+    not for C2R lines of even length."""
+    r = subprocess.run([emu, "blue"], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-2000:]
+    assert "lines without a plan: ok" in r.stdout
