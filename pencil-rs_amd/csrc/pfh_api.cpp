@@ -1269,7 +1269,9 @@ static pfh_status twiddle_table(PlanImpl &P, int64_t M, int64_t &off, int &bsh)
 
 // Splits up to this length keep all their twiddles in one table (8 MiB f32 at
 // 2^20), read along neighbouring lines: one rounding and one load per value;
-// longer ones multiply three table entries.
+// longer ones multiply two table entries (a third, shared by the values of a
+// butterfly, saves loads and costs a rounding: relative L2 error of 2^21 points
+// f32 1.73e-7 against 1.71e-7).
 constexpr int64_t kFullTwiddles = 1 << 20;
 
 // exp(-2 pi i d k / (n1 n2)) at [k][d], k < n1, d < n2.
@@ -1322,19 +1324,9 @@ static pfh_status make_piece(PlanImpl &P, Step &p, int64_t N, std::vector<PieceD
     pfh_status st = plan_table(P, "pass:" + std::to_string(N) + ":" + (p.line_plan ? "line" : std::to_string(max_r)),
                                base, [&](std::vector<double> &t) { pass_tables(p.radices, &t, twoff, p.line_plan); });
     if (st) return st;
-    if (p.line_plan && (x.flags & F_XTW)) {
-        const int RL = p.radices.back();
-        const int64_t n2 = x.tw_m / N;
-        p.xtw_full = x.tw_m <= kFullTwiddles;
-        if (p.xtw_full)
-            st = full_twiddles(P, N, n2, p.xtwr);
-        else
-            st = plan_table(P, "twr:" + std::to_string(RL) + ":" + std::to_string(n2), p.xtwr,
-                            [&](std::vector<double> &t) {
-                                for (int r = 0; r < RL; ++r)
-                                    for (int64_t d = 0; d < n2; ++d)
-                                        push_cexp(t, (long long)r * d, (long long)RL * n2);
-                            });
+    p.xtw_full = p.line_plan && (x.flags & F_XTW) && x.tw_m <= kFullTwiddles;
+    if (p.xtw_full) {
+        st = full_twiddles(P, N, x.tw_m / N, p.xtwr);
         if (st) return st;
     }
     p.tw_base = base;

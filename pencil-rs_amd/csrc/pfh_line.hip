@@ -347,12 +347,12 @@ __global__ __launch_bounds__(kLinePlanThreads) void k_line_plan(const StageArgs<
                         for (int r = 0; r < RL; ++r)
                             v[b][r] = cmul(v[b][r], gread<cpx<T>>(a.xtwr, w0 + (uint32_t)(r * NB) * n2 * (uint32_t)(2 * sizeof(T))));
                     } else {
-                        const uint32_t q = odco * (uint32_t)j;
-                        const cpx<T> w = cmul(get<T>(reinterpret_cast<const V *>(a.xtw) + (q & lo)), get<T>(hi + (q >> a.xtw_bsh)));
-                        v[b][0] = cmul(v[b][0], w);
+                        const V *two = reinterpret_cast<const V *>(a.xtw);
 #pragma unroll
-                        for (int r = 1; r < RL; ++r)
-                            v[b][r] = cmul(v[b][r], cmul(w, gread<cpx<T>>(a.xtwr, ((uint32_t)r * n2 + odco) * (uint32_t)(2 * sizeof(T)))));
+                        for (int r = 0; r < RL; ++r) {
+                            const uint32_t q = odco * (uint32_t)(j + r * NB);
+                            v[b][r] = cmul(v[b][r], cmul(get<T>(two + (q & lo)), get<T>(hi + (q >> a.xtw_bsh))));
+                        }
                     }
                 }
             }

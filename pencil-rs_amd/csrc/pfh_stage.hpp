@@ -169,8 +169,8 @@ struct StageArgs {
     int xmul_in, xmul_out;
     int xvalid_in, xvalid_out;
     int xtw_m, xtw_bsh;
-    // k_line_plan: the split's twiddles at [k][d], exp(-2 pi i d k / xtw_m), d < n2 = xtw_m / m (xtw_full), or
-    // at [r][d], exp(-2 pi i d r / (RL n2)), r < RL (the last radix), a factor of the two-level table's
+    // k_line_plan: the split's twiddles in one table, exp(-2 pi i d k / xtw_m) at [k][d], d < n2 = xtw_m / m
+    // (xtw_full; a longer split takes the two-level table)
     const cpx<T> *xtwr;
     int xtw_full;
     // Pointwise steps in the last stage's store (k_line_plan KIND 5 and 6).

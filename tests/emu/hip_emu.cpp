@@ -407,10 +407,20 @@ static void emulate_math(const char *what, const StageArgs<T> &a)
             if (a.flags & F_XTW) {
                 const int64_t q = (int64_t)dco * k;
                 if (q >= a.xtw_m) fail("%s: twiddle index %" PRId64 " >= %d", what, q, a.xtw_m);
-                const int64_t lo = q & ((1 << a.xtw_bsh) - 1), hi = (1 << a.xtw_bsh) + (q >> a.xtw_bsh);
-                if (!check_read("xtw", a.xtw + lo, sizeof(cpx<T>)) || !check_read("xtw", a.xtw + hi, sizeof(cpx<T>)))
-                    return;
-                w = cmul_l(w, cmul_l({(ld)a.xtw[lo].x, (ld)a.xtw[lo].y}, {(ld)a.xtw[hi].x, (ld)a.xtw[hi].y}));
+                if (a.xtw_full) {
+                    // one table at [k][d]
+                    const int64_t n2 = a.xtw_m / m;
+                    const cpx<T> *t = a.xtwr + (int64_t)k * n2 + dco;
+                    if (!(a.flags & F_LINE_PLAN) || dco >= n2) fail("%s: full twiddle table, digit %d", what, dco);
+                    if (!check_read("xtwr", t, sizeof(cpx<T>))) return;
+                    w = cmul_l(w, {(ld)t->x, (ld)t->y});
+                } else {
+                    if (a.xtwr) fail("%s: a third twiddle factor", what);
+                    const int64_t lo = q & ((1 << a.xtw_bsh) - 1), hi = (1 << a.xtw_bsh) + (q >> a.xtw_bsh);
+                    if (!check_read("xtw", a.xtw + lo, sizeof(cpx<T>)) || !check_read("xtw", a.xtw + hi, sizeof(cpx<T>)))
+                        return;
+                    w = cmul_l(w, cmul_l({(ld)a.xtw[lo].x, (ld)a.xtw[lo].y}, {(ld)a.xtw[hi].x, (ld)a.xtw[hi].y}));
+                }
             }
             if (a.flags & F_CONJ_OUT) w.im = -w.im;
             w = {w.re * (ld)a.scale, w.im * (ld)a.scale};
@@ -2215,6 +2225,9 @@ void long_cases()
         local_long_case<double>(PFH_LOCAL_C2C, 0, n, PFH_FORWARD, 2, 0);
         local_long_case<float>(PFH_LOCAL_R2R, PFH_DCT2, 2 * n, PFH_FORWARD, 2, 0);
     }
+    // a split above 2^20 points and a convolution above it
+    local_long_case<float>(PFH_LOCAL_C2C, 0, 1 << 21, PFH_FORWARD, 1, 0);
+    local_long_case<float>(PFH_LOCAL_C2C, 0, 700001, PFH_INVERSE, 1, 0);
     for (int64_t n : {10006, 65535}) local_long_case<double>(PFH_LOCAL_R2R, PFH_DST1, n, PFH_FORWARD, 2, 0);
     for (int op : {PFH_FORWARD, PFH_INVERSE}) {
         route_long_case<float>({10007, 3, 4}, 2, op, 0);
