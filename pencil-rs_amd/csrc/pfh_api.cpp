@@ -692,12 +692,19 @@ static int g_column_lines = []() {
 // without permutation (808-byte rows) 292 us with single tiles, 274 / 262 / 254
 // / 249 us with runs of 2 / 4 / 8 / 16, 257 / 280 us with 64 / 128; 512^3 R2C +
 // C2R f32 1190 -> 1169 us, f64 2279 -> 2160 us (one contiguous eighth per XCD:
-// 1308 / 2320 us). PFH_XCD overrides the run length, 0 turns it off.
+// 1308 / 2320 us). PFH_XCD overrides the run length, 0 turns it off. Copy stages
+// whose points and nearest lines are both powers of two keep single tiles: no
+// cache line is shared unevenly there, and runs took longer (16-byte elements,
+// 1024 x 32 x 256 -> 1024 x 256 x 32 36 -> 45 us, 16384 x 128 x 4 38 -> 46 us; but 928 x
+// 70 x 129 60 -> 43 us).
 static void set_tiles(Step &st, const Tuning &tu)
 {
     st.tiles = (st.nlines + st.lt - 1) / st.lt;
     static const int xcd_env = env_int("PFH_XCD", 16);
     int64_t run = std::min<int64_t>(xcd_env, st.tiles / 64);
+    if ((st.mode == M_COPY_C || st.mode == M_COPY_R) && (st.nin & (st.nin - 1)) == 0 &&
+        (st.g.nd == 0 || (st.g.ext[0] & (st.g.ext[0] - 1)) == 0))
+        run = 0;
     int64_t p = 1;
     while (2 * p <= run) p *= 2;
     st.xcd_per = 0;

@@ -10,11 +10,13 @@
 //    elements: 32), 16 (4) loads in flight a thread;
 //  - they are the same: rows, moved in 16-byte pieces where lengths, strides
 //    and addresses allow.
-// Both are bound by HBM. 256 x 384 x 240 complex f32, z,y,x -> x,z,y (189 MB
+// Each is taken where it beats the callers' own kernels (pfh_copy.hpp); both are
+// bound by HBM. 256 x 384 x 240 complex f32, z,y,x -> x,z,y (189 MB
 // each way) on MI355X: 74 us; the line kernel's copy stage, which held whole
 // lines on one wave per workgroup in LDS, took 154 us.
 #include <hip/hip_runtime.h>
 
+#include "pfh_copy.hpp"
 #include "pfh_kernels.hpp"
 
 namespace pfh {
@@ -93,8 +95,8 @@ __global__ __launch_bounds__(256) void k_copy_tile(const CopyArgs a)
 }
 
 // rows (ss_p == ds_p == 1): cols threads along a row, 256 / cols rows at a
-// time, kRows such groups per workgroup; grid.y = pieces of 256 points
-constexpr int kRows = 8;
+// time, kCopyRows such groups per workgroup; grid.y = pieces of 256 points
+constexpr int kRows = kCopyRows;
 template <typename W>
 __global__ __launch_bounds__(256) void k_copy_rows(const CopyArgs a, uint32_t rows, int cols, int csh)
 {
@@ -120,12 +122,13 @@ __global__ __launch_bounds__(256) void k_copy_rows(const CopyArgs a, uint32_t ro
     }
 }
 
-template <typename W, int TILE>
+template <typename W>
 hipError_t run_tile(CopyArgs &a, int64_t rest, hipStream_t s, bool &done)
 {
+    constexpr int TILE = copy_tile((int)sizeof(W));
     a.tiles_p = (a.n + TILE - 1) / TILE;
     a.tiles_l = (a.e0 + TILE - 1) / TILE;
-    const int64_t grid = a.tiles_p * a.tiles_l * rest;
+    const int64_t grid = copy_tile_blocks((int)sizeof(W), a.n, a.e0, rest);
     if (grid > INT32_MAX) return hipSuccess;
     done = true;
     hipLaunchKernelGGL((k_copy_tile<W, TILE>), dim3((unsigned)grid), dim3(256), 0, s, a);
@@ -135,15 +138,12 @@ hipError_t run_tile(CopyArgs &a, int64_t rest, hipStream_t s, bool &done)
 template <typename W>
 hipError_t run_rows(const CopyArgs &a, int64_t rows, hipStream_t s)
 {
-    int cols = 1, csh = 0;
-    while (cols < 256 && cols < a.n) {
-        cols *= 2;
-        ++csh;
-    }
-    const int64_t per = (256 >> csh) * kRows;
+    const int cols = copy_row_cols(a.n);
+    int csh = 0;
+    while ((1 << csh) < cols) ++csh;
     int64_t gy = (a.n + cols - 1) / cols;
     if (gy > 64) gy = 64;
-    hipLaunchKernelGGL(k_copy_rows<W>, dim3((unsigned)((rows + per - 1) / per), (unsigned)gy), dim3(256), 0, s, a,
+    hipLaunchKernelGGL(k_copy_rows<W>, dim3((unsigned)copy_row_blocks(rows, a.n), (unsigned)gy), dim3(256), 0, s, a,
                        (uint32_t)rows, cols, csh);
     return hipGetLastError();
 }
@@ -151,7 +151,7 @@ hipError_t run_rows(const CopyArgs &a, int64_t rows, hipStream_t s)
 } // namespace
 
 // Copies the axes of c; done stays false (nothing launched) where neither
-// shape applies. Axes of extent 1 may be listed. src and dst do not overlap
+// shape applies or pays (pfh_copy.hpp). Axes of extent 1 may be listed. src and dst do not overlap
 // unless they are the same array in the same layout.
 hipError_t launch_copy_axes(const CopyAxes &c, const void *src, void *dst, int word, const int *gate, hipStream_t s,
                             bool &done)
@@ -202,18 +202,20 @@ hipError_t launch_copy_axes(const CopyAxes &c, const void *src, void *dst, int w
         a.e0 = c.ext[il];
         a.ss_l = 1;
         a.ds_l = c.os[il];
+        if (!copy_tile_pays(word, a.n, a.e0)) return hipSuccess;
         switch (word) {
-        case 1: return run_tile<uint8_t, 64>(a, rest, s, done);
-        case 2: return run_tile<uint16_t, 64>(a, rest, s, done);
-        case 4: return run_tile<uint32_t, 64>(a, rest, s, done);
-        case 8: return run_tile<uint64_t, 64>(a, rest, s, done);
-        case 16: return run_tile<W16, 32>(a, rest, s, done);
+        case 1: return run_tile<uint8_t>(a, rest, s, done);
+        case 2: return run_tile<uint16_t>(a, rest, s, done);
+        case 4: return run_tile<uint32_t>(a, rest, s, done);
+        case 8: return run_tile<uint64_t>(a, rest, s, done);
+        case 16: return run_tile<W16>(a, rest, s, done);
         default: return hipSuccess;
         }
     }
     // rows: the widest word that lengths, strides and addresses are multiples of
     a.ss_l = a.ds_l = 0;
     a.e0 = 1;
+    const int word0 = word;
     while (word < 16) {
         bool even = a.n % 2 == 0 && reinterpret_cast<uintptr_t>(src) % (2 * (size_t)word) == 0 &&
                     reinterpret_cast<uintptr_t>(dst) % (2 * (size_t)word) == 0;
@@ -226,6 +228,7 @@ hipError_t launch_copy_axes(const CopyAxes &c, const void *src, void *dst, int w
             a.os[i] /= 2;
         }
     }
+    if (!copy_rows_pay(word0, c.ext[ip], a.n)) return hipSuccess;
     done = true;
     switch (word) {
     case 1: return run_rows<uint8_t>(a, rest, s);

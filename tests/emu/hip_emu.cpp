@@ -28,6 +28,7 @@
 
 #include "../../include/pencil_fft_hip.h"
 #include "../../pencil-rs_amd/csrc/pfh_collectives.hpp"
+#include "../../pencil-rs_amd/csrc/pfh_copy.hpp"
 #include "../../pencil-rs_amd/csrc/pfh_kernels.hpp"
 
 namespace {
@@ -2111,6 +2112,31 @@ void fold_cases()
             }
 }
 
+// The rules that pick a copy's kernel, at measured shapes on both sides.
+void copy_rules()
+{
+    const int before = g_fail;
+    struct R {
+        int word;
+        int64_t p, l;
+        bool want;
+    };
+    for (const R &r : std::vector<R>{{4, 2, 2, false},    {1, 64, 12, false},  {2, 64, 16, true},  {4, 3, 1000, false},
+                                     {4, 64, 64, true},   {8, 16, 64, false},  {8, 32, 48, true},  {8, 256, 16, true},
+                                     {8, 384, 256, true}, {16, 64, 64, false}, {16, 256, 256, false},
+                                     {16, 1000, 64, true}, {16, 4, 64, true},  {16, 8, 64, false}})
+        if (pfh::copy_tile_pays(r.word, r.p, r.l) != r.want)
+            fail("tile rule: %d bytes %" PRId64 " x %" PRId64, r.word, r.p, r.l);
+    // (word, n, nw)
+    for (const R &r : std::vector<R>{{1, 3, 3, false},   {1, 4, 1, true},    {1, 33, 33, false}, {2, 7, 7, true},
+                                     {4, 3, 3, false},   {4, 12, 3, false},  {4, 16, 4, true},   {4, 17, 17, false},
+                                     {8, 12, 6, false},  {8, 24, 12, false}, {8, 32, 16, true},  {8, 65, 65, true},
+                                     {16, 64, 64, false}, {16, 129, 129, false}, {16, 100, 100, true}})
+        if (pfh::copy_rows_pay(r.word, r.p, r.l) != r.want)
+            fail("row rule: %d bytes %" PRId64 " / %" PRId64, r.word, r.p, r.l);
+    std::printf("copy rules: %s\n", g_fail == before ? "ok" : "FAILED");
+}
+
 // Which kernel a line without a plan takes: the generic one for prime factors
 // up to 73, k_line_blue from 79 on, the pieces of a long line for C2R lines of
 // even length with a factor above 127. Identity arithmetic.
@@ -2344,6 +2370,11 @@ int main(int argc, char **argv)
     }
     if (argc == 2 && std::strcmp(argv[1], "blue") == 0) {
         blue_routes();
+        std::printf("launches %d, failures %d\n", pfh::g_launches, g_fail);
+        return g_fail ? 1 : 0;
+    }
+    if (argc == 2 && std::strcmp(argv[1], "copies") == 0) {
+        copy_rules();
         std::printf("launches %d, failures %d\n", pfh::g_launches, g_fail);
         return g_fail ? 1 : 0;
     }

@@ -91,3 +91,10 @@ def test_lines_without_a_plan_keep_their_accuracy(emu):
     r = subprocess.run([emu, "blue"], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-2000:]
     assert "lines without a plan: ok" in r.stdout
+
+
+def test_copy_rules(emu):
+    """Short axes and narrow rows are left to the callers' kernels."""
+    r = subprocess.run([emu, "copies"], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-2000:]
+    assert "copy rules: ok" in r.stdout
