@@ -16,6 +16,7 @@
 // lines on one wave per workgroup in LDS, took 154 us.
 #include <hip/hip_runtime.h>
 
+#include "pfh_bounds.hpp"
 #include "pfh_copy.hpp"
 #include "pfh_kernels.hpp"
 
@@ -129,7 +130,7 @@ hipError_t run_tile(CopyArgs &a, int64_t rest, hipStream_t s, bool &done)
     a.tiles_p = (a.n + TILE - 1) / TILE;
     a.tiles_l = (a.e0 + TILE - 1) / TILE;
     const int64_t grid = copy_tile_blocks((int)sizeof(W), a.n, a.e0, rest);
-    if (grid > INT32_MAX) return hipSuccess;
+    if (grid >= kMaxBlocks256) return hipSuccess; // left to the caller's kernel
     done = true;
     hipLaunchKernelGGL((k_copy_tile<W, TILE>), dim3((unsigned)grid), dim3(256), 0, s, a);
     return hipGetLastError();
@@ -228,7 +229,7 @@ hipError_t launch_copy_axes(const CopyAxes &c, const void *src, void *dst, int w
             a.os[i] /= 2;
         }
     }
-    if (!copy_rows_pay(word0, c.ext[ip], a.n)) return hipSuccess;
+    if (!copy_rows_pay(word0, c.ext[ip], a.n) || copy_row_blocks(rest, a.n) >= kMaxBlocks256) return hipSuccess;
     done = true;
     switch (word) {
     case 1: return run_rows<uint8_t>(a, rest, s);

@@ -6,6 +6,7 @@
 // memory-bound element kernels.
 #include <hip/hip_runtime.h>
 
+#include "pfh_bounds.hpp"
 #include "pfh_kernels.hpp"
 
 namespace pfh {
@@ -22,7 +23,7 @@ constexpr int kBlock = 256;
 // keep the row's index arithmetic off the elements and their loads in flight.
 // 256^3 f32 half spectrum (67 MB) on MI355X: 41 us with one element and its
 // 64-bit divisions a thread, 30 us so.
-constexpr int kRows = 4;
+constexpr int kRows = kScaleRows;
 template <typename T, int C, bool CF>
 __global__ __launch_bounds__(kBlock) void k_scale_axes(ScaleAxesArgs s, T *data, const T *f, uint32_t rows, int cols,
                                                        int csh)
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(kBlock) void k_scale_axes(ScaleAxesArgs s, T *data,
 // Elementwise kernels: kUnroll elements a thread, all loads issued first.
 // 256^3 f32 on MI355X, one element a thread before: quadratic step (134 MB) 32
 // -> 22 us, its adjoint (201 MB) 52 -> 36 us.
-constexpr int kUnroll = 8;
+constexpr int kUnroll = kElementsPerBlock / kBlock;
 unsigned chunks_for(int64_t n)
 {
     return (unsigned)((n + (int64_t)kBlock * kUnroll - 1) / ((int64_t)kBlock * kUnroll));
@@ -162,59 +163,34 @@ __global__ __launch_bounds__(kBlock) void k_sumsq_final(const double *partial, i
 template <typename T>
 hipError_t launch_scale_axes(const ScaleAxesArgs &s0, void *data, const void *factors, hipStream_t st)
 {
-    const int64_t total = s0.len * s0.extra;
-    if (total <= 0) return hipSuccess;
-    ScaleAxesArgs s = s0;
-    const int64_t nx = s.mext[s.nd - 1];
-    const int64_t rows64 = total / nx;
-    if (rows64 > INT32_MAX) {
-        // the kernel divides row indexes in 32 bits: halves of the extras,
-        // then of the slowest axis
-        const int64_t eb = (s.complex_data ? 2 : 1) * (int64_t)sizeof(T);
-        ScaleAxesArgs lo = s0, hi = s0;
-        int64_t skip;
-        if (s0.extra > 1) {
-            lo.extra = s0.extra / 2;
-            hi.extra = s0.extra - lo.extra;
-            skip = lo.extra * s0.len;
-        } else if (s0.nd > 1 && s0.mext[0] > 1) {
-            lo.mext[0] = s0.mext[0] / 2;
-            hi.mext[0] = s0.mext[0] - lo.mext[0];
-            hi.foff[0] += lo.mext[0];
-            lo.len = s0.len / s0.mext[0] * lo.mext[0];
-            hi.len = s0.len - lo.len;
-            skip = lo.len;
-        } else {
-            return hipErrorInvalidValue;
+    if (s0.len * s0.extra <= 0) return hipSuccess;
+    hipError_t err = hipSuccess;
+    scale_axes_parts(s0, 0, [&](const ScaleAxesArgs &part, int64_t first) {
+        if (err != hipSuccess) return;
+        ScaleAxesArgs s = part;
+        const int64_t nx = s.mext[s.nd - 1], rows = s.len * s.extra / nx;
+        for (int p = 0; p + 1 < s.nd; ++p) {
+            const FastDiv d = make_fastdiv((uint32_t)s.mext[p]);
+            s.dmag[p] = d.mag;
+            s.dsh[p] = d.sh;
         }
-        const hipError_t e = launch_scale_axes<T>(lo, data, factors, st);
-        if (e != hipSuccess) return e;
-        return launch_scale_axes<T>(hi, static_cast<char *>(data) + skip * eb, factors, st);
-    }
-    for (int p = 0; p + 1 < s.nd; ++p) {
-        const FastDiv d = make_fastdiv((uint32_t)s.mext[p]);
-        s.dmag[p] = d.mag;
-        s.dsh[p] = d.sh;
-    }
-    int cols = 1, csh = 0;
-    while (cols < kBlock && cols < nx) {
-        cols *= 2;
-        ++csh;
-    }
-    const int64_t per = (int64_t)(kBlock >> csh) * kRows;
-    int64_t gy = (nx + cols - 1) / cols;
-    if (gy > 64) gy = 64;
-    const dim3 grid((unsigned)((rows64 + per - 1) / per), (unsigned)gy);
-    T *d = static_cast<T *>(data);
-    const T *f = static_cast<const T *>(factors);
-    const uint32_t rows = (uint32_t)rows64;
-    if (s.complex_factors)
-        hipLaunchKernelGGL((k_scale_axes<T, 2, true>), grid, dim3(kBlock), 0, st, s, d, f, rows, cols, csh);
-    else if (s.complex_data)
-        hipLaunchKernelGGL((k_scale_axes<T, 2, false>), grid, dim3(kBlock), 0, st, s, d, f, rows, cols, csh);
-    else
-        hipLaunchKernelGGL((k_scale_axes<T, 1, false>), grid, dim3(kBlock), 0, st, s, d, f, rows, cols, csh);
-    return hipGetLastError();
+        const int cols = scale_axes_cols(nx);
+        int csh = 0;
+        while ((1 << csh) < cols) ++csh;
+        int64_t gy = (nx + cols - 1) / cols;
+        if (gy > 64) gy = 64;
+        const dim3 grid((unsigned)scale_axes_blocks(rows, nx), (unsigned)gy);
+        T *d = static_cast<T *>(data) + first * (s.complex_data ? 2 : 1);
+        const T *f = static_cast<const T *>(factors);
+        if (s.complex_factors)
+            hipLaunchKernelGGL((k_scale_axes<T, 2, true>), grid, dim3(kBlock), 0, st, s, d, f, (uint32_t)rows, cols, csh);
+        else if (s.complex_data)
+            hipLaunchKernelGGL((k_scale_axes<T, 2, false>), grid, dim3(kBlock), 0, st, s, d, f, (uint32_t)rows, cols, csh);
+        else
+            hipLaunchKernelGGL((k_scale_axes<T, 1, false>), grid, dim3(kBlock), 0, st, s, d, f, (uint32_t)rows, cols, csh);
+        err = hipGetLastError();
+    });
+    return err;
 }
 template hipError_t launch_scale_axes<float>(const ScaleAxesArgs &, void *, const void *, hipStream_t);
 template hipError_t launch_scale_axes<double>(const ScaleAxesArgs &, void *, const void *, hipStream_t);
@@ -222,10 +198,14 @@ template hipError_t launch_scale_axes<double>(const ScaleAxesArgs &, void *, con
 template <typename T>
 hipError_t launch_quadratic(const void *w, void *u, int64_t n, double a, hipStream_t st)
 {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_quadratic<T>, dim3(chunks_for(n)), dim3(kBlock), 0, st, static_cast<const T *>(w),
-                       static_cast<T *>(u), n, (T)a);
-    return hipGetLastError();
+    for (int64_t i = 0; i < n; i += kElementsPerLaunch) {
+        const int64_t m = n - i < kElementsPerLaunch ? n - i : kElementsPerLaunch;
+        hipLaunchKernelGGL(k_quadratic<T>, dim3(chunks_for(m)), dim3(kBlock), 0, st, static_cast<const T *>(w) + i,
+                           static_cast<T *>(u) + i, m, (T)a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 template hipError_t launch_quadratic<float>(const void *, void *, int64_t, double, hipStream_t);
 template hipError_t launch_quadratic<double>(const void *, void *, int64_t, double, hipStream_t);
@@ -233,10 +213,15 @@ template hipError_t launch_quadratic<double>(const void *, void *, int64_t, doub
 template <typename T>
 hipError_t launch_quadratic_adjoint(const void *w, const void *g, void *out, int64_t n, double a, hipStream_t st)
 {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_quadratic_adjoint<T>, dim3(chunks_for(n)), dim3(kBlock), 0, st, static_cast<const T *>(w),
-                       static_cast<const T *>(g), static_cast<T *>(out), n, (T)a);
-    return hipGetLastError();
+    for (int64_t i = 0; i < n; i += kElementsPerLaunch) {
+        const int64_t m = n - i < kElementsPerLaunch ? n - i : kElementsPerLaunch;
+        hipLaunchKernelGGL(k_quadratic_adjoint<T>, dim3(chunks_for(m)), dim3(kBlock), 0, st,
+                           static_cast<const T *>(w) + i, static_cast<const T *>(g) + i, static_cast<T *>(out) + i, m,
+                           (T)a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 template hipError_t launch_quadratic_adjoint<float>(const void *, const void *, void *, int64_t, double, hipStream_t);
 template hipError_t launch_quadratic_adjoint<double>(const void *, const void *, void *, int64_t, double,

@@ -28,6 +28,7 @@
 
 #include "../../include/pencil_fft_hip.h"
 #include "../../pencil-rs_amd/csrc/pfh_collectives.hpp"
+#include "../../pencil-rs_amd/csrc/pfh_bounds.hpp"
 #include "../../pencil-rs_amd/csrc/pfh_copy.hpp"
 #include "../../pencil-rs_amd/csrc/pfh_kernels.hpp"
 
@@ -2137,6 +2138,56 @@ void copy_rules()
     std::printf("copy rules: %s\n", g_fail == before ? "ok" : "FAILED");
 }
 
+// Launches of arrays beyond 2^24 workgroups: copies are refused by their rules
+// or by the count, scaling and elementwise steps run in parts that cover every
+// element once with the factors of their own coordinates.
+void launch_bounds()
+{
+    const int before = g_fail;
+    using namespace pfh;
+    // 20 million planes of 2 x 2: too many workgroups, and refused for its tiles
+    if (copy_tile_blocks(4, 2, 2, 20000000) < kMaxBlocks256 || copy_tile_pays(4, 2, 2)) fail("copy of 2 x 2 planes");
+    if (copy_tile_blocks(1, 64, 64, 1 << 24) < kMaxBlocks256) fail("copy of 2^24 tiles");
+    if (copy_row_blocks((int64_t)1 << 27, 255) < kMaxBlocks256) fail("copy of 2^27 odd rows");
+    struct S {
+        std::vector<int64_t> ext; // slowest first
+        int64_t extra;
+    };
+    for (const S &c : std::vector<S>{{{70000000, 3, 200}, 1}, {{1, 80000000, 300}, 1}, {{20000, 5000, 129}, 7},
+                                     {{1 << 16, 1 << 16, 2}, 3}, {{4, 5, 6}, 2}, {{1000}, 1}}) {
+        ScaleAxesArgs s{};
+        s.nd = (int)c.ext.size();
+        s.extra = c.extra;
+        s.len = 1;
+        for (int p = 0; p < s.nd; ++p) {
+            s.mext[p] = c.ext[p];
+            s.len *= c.ext[p];
+        }
+        int64_t at = 0, parts = 0;
+        scale_axes_parts(s, 0, [&](const ScaleAxesArgs &q, int64_t first) {
+            ++parts;
+            const int64_t nx = q.mext[q.nd - 1], rows = q.len * q.extra / nx;
+            int64_t len = 1;
+            for (int p = 0; p < q.nd; ++p) len *= q.mext[p];
+            if (first != at) fail("scale part at %" PRId64 ", expected %" PRId64, first, at);
+            if (len != q.len || q.mext[q.nd - 1] != s.mext[s.nd - 1]) fail("scale part extents");
+            if (rows > INT32_MAX || scale_axes_blocks(rows, nx) >= kMaxBlocks256) fail("scale part of %" PRId64 " rows", rows);
+            // the part's first coordinates
+            int64_t rem = first % s.len;
+            for (int p = s.nd - 1; p >= 0; --p) {
+                if (q.mext[p] != s.mext[p] && q.foff[p] != rem % s.mext[p]) fail("scale part's factors on axis %d", p);
+                if (q.mext[p] == s.mext[p] && q.foff[p] != 0) fail("scale part's factors on whole axis %d", p);
+                rem /= s.mext[p];
+            }
+            at += q.len * q.extra;
+        });
+        if (at != s.len * s.extra) fail("scale parts cover %" PRId64 " of %" PRId64, at, s.len * s.extra);
+        if (s.len * s.extra / s.mext[s.nd - 1] <= 1000 && parts != 1) fail("scale parts of a small array");
+    }
+    if ((kElementsPerLaunch + kElementsPerBlock - 1) / kElementsPerBlock >= kMaxBlocks256) fail("elementwise launch");
+    std::printf("launch bounds: %s\n", g_fail == before ? "ok" : "FAILED");
+}
+
 // Which kernel a line without a plan takes: the generic one for prime factors
 // up to 73, k_line_blue from 79 on, the pieces of a long line for C2R lines of
 // even length with a factor above 127. Identity arithmetic.
@@ -2375,6 +2426,7 @@ int main(int argc, char **argv)
     }
     if (argc == 2 && std::strcmp(argv[1], "copies") == 0) {
         copy_rules();
+        launch_bounds();
         std::printf("launches %d, failures %d\n", pfh::g_launches, g_fail);
         return g_fail ? 1 : 0;
     }
