@@ -715,6 +715,14 @@ static void set_tiles(Step &st, const Tuning &tu)
     }
 }
 
+// Lines of a step that one launch holds (HIP refuses 2^32 threads and more);
+// the grid may be rounded up by a round of tile runs.
+static int64_t lines_per_launch(const Step &st, const Tuning &tu)
+{
+    const int64_t tiles = tu.max_launch_threads / std::max(st.threads, 1) - 8LL * std::max(st.xcd_per, 0);
+    return std::max<int64_t>(tiles, 1) * st.lt;
+}
+
 // Line grid and access patterns of a step whose in/out layouts are set.
 static pfh_status step_geometry(Step &st)
 {
@@ -2394,6 +2402,9 @@ static pfh_status create_impl(const pfh_desc *d, PlanImpl &P)
     if (P.precision != PFH_F32 && P.precision != PFH_F64) return set_err(PFH_ERR_INVALID_ARGUMENT, "precision");
     pfh_status st = device_info(P.dev);
     if (st) return st;
+    // (PFH_LAUNCH_THREADS: a smaller bound, so that tests reach the parts)
+    if (const char *e = std::getenv("PFH_LAUNCH_THREADS"))
+        if (std::atoll(e) > 0) P.tuning.max_launch_threads = std::min<int64_t>(std::atoll(e), kMaxLaunchThreads);
     P.extra = 1;
     if (d->extra_ndim < 0 || d->extra_ndim > PFH_MAX_DIMS) return set_err(PFH_ERR_INVALID_ARGUMENT, "extra_ndim");
     for (int i = 0; i < d->extra_ndim; ++i) P.extra *= (int64_t)d->extra_shape[i];
@@ -3580,9 +3591,32 @@ static pfh_status local_execute_impl(pfh_plan plan, int op, const void *src, siz
     s.in.extra = s.out.extra = batch;
     pfh_status st = finish_step(s, P.dev, tb, P.tuning);
     if (st) return st;
-    void *bufs[4] = {const_cast<void *>(src), dst, nullptr, nullptr};
-    st = run_op(P, o, bufs, wv, stream, nullptr);
-    if (st) return st;
+    // more threads than one launch may have (line plans take several a line:
+    // 2^31 lines of 8 points): parts of the batch, after the boundary check of
+    // all of it
+    const int64_t part = lines_per_launch(s, P.tuning);
+    if (part < batch) {
+        if (c2r_check) {
+            PFH_HIP_CHECK(P.precision == PFH_F32
+                              ? launch_local_endpoint_check<float>(src, batch, s.nin, (s.n % 2 == 0) ? 1 : 0,
+                                                                   wv.first_code, wv.gate, wv.status, stream)
+                              : launch_local_endpoint_check<double>(src, batch, s.nin, (s.n % 2 == 0) ? 1 : 0,
+                                                                    wv.first_code, wv.gate, wv.status, stream));
+            s.local_endpoint_check = false;
+            s.gated = true;
+        }
+    }
+    for (int64_t l0 = 0; l0 < batch; l0 += part) {
+        if (part < batch) {
+            s.in.extra = s.out.extra = std::min(part, batch - l0);
+            st = finish_step(s, P.dev, tb, P.tuning);
+            if (st) return st;
+        }
+        void *bufs[4] = {const_cast<char *>(static_cast<const char *>(src)) + l0 * lin * tmpl.in.elem,
+                         static_cast<char *>(dst) + l0 * lout * tmpl.out.elem, nullptr, nullptr};
+        st = run_op(P, o, bufs, wv, stream, nullptr);
+        if (st) return st;
+    }
     if (c2r_check && !(flags & PFH_EXEC_DEFER_STATUS)) return collect_status(P, wv, stream);
     return ok();
 }
