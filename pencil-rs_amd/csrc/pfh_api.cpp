@@ -340,13 +340,9 @@ static int env_int(const char *name, int dflt)
 }
 
 // The line plan (k_line_plan) of an FFT length; radices 0 if there is none.
-// dct4: an even DCT-IV or DST-IV line. It loads and stores as a C2C line does, with
-// one twiddle a value, and where 12 divides the length it does no better with twice
-// the threads (MI355X, n^3 f32 DCT-IV, forward + inverse, one and two times the
-// threads: FFT of 72 154 / 158 us, 84 97 / 97, 96 123 / 127, 120 177 / 184 us; but 75
-// 180 / 177, 105 159 / 140, 112 176 / 161, 128 221 / 185; f64 72 279 / 282, 84 132 / 131,
-// 120 349 / 352, the others equal). 256 x 384 x 240 f32 R2R 326 -> 319 us.
-static void find_line_plan(int m, int tbytes, int r[3], int &em, bool real_modes = false, bool dct4 = false)
+// real_modes: the plan with twice the threads a line where the length has one
+// (line_plan_real_only).
+static void find_line_plan(int m, int tbytes, int r[3], int &em, bool real_modes = false)
 {
     using Entry = std::array<int, 4>;
     using Table = std::map<int, Entry>;
@@ -361,11 +357,10 @@ static void find_line_plan(int m, int tbytes, int r[3], int &em, bool real_modes
     }();
     r[0] = 0;
     const std::array<Table, 2> &own = plans[tbytes == 4 ? 0 : 1];
-    const auto every = own[0].find(m), own_real = own[1].find(m);
-    const bool has = every != own[0].end();
-    const bool real = real_modes && own_real != own[1].end() && !(dct4 && has && m % 12 == 0);
-    if (!has && !real) return;
-    const Entry &e = real ? own_real->second : every->second;
+    const Table &t = real_modes && own[1].count(m) ? own[1] : own[0];
+    const auto it = t.find(m);
+    if (it == t.end()) return;
+    const Entry &e = it->second;
     for (int i = 0; i < 3; ++i) r[i] = e[i];
     em = e[3];
 }
@@ -415,7 +410,7 @@ static bool choose_line_plan(Step &st, int tbytes, bool in_stage)
     int r[3], em = 0;
     // (f64 half-complex stages take the variants too: 256 x 384 x 240 f64 DHT
     // forward + inverse 444 -> 415 us on MI355X; f32 ones gain nothing)
-    find_line_plan(st.m, tbytes, r, em, r2r || (tbytes == 8 && st.mode != M_C2C), st.mode == M_DCT4);
+    find_line_plan(st.m, tbytes, r, em, r2r || (tbytes == 8 && st.mode != M_C2C));
     if (r2r && st.m > kLinePlanRealMax) r[0] = 0;
     st.blue = 0;
     // a length without a plan: Bluestein in the workgroup. (PFH_BLUESTEIN_PRIME,
