@@ -1259,8 +1259,8 @@ struct PieceDigit {
 struct PieceX {
     int flags = 0; // F_CONJ_IN / F_CONJ_OUT / F_XIN / F_XOUT / F_XTW
     double scale = 1.0;
-    int64_t tab_in = -1, tab_out = -1, tw = -1;
-    int mul_in = 1, mul_out = 1, valid_in = 0, valid_out = 0, tw_m = 0, tw_bsh = 0;
+    int64_t tab_in = -1, tab_out = -1;
+    int mul_in = 1, mul_out = 1, valid_in = 0, valid_out = 0, tw_m = 0;
 };
 
 // Two-level table of exp(-2 pi i q / M): 2^bsh low entries, then the
@@ -1335,8 +1335,8 @@ static pfh_status make_piece(PlanImpl &P, Step &p, int64_t N, std::vector<PieceD
                                base, [&](std::vector<double> &t) { pass_tables(p.radices, &t, twoff, p.line_plan); });
     if (st) return st;
     p.xtw_full = p.line_plan && (x.flags & F_XTW) && x.tw_m <= kFullTwiddles;
-    if (p.xtw_full) {
-        st = full_twiddles(P, N, x.tw_m / N, p.xtwr);
+    if (x.flags & F_XTW) {
+        st = p.xtw_full ? full_twiddles(P, N, x.tw_m / N, p.xtwr) : twiddle_table(P, x.tw_m, p.xtw, p.xtw_bsh);
         if (st) return st;
     }
     p.tw_base = base;
@@ -1369,13 +1369,11 @@ static pfh_status make_piece(PlanImpl &P, Step &p, int64_t N, std::vector<PieceD
     p.out_buf = out_buf;
     p.xtab_in = x.tab_in;
     p.xtab_out = x.tab_out;
-    p.xtw = x.tw;
     p.xmul_in = x.mul_in;
     p.xmul_out = x.mul_out;
     p.xvalid_in = x.valid_in;
     p.xvalid_out = x.valid_out;
     p.xtw_m = x.tw_m;
-    p.xtw_bsh = x.tw_bsh;
     Tuning tu = P.tuning;
     tu.allow_fast = false;
     return size_step(p, P.dev, tb, tu);
@@ -1425,11 +1423,9 @@ static pfh_status fft_pieces(PlanImpl &P, const Step &outer, int64_t N, const Li
         x.tab_in = xin.tab_in;
         x.mul_in = (int)N2;
         x.valid_in = xin.valid_in;
-        pfh_status st = twiddle_table(P, N, x.tw, x.tw_bsh);
-        if (st) return st;
         x.tw_m = (int)N;
         Step p;
-        st = make_piece(P, p, N1, digs, N2 * in.point, N2, in.buf, rs_buf, x, tb, big);
+        pfh_status st = make_piece(P, p, N1, digs, N2 * in.point, N2, in.buf, rs_buf, x, tb, big);
         if (st) return st;
         pieces.push_back(p);
     }
@@ -1521,8 +1517,6 @@ static pfh_status core_pieces(PlanImpl &P, const Step &outer, int64_t m, const L
             x.tab_in = c_off;
             x.mul_in = (int)n2;
             x.valid_in = (int)m;
-            st = twiddle_table(P, M, x.tw, x.tw_bsh);
-            if (st) return st;
             x.tw_m = (int)M;
             Step p;
             st = make_piece(P, p, n1, digs, n2 * in.point, n2, in.buf, rs_buf, x, tb, big);

@@ -80,7 +80,6 @@ enum StageFlags : int {
     F_HERM_DOUBLE = 64, // R2C adjoint weights: x2 on interior bins, Im := 0 at DC/Nyquist
     F_HERM_HALF = 128,  // C2R adjoint weights: x1/2 on interior bins
     F_WEIGHTS = 256,    // apply pre/post edge weights (R2R adjoints)
-    F_XCD_REMAP = 512,  // (unused) contiguous eighths of the tiles per XCD
     F_DIRECT_FIRST = 1024, // first radix pass reads global memory into registers
     F_DIRECT_LAST = 2048,  // last radix pass writes global memory from registers (C2C)
     F_NT = 4096,           // stage arrays exceed the last-level cache: non-temporal loads and stores

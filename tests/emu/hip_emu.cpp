@@ -464,11 +464,100 @@ static T axis_factor(const char *what, const StageArgs<T> &a, int64_t line, int 
     return f;
 }
 
+// The middle of a split Bluestein convolution (k_line_plan KIND 4): row k1 of m
+// values, DFT, times the transformed chirp [k1][k2], conjugated, DFT, times the
+// split's twiddles [k1][q2], in place.
+template <typename T>
+static void emulate_conv(const char *what, const StageArgs<T> &a)
+{
+    const int m = a.m;
+    const ld pi = 3.141592653589793238462643383279502884L;
+    std::vector<cld> z(m), Z(m);
+    auto dft = [&]() {
+        for (int k = 0; k < m; ++k) {
+            cld acc{0, 0};
+            for (int p = 0; p < m; ++p) {
+                const ld ang = -2 * pi * (ld)(((int64_t)p * k) % m) / (ld)m;
+                acc = {acc.re + z[p].re * cosl(ang) - z[p].im * sinl(ang), acc.im + z[p].re * sinl(ang) + z[p].im * cosl(ang)};
+            }
+            Z[k] = acc;
+        }
+    };
+    if (a.mode != M_C2C || a.nin != m || a.nout != m || !a.xtab_out || !a.xtwr || a.xdig < 0 || a.scale != (T)1 ||
+        (a.flags & (F_CONJ_IN | F_CONJ_OUT | F_XIN | F_XOUT | F_XTW)))
+        fail("%s: shape of a convolution's middle", what);
+    for (int64_t line = 0; line < a.nlines; ++line) {
+        int64_t io, oo, x = line, row = 0;
+        offsets(a.g, line, io, oo);
+        for (int d = 0; d < a.g.nd; ++d) {
+            if (d == a.xdig) row = x % a.g.ext[d];
+            x /= a.g.ext[d];
+        }
+        const cpx<T> *bh = a.xtab_out + row * m, *tw = a.xtwr + row * m;
+        const cpx<T> *q = reinterpret_cast<const cpx<T> *>(a.src) + io;
+        cpx<T> *o = reinterpret_cast<cpx<T> *>(a.dst) + oo;
+        if (!check_read("chirp rows", bh, m * sizeof(cpx<T>)) || !check_read("twiddle rows", tw, m * sizeof(cpx<T>))) return;
+        for (int p = 0; p < m; ++p) {
+            if (!check_read(what, q + (int64_t)p * a.ips, sizeof(*q))) return;
+            z[p] = {(ld)q[(int64_t)p * a.ips].x, (ld)q[(int64_t)p * a.ips].y};
+        }
+        if (g_math_dft) {
+            dft();
+            for (int k = 0; k < m; ++k) {
+                const cld w = cmul_l(Z[k], {(ld)bh[k].x, (ld)bh[k].y});
+                z[k] = {w.re, -w.im};
+            }
+            dft();
+        }
+        for (int p = 0; p < m; ++p) {
+            const cld w = g_math_dft ? cmul_l(Z[p], {(ld)tw[p].x, (ld)tw[p].y}) : z[p];
+            if (!check_write(what, o + (int64_t)p * a.ops, sizeof(*o))) return;
+            o[(int64_t)p * a.ops].x = (T)w.re;
+            o[(int64_t)p * a.ops].y = (T)w.im;
+        }
+    }
+}
+
+// Tables of k_line_blue: M >= 2 m - 1, the chirp and a few values of the
+// transformed conjugate chirp over M.
+template <typename T>
+static void check_blue(const char *what, const StageArgs<T> &a)
+{
+    const int64_t m = a.xvalid_in, M = a.m;
+    const ld pi = 3.141592653589793238462643383279502884L, eps = sizeof(T) == 4 ? 1e-7L : 1e-15L;
+    const int64_t fft = mode_cin(a.mode) && a.mode == M_C2C ? a.nin : m;
+    if (m < 1 || 2 * m - 1 > M || fft != m) fail("%s: Bluestein of %" PRId64 " in %" PRId64, what, m, M);
+    if (!check_read("chirp", a.xtab_in, (size_t)m * sizeof(cpx<T>)) ||
+        !check_read("transformed chirp", a.xtab_out, (size_t)M * sizeof(cpx<T>)))
+        return;
+    for (int64_t j = 0; j < m; ++j) {
+        const ld t = pi * (ld)((j * j) % (2 * m)) / (ld)m;
+        if (fabsl((ld)a.xtab_in[j].x - cosl(t)) > eps || fabsl((ld)a.xtab_in[j].y + sinl(t)) > eps) {
+            fail("%s: chirp entry %" PRId64, what, j);
+            return;
+        }
+    }
+    for (int64_t k : {(int64_t)0, (int64_t)1, M / 3, M / 2, M - 1}) {
+        cld acc{0, 0};
+        for (int64_t j = 1 - m; j < m; ++j) {
+            const int64_t i = j < 0 ? -j : j, at = (j + M) % M;
+            const ld t = pi * (ld)((i * i) % (2 * m)) / (ld)m - 2 * pi * (ld)((at * k) % M) / (ld)M;
+            acc = {acc.re + cosl(t) / M, acc.im + sinl(t) / M};
+        }
+        if (fabsl((ld)a.xtab_out[k].x - acc.re) > eps || fabsl((ld)a.xtab_out[k].y - acc.im) > eps)
+            fail("%s: transformed chirp entry %" PRId64, what, k);
+    }
+}
+
 // identity-on-points emulation of one line stage
 template <typename T>
 static void emulate(const char *what, const StageArgs<T> &a)
 {
     if (a.gate && *a.gate) return;
+    if (a.flags & F_LINE_CONV) {
+        emulate_conv(what, a);
+        return;
+    }
     if (g_math) {
         emulate_math(what, a);
         return;
@@ -504,18 +593,31 @@ static void emulate(const char *what, const StageArgs<T> &a)
     }
 }
 
+// Every tile by exactly one workgroup (runs of tiles per XCD permute them).
 template <typename T>
 static void check_grid(const char *what, const StageArgs<T> &a, int64_t grid)
 {
-    if (a.flags & F_XCD_REMAP) {
-        if (grid != 8LL * a.xcd_per || 8LL * a.xcd_per < a.ntiles) fail("%s: XCD grid", what);
-    } else if (grid < a.ntiles) {
-        fail("%s: grid %" PRId64 " < tiles %" PRId64, what, grid, a.ntiles);
+    if (grid < a.ntiles) fail("%s: grid %" PRId64 " < tiles %" PRId64, what, grid, a.ntiles);
+    if (a.xcd_per > 0 && grid % (8LL * a.xcd_per) != 0) fail("%s: grid %" PRId64 " for runs of %d", what, grid, a.xcd_per);
+    if (grid > (1 << 22)) return;
+    std::vector<char> hit((size_t)a.ntiles, 0);
+    for (int64_t b = 0; b < grid; ++b) {
+        const int64_t t = tile_of_block(a, (uint32_t)b);
+        if (t < a.ntiles && hit[(size_t)t]++) {
+            fail("%s: tile %" PRId64 " twice", what, t);
+            return;
+        }
     }
+    for (int64_t t = 0; t < a.ntiles; ++t)
+        if (!hit[(size_t)t]) {
+            fail("%s: tile %" PRId64 " by no workgroup", what, t);
+            return;
+        }
 }
 
 int g_launches = 0;
 int g_blue_launches = 0;         // stages on k_line_blue
+int g_conv_launches = 0;         // middles of three-launch convolutions
 int g_all_launches = 0;         // every device launch, fills included
 bool g_reject_endpoints = false; // the emulated C2R boundary check rejects every spectrum
 static const bool g_trace = std::getenv("PFH_EMU_TRACE") != nullptr;
@@ -716,7 +818,11 @@ hipError_t launch_line_fast(const StageArgs<T> &a, int r0, int r1, int r2, int e
     ++g_launches;
     ++g_all_launches;
     begin_launch();
-    if (a.flags & F_LINE_BLUE) ++g_blue_launches;
+    if (a.flags & F_LINE_BLUE) {
+        ++g_blue_launches;
+        check_blue("line_fast", a);
+    }
+    if (a.flags & F_LINE_CONV) ++g_conv_launches;
     if (threads > 512) fail("line_fast: %d threads", threads);
     if (!fast_plan_available((int)sizeof(T), r0, r1, r2, em)) fail("line_fast: plan not instantiated");
     if (a.radix[0] != r0 || a.radix[1] != r1 || (r2 && a.radix[2] != r2)) fail("line_fast: radices differ");
@@ -2291,6 +2397,16 @@ void long_cases()
     }
     unsetenv("PFH_LONG_LINE_MAX");
     unsetenv("PFH_BLUESTEIN_PRIME");
+    // the three-launch convolution, which PFH_BLUESTEIN_PRIME turns off
+    const int conv = pfh::g_conv_launches;
+    for (int op : {PFH_FORWARD, PFH_INVERSE}) {
+        for (int64_t n : {521, 1042, 1031}) local_long_case<double>(PFH_LOCAL_C2C, 0, n, op, 2, 1e-12);
+        for (int64_t n : {521, 1042}) local_long_case<double>(PFH_LOCAL_R2C, 0, n, op, 2, 1e-12);
+    }
+    local_long_case<float>(PFH_LOCAL_C2C, 0, 523, PFH_FORWARD, 2, 2e-6);
+    local_long_case<double>(PFH_LOCAL_R2R, PFH_DCT2, 541, PFH_FORWARD, 1, 1e-12);
+    route_long_case<double>({521, 3, 2}, 2, PFH_FORWARD, 1e-12);
+    if (pfh::g_conv_launches - conv < 13) fail("three-launch convolutions: %d", pfh::g_conv_launches - conv);
     // real-size lines with the default thresholds: launch shapes, thread
     // mappings, LDS and every address, without the arithmetic
     pfh::g_math_dft = false;
