@@ -14,7 +14,7 @@
 //    or the generic kernel);
 //  - real transforms handle the spectrum in pairs X_q, X_{m-q}: one twiddle
 //    product gives both, and their two (DCT-IV), three or four real outputs;
-//  - composite radices (6, 9, 10, 12, 14, 15, 16) keep lengths up to 256 at
+//  - composite radices (6, 9, 10, 12, 14, 15, 16) keep most lengths up to 256 at
 //    two passes, one LDS exchange.
 // Measured per launch on MI355X, before (generic kernel, or k_line_fast with
 // run-time threads per line) and after: 180 x 225 x 200 x 3 f32 R2C, 97 MB in

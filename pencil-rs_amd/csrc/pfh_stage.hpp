@@ -34,8 +34,8 @@ constexpr int kEmax = 8;         // generic kernel values per thread and pass
 // Generic kernel budgets. The instantiation with the odd-prime passes gives
 // the radix 5 and 7 passes 3 and 2 butterflies per thread and, in f32, the
 // radix 11 / 13 passes 2 and the pre-processing 16 values per thread, so a
-// 385-point line (5 x 7 x 11) takes 32 threads (f32) or 64 (f64) instead of
-// 128; f64 keeps the smaller budgets, whose registers would spill.
+// line of 5 x 7 x 11 points takes 32 threads (f32) or 64 (f64) instead of 128; f64
+// keeps the smaller budgets, whose registers would spill.
 constexpr int generic_pre_e(bool wide, bool f32) { return (wide && f32) ? 16 : kEmax; }
 
 constexpr int generic_mb(int R, bool wide, bool f32)
@@ -242,11 +242,18 @@ struct PlaneArgs {
 
 // Line plans {R0, R1, R2, EM}: the radix sequence and the values per thread
 // and pass of the route stages that k_line_plan runs (pfh_line.hip): every
-// length 2^a 3^b 5^c 7^d from 8 to 1024 that three radices up to 16 reach, and
-// the 385-point FFT of a DST-I line of 384 points. Of the splits of a length
-// the one with the fewest lane instructions is taken, idle lanes of partial
-// passes and about 14 per value and LDS exchange included; lengths below 64
-// keep at most 8 values per thread, so that a wave still covers long runs.
+// length 2^a 3^b 5^c 7^d from 8 to 1024 that two or three radices of 2 to 10, 12,
+// 14, 15 and 16 reach, and 385 = 5 x 7 x 11, the FFT of a DST-I line of 384 points,
+// which has had a plan of its own from the start. The rule of the table, of
+// all radix sequences and EM from the largest radix to 16 (8 below 64 points, so
+// that a wave still covers long runs): the least sum over the passes of rounds x
+// threads x (instructions of the radix-R butterfly + 14 R for the LDS exchange),
+// idle lanes of partial rounds so included, times 1 + 0.002 EM, 1.03 above 32
+// threads a line and 1.2 above 64; butterflies of 2 3 4 5 7 8 9 11 16 count 4 16 16 36
+// 66 56 136 150 170 lane instructions, the composite ones B ops(A) + A ops(B). The
+// variants with EM = R0 (line_plan_real_only) stand beside the plans of 65 to 128
+// points that have at most 8 threads a line. tests/test_line_plan_table.py derives
+// the table from this.
 #define PFH_FAST_ROUTE_PLANS(X) \
     X(float, 2, 4, 0, 4)       \
     X(float, 3, 3, 0, 3)       \
