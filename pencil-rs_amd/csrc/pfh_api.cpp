@@ -88,6 +88,7 @@ struct pfh_plan_s {
 // device information
 // ---------------------------------------------------------------------------
 
+constexpr size_t kStaticLds = 256; // of the kernels that have any (device_info)
 static std::mutex g_dev_mu;
 static std::vector<DeviceInfo> g_devs;
 static std::vector<int> g_dev_ready;
@@ -110,7 +111,6 @@ static pfh_status device_info(DeviceInfo &out)
         std::snprintf(d.arch, sizeof d.arch, "%s", prop.gcnArchName);
         // The planner's budget leaves kStaticLds bytes per workgroup for the
         // kernels' static LDS (the pass plan copy of k_line_stage).
-        constexpr size_t kStaticLds = 256;
         size_t lim = prop.sharedMemPerBlock;
         if (lim < 65536) lim = 65536;
         if (lim > 65536) {
@@ -796,7 +796,10 @@ static int threads_per_line(const Step &st, int tbytes)
 // of lines whose points are runs of 256 bytes (complex) or 128 bytes (real),
 // halved while the workgroup is too large, or, down to 128-byte (complex) and
 // 64-byte runs, while two workgroups do not share a CU's LDS. Rows: about 256
-// threads.
+// threads, fewer lines while two workgroups do not share a CU's LDS (f64 lines of
+// 256 points and more: 12 lines of 300 points, rows of 4 padded to 5, take 87 KB with
+// their tables). 2^22 points of f64 lines on MI355X, one workgroup a CU and two:
+// DCT-III of 600 points 49 -> 37 us, DST-I of 511 48 -> 34, C2C of 450 34 -> 28.
 static pfh_status size_line_plan(Step &st, const DeviceInfo &dev, int tbytes, const Tuning &tu)
 {
     const int cb = 2 * tbytes;
@@ -816,6 +819,7 @@ static pfh_status size_line_plan(Step &st, const DeviceInfo &dev, int tbytes, co
         while (lt / 2 >= least && lds_of(lt) > dev.lds_limit / 2) lt /= 2;
     } else {
         lt = (int)std::max<int64_t>(1, std::min<int64_t>(256 / tpl, st.nlines));
+        while (lt > 1 && lds_of(lt) > (dev.lds_limit + kStaticLds) / 2) --lt; // (no static LDS here)
     }
     while (lt > 1 && lds_of(lt) > dev.lds_limit) lt /= 2;
     if (lds_of(lt) > dev.lds_limit) return set_err(PFH_ERR_UNSUPPORTED, "line does not fit in LDS");

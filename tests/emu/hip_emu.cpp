@@ -617,6 +617,8 @@ static void check_grid(const char *what, const StageArgs<T> &a, int64_t grid)
 
 int g_launches = 0;
 int g_blue_launches = 0;         // stages on k_line_blue
+size_t g_last_lds = 0;            // of the last stage on a compile-time plan
+int g_last_flags = 0, g_last_lt = 0;
 int g_conv_launches = 0;         // middles of three-launch convolutions
 int g_all_launches = 0;         // every device launch, fills included
 bool g_reject_endpoints = false; // the emulated C2R boundary check rejects every spectrum
@@ -823,6 +825,9 @@ hipError_t launch_line_fast(const StageArgs<T> &a, int r0, int r1, int r2, int e
         check_blue("line_fast", a);
     }
     if (a.flags & F_LINE_CONV) ++g_conv_launches;
+    g_last_lds = lds_bytes;
+    g_last_flags = a.flags;
+    g_last_lt = a.lt;
     if (threads > 512) fail("line_fast: %d threads", threads);
     if (!fast_plan_available((int)sizeof(T), r0, r1, r2, em)) fail("line_fast: plan not instantiated");
     if (a.radix[0] != r0 || a.radix[1] != r1 || (r2 && a.radix[2] != r2)) fail("line_fast: radices differ");
@@ -2219,6 +2224,47 @@ void fold_cases()
             }
 }
 
+// Tiles of f64 rows: two workgroups a CU, 16 lines of 256 points at exactly half of
+// its LDS among them, and k_line_fast where the line plan saves no pass.
+void row_tiles()
+{
+    const int before = g_fail;
+    struct R {
+        int kind, r2r;
+        int64_t n, lines;
+        bool two, plan;
+    };
+    for (const R &c : std::vector<R>{{PFH_LOCAL_R2R, PFH_DCT3, 600, 6990, true, true},
+                                     {PFH_LOCAL_R2R, PFH_DST1, 511, 8208, true, true},
+                                     {PFH_LOCAL_C2C, 0, 450, 9320, true, true},
+                                     {PFH_LOCAL_R2R, PFH_DCT4, 512, 8192, true, true},
+                                     {PFH_LOCAL_C2C, 0, 512, 8192, true, false},
+                                     {PFH_LOCAL_R2C, 0, 1024, 4096, true, false},
+                                     {PFH_LOCAL_C2C, 0, 256, 4096, true, true}}) {
+        pfh_desc d;
+        std::memset(&d, 0, sizeof d);
+        d.kind = c.kind;
+        d.precision = PFH_F64;
+        d.line_len = (size_t)c.n;
+        d.r2r_kind = c.r2r;
+        pfh_plan p = nullptr;
+        if (pfh_plan_create(&d, &p) != PFH_OK) fail("row tiles: plan of %" PRId64, c.n);
+        const int64_t out = c.kind == PFH_LOCAL_R2C ? c.n / 2 + 1 : c.n;
+        void *src = dmalloc((size_t)(c.lines * c.n) * 16, true), *dst = dmalloc((size_t)(c.lines * out) * 16);
+        if (pfh_local_execute(p, PFH_FORWARD, src, (size_t)(c.lines * c.n), dst, (size_t)(c.lines * out), nullptr, 0,
+                              nullptr, 0) != PFH_OK)
+            fail("row tiles: execute %" PRId64, c.n);
+        const bool plan = (pfh::g_last_flags & pfh::F_LINE_PLAN) != 0;
+        if (plan != c.plan || (plan && (pfh::g_last_lds * 2 <= kLdsLimit) != c.two))
+            fail("row tiles: kind %d n %" PRId64 ": plan %d, %zu bytes of LDS, %d lines", c.kind, c.n, plan ? 1 : 0,
+                 pfh::g_last_lds, pfh::g_last_lt);
+        if (c.r2r == PFH_DCT4 && pfh::g_last_lt != 16) fail("row tiles: %d lines of DCT-IV", pfh::g_last_lt);
+        for (void *q : {src, dst}) (void)hipFree(q);
+        pfh_plan_destroy(p);
+    }
+    std::printf("row tiles: %s\n", g_fail == before ? "ok" : "FAILED");
+}
+
 // The rules that pick a copy's kernel, at measured shapes on both sides.
 void copy_rules()
 {
@@ -2543,6 +2589,7 @@ int main(int argc, char **argv)
     if (argc == 2 && std::strcmp(argv[1], "copies") == 0) {
         copy_rules();
         launch_bounds();
+        row_tiles();
         std::printf("launches %d, failures %d\n", pfh::g_launches, g_fail);
         return g_fail ? 1 : 0;
     }
