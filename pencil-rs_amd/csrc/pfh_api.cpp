@@ -433,8 +433,8 @@ static bool choose_line_plan(Step &st, int tbytes, bool in_stage)
 }
 
 // Picks a compile-time specialized kernel: k_line_fast's plans for the
-// batched kernels and for stages larger than the last-level cache (its
-// non-temporal instances), k_line_plan otherwise. PFH_FAST=0 disables both,
+// batched kernels, for stages larger than the last-level cache (its
+// non-temporal instances) and for f64 lines of 512 points, k_line_plan otherwise. PFH_FAST=0 disables both,
 // PFH_FAST512=<0|1|2> selects k_line_fast's 512-point f32 variant (16x32 with
 // 16 registers, 8x8x8, 16x32 with 32).
 static void choose_fast(Step &st, int tbytes, const Tuning &tu)
@@ -1184,7 +1184,9 @@ static int64_t split_factor(PlanImpl &P, int64_t m, int tb)
 
 // Relative cost per value of one piece of length len: a line plan streams at
 // about 4.5 TB/s on MI355X with two radix passes and at 3.6 with three, the
-// generic kernel at about 1.8 TB/s with four and in proportion to them.
+// generic kernel at about 1.8 TB/s with four and in proportion to them, a good
+// third less with radix 7 (the instance of the odd radices: convolutions of 1792
+// points in one piece took 156 us for 2^22 points f32, of 2048 124, the split 80).
 static double piece_cost(int64_t len, int tb, const Tuning &tu)
 {
     int lp[3], em = 0;
@@ -1192,7 +1194,9 @@ static double piece_cost(int64_t len, int tb, const Tuning &tu)
     if (has_line_plan(len, tb, tu)) return lp[2] ? 1.25 : 1.0;
     std::vector<int> r;
     const int max_r = tu.max_radix ? tu.max_radix : (tb == 4 ? 16 : 8);
-    return radix_plan((int)len, r, max_r) ? std::max(1.0, 0.62 * (double)r.size()) : 64.0;
+    if (!radix_plan((int)len, r, max_r)) return 64.0;
+    const bool wide = std::any_of(r.begin(), r.end(), is_wide_radix);
+    return std::max(1.0, (wide ? 0.87 : 0.62) * (double)r.size());
 }
 
 // Does an FFT of length m that fits one generic stage run faster as a split

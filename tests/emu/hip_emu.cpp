@@ -2407,6 +2407,14 @@ void blue_routes()
         blue_route<float>(PFH_LOCAL_R2R, PFH_DCT1, m + 1, PFH_FORWARD, m, want);
         blue_route<double>(PFH_LOCAL_R2R, PFH_DST1, m - 1, PFH_FORWARD, m, want);
     }
+    // convolutions whose one-piece lengths have a radix 7 (1680 .. 1792): split
+    pfh::g_math = true;
+    for (int64_t n : {839, 883, 894}) {
+        const int conv = pfh::g_conv_launches;
+        blue_route<float>(PFH_LOCAL_C2C, 0, n, PFH_FORWARD, n, 2);
+        if (pfh::g_conv_launches == conv) fail("%" PRId64 " points: not a three-launch convolution", n);
+    }
+    pfh::g_math = false;
     pfh::g_math_dft = true;
     std::printf("lines without a plan: %s\n", g_fail == before ? "ok" : "FAILED");
 }
