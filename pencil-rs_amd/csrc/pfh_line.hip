@@ -19,7 +19,7 @@
 // Measured per launch on MI355X, before (generic kernel, or k_line_fast with
 // run-time threads per line) and after: 180 x 225 x 200 x 3 f32 R2C, 97 MB in
 // and out, 147 / 159 / 176 -> 48 / 37 / 35 us; 256 x 384 x 240 f32, 94 MB in
-// and out, DST-I 124 -> 75 us, DCT-II / III 71 / 78 -> 49 us, DCT-IV 75 -> 51
+// and out, DST-I 124 -> 75 us, DCT-II / III 71 / 78 -> 49 us, DCT-IV 75 -> 57
 // us; f64 DCT-I of 129 points 41 -> 26 us (32 MB), FFT of 192 points 24 -> 15
 // us.
 // This file is compiled once per precision and kind (PFH_LINE_F64,
