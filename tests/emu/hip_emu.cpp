@@ -619,6 +619,7 @@ int g_launches = 0;
 int g_blue_launches = 0;         // stages on k_line_blue
 size_t g_last_lds = 0;            // of the last stage on a compile-time plan
 int g_last_flags = 0, g_last_lt = 0;
+std::vector<int> g_lengths;         // FFT lengths of the launches
 int g_conv_launches = 0;         // middles of three-launch convolutions
 int g_all_launches = 0;         // every device launch, fills included
 bool g_reject_endpoints = false; // the emulated C2R boundary check rejects every spectrum
@@ -647,6 +648,7 @@ hipError_t launch_line_stage(const StageArgs<T> &a, bool wide, int threads, size
     if (threads > (wide ? kMaxThreadsWide : kMaxThreads)) fail("line_stage: %d threads", threads);
     trace("line_stage", a, threads, grid);
     check_shape("line_stage", a, threads, lds_bytes, Regs<T>::emax, false, 0, wide);
+    g_lengths.push_back(a.m);
     check_grid("line_stage", a, grid);
     if (a.twn > 0) check_read("line_stage tables", a.tw, (size_t)a.twn * 2 * sizeof(T));
     emulate("line_stage", a);
@@ -825,6 +827,7 @@ hipError_t launch_line_fast(const StageArgs<T> &a, int r0, int r1, int r2, int e
         check_blue("line_fast", a);
     }
     if (a.flags & F_LINE_CONV) ++g_conv_launches;
+    g_lengths.push_back(a.m);
     g_last_lds = lds_bytes;
     g_last_flags = a.flags;
     g_last_lt = a.lt;
@@ -2413,6 +2416,18 @@ void blue_routes()
         const int conv = pfh::g_conv_launches;
         blue_route<float>(PFH_LOCAL_C2C, 0, n, PFH_FORWARD, n, 2);
         if (pfh::g_conv_launches == conv) fail("%" PRId64 " points: not a three-launch convolution", n);
+    }
+    // splits: two line plans whatever their lengths, one only near the root
+    struct S {
+        int64_t n;
+        int a, b;
+    };
+    for (const S &c : std::vector<S>{{21321, 103, 207}, {23100, 60, 385}}) {
+        pfh::g_lengths.clear();
+        blue_route<float>(PFH_LOCAL_C2C, 0, c.n, PFH_FORWARD, c.n, 2);
+        const std::vector<int> &g = pfh::g_lengths;
+        if (g.size() != 2 || std::min(g[0], g[1]) != c.a || std::max(g[0], g[1]) != c.b)
+            fail("%" PRId64 " points: pieces %d x %d", c.n, g.empty() ? 0 : g[0], g.size() < 2 ? 0 : g[1]);
     }
     pfh::g_math = false;
     pfh::g_math_dft = true;
