@@ -1216,7 +1216,9 @@ static bool split_pays(PlanImpl &P, int64_t m, int tb, int64_t &n1)
 // Length of Bluestein's cyclic convolution for an FFT of length m: a
 // 7-smooth M >= 2m - 1 that runs as one piece or a split, the cheapest (M x
 // the cost of its pieces) among those up to 25% above the smallest. For m =
-// 10007: 20160 = 140 x 144, two passes each.
+// 10007: 20160 = 140 x 144, two passes each. Lengths with a factor 3^6 are avoided:
+// the roundings of radix 3 add up (f64 relative L2 error of 4342 points 4.8e-16 with M =
+// 8748, 3.7e-16 without; C2R of 362 points 3.6e-16 with 729, 2.5e-16).
 static int64_t bluestein_length(PlanImpl &P, int64_t m, int tb)
 {
     const Tuning &tu = P.tuning;
@@ -1238,6 +1240,7 @@ static int64_t bluestein_length(PlanImpl &P, int64_t m, int tb)
             cost = piece_cost(n1, tb, tu) + piece_cost(M / n1, tb, tu);
         }
         cost *= (double)M;
+        if (M % 729 == 0) cost *= 1.5;
         if (!best || cost < best_cost) {
             best = M;
             best_cost = cost;

@@ -2417,6 +2417,13 @@ void blue_routes()
         blue_route<float>(PFH_LOCAL_C2C, 0, n, PFH_FORWARD, n, 2);
         if (pfh::g_conv_launches == conv) fail("%" PRId64 " points: not a three-launch convolution", n);
     }
+    // convolution lengths without 3^6
+    for (int64_t n : {4342, 5826}) {
+        pfh::g_lengths.clear();
+        blue_route<double>(PFH_LOCAL_C2C, 0, n, PFH_FORWARD, n, 2);
+        const std::vector<int> &g = pfh::g_lengths;
+        if (g.size() != 3 || ((int64_t)g[0] * g[1]) % 729 == 0) fail("%" PRId64 " points: convolution of 3^6", n);
+    }
     // splits: two line plans whatever their lengths, one only near the root
     struct S {
         int64_t n;
