@@ -1208,10 +1208,17 @@ static bool split_pays(PlanImpl &P, int64_t m, int tb, int64_t &n1)
 {
     const Tuning &tu = P.tuning;
     n1 = 0;
-    if (has_line_plan(m, tb, tu)) return false;
+    if (tu.least_regions || has_line_plan(m, tb, tu)) return false;
     n1 = split_factor(P, m, tb);
     return n1 > 0 && piece_cost(n1, tb, tu) + piece_cost(m / n1, tb, tu) < piece_cost(m, tb, tu);
 }
+
+// Splits up to this length keep all their twiddles in one table (8 MiB f32 at
+// 2^20), read along neighbouring lines: one rounding and one load per value;
+// longer ones multiply two table entries (a third, shared by the values of a
+// butterfly, saves loads and costs a rounding: relative L2 error of 2^21 points
+// f32 1.73e-7 against 1.71e-7).
+constexpr int64_t kFullTwiddles = 1 << 20;
 
 // Length of Bluestein's cyclic convolution for an FFT of length m: a
 // 7-smooth M >= 2m - 1 that runs as one piece or a split, the cheapest (M x
@@ -1241,6 +1248,10 @@ static int64_t bluestein_length(PlanImpl &P, int64_t m, int tb)
         }
         cost *= (double)M;
         if (M % 729 == 0) cost *= 1.5;
+        // one region, or two for a split that is not run as three launches
+        if (tu.least_regions)
+            cost = (double)M * (n1 > 0 && !(M <= kFullTwiddles && has_line_plan(n1, tb, tu) && has_line_plan(M / n1, tb, tu))
+                                    ? 2.0 : 1.0);
         if (!best || cost < best_cost) {
             best = M;
             best_cost = cost;
@@ -1297,13 +1308,6 @@ static pfh_status twiddle_table(PlanImpl &P, int64_t M, int64_t &off, int &bsh)
         for (int64_t h = 0; h * B < M; ++h) push_cexp(t, h * B, M);
     });
 }
-
-// Splits up to this length keep all their twiddles in one table (8 MiB f32 at
-// 2^20), read along neighbouring lines: one rounding and one load per value;
-// longer ones multiply two table entries (a third, shared by the values of a
-// butterfly, saves loads and costs a rounding: relative L2 error of 2^21 points
-// f32 1.73e-7 against 1.71e-7).
-constexpr int64_t kFullTwiddles = 1 << 20;
 
 // exp(-2 pi i d k / (n1 n2)) at [k][d], k < n1, d < n2.
 static pfh_status full_twiddles(PlanImpl &P, int64_t n1, int64_t n2, int64_t &off)
@@ -3223,6 +3227,29 @@ static pfh_status execute_impl(PlanImpl &P, int op, const void *src, size_t src_
 // C ABI
 // ---------------------------------------------------------------------------
 
+// Operations of a route plan whose workspace exceeds the scratch of the
+// allocation-free entry point.
+static int over_scratch(const PlanImpl &P)
+{
+    int n = 0;
+    for (int op = 0; op < 6; ++op) {
+        if (P.ops[op].valid && op_ws_bytes(P, P.ops[op]) > (int64_t)kNoallocBytes) ++n;
+        if (P.ops_inplace[op].valid && op_ws_bytes(P, P.ops_inplace[op]) > (int64_t)kNoallocBytes) ++n;
+    }
+    return n;
+}
+
+static bool needs_least_regions(const PlanImpl &P)
+{
+    if (P.kind <= PFH_LOCAL_DHT || P.tuning.least_regions || over_scratch(P) == 0) return false;
+    for (const OpPlan &o : P.ops)
+        for (const Step &s : o.steps)
+            if (!s.pieces.empty()) return true;
+    return false;
+}
+
+static bool fewer_over_scratch(const PlanImpl &a, const PlanImpl &b) { return over_scratch(a) < over_scratch(b); }
+
 extern "C" {
 
 const char *pfh_version(void) { return "pencil-fft-hip 0.1.0 (gfx950)"; }
@@ -3295,6 +3322,18 @@ pfh_status pfh_plan_create(const pfh_desc *desc, pfh_plan *out)
     if (st) {
         delete p;
         return st;
+    }
+    // Faster pieces of long lines may take larger regions; where only those
+    // keep an operation from the allocation-free entry point, the smallest ones
+    if (needs_least_regions(p->impl)) {
+        pfh_plan q = new (std::nothrow) pfh_plan_s;
+        const pfh_error_info saved = g_err;
+        if (q) {
+            q->impl.tuning.least_regions = true;
+            if (create_impl(desc, q->impl) == PFH_OK && fewer_over_scratch(q->impl, p->impl)) std::swap(p, q);
+            delete q;
+        }
+        g_err = saved;
     }
     *out = p;
     return ok();

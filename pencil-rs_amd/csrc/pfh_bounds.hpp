@@ -2,6 +2,7 @@
 // that needs more runs as several launches.
 #pragma once
 
+#include <cstddef>
 #include <cstdint>
 
 #include "pfh_kernels.hpp"
@@ -10,6 +11,9 @@ namespace pfh {
 
 constexpr int64_t kMaxLaunchThreads = ((int64_t)1 << 32) - 1;
 constexpr int64_t kMaxBlocks256 = (int64_t)1 << 24; // one more than workgroups of 256 may have
+
+// Device scratch of the allocation-free entry point (pfh_noalloc.hip).
+constexpr size_t kNoallocBytes = (size_t)128 << 20;
 
 // Elementwise kernels: elements of a workgroup and of one launch.
 constexpr int kElementsPerBlock = 256 * 8;

@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "../../include/pencil_fft_hip.h"
+#include "pfh_bounds.hpp"
 
 namespace pfh {
 pfh_status set_error(pfh_status st, const char *msg, size_t required, size_t actual, size_t batch, size_t index,
@@ -28,7 +29,7 @@ pfh_status execute_on_scratch(pfh_plan plan, int op, const void *src, size_t src
 
 namespace {
 
-constexpr size_t kScratchBytes = size_t(128) << 20; // 128 MiB per GPU
+constexpr size_t kScratchBytes = pfh::kNoallocBytes; // 128 MiB per GPU
 constexpr int kMaxDevices = 64;
 
 __device__ __align__(256) unsigned char scratch[kScratchBytes];

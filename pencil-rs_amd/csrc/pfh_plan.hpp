@@ -155,6 +155,7 @@ struct Tuning {
     bool allow_line_plan = true; // route and local stages on k_line_plan (the batched kernels carry
                                  // the plans of PFH_FAST_PLANS only)
     bool allow_xcd = true;
+    bool least_regions = false; // long lines: the smallest regions, not the cheapest pieces
     int64_t max_launch_threads = kMaxLaunchThreads; // local lines beyond it run as several launches
     int slab_mb = -1;    // slab intermediate target in MiB (0: no slab pipelining, -1: default)
     bool fill_block = false; // column-access tiles also take `block` threads (batched launches)

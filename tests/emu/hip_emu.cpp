@@ -2227,6 +2227,27 @@ void fold_cases()
             }
 }
 
+// Workspaces of routes with long lines: faster pieces may take another region, but
+// not where that alone exceeds the allocation-free entry point's scratch. Real lines
+// of 4235 points (one piece 102 KB a line, a split 169 KB).
+void scratch_limit()
+{
+    const int before = g_fail;
+    auto bytes = [](size_t a) {
+        pfh_desc d = route_desc(PFH_R2C, PFH_F64, {a, a, 4235}, {});
+        pfh_plan p = nullptr;
+        size_t b = 0;
+        if (pfh_plan_create(&d, &p) != PFH_OK || pfh_plan_workspace_bytes(p, PFH_FORWARD, &b) != PFH_OK)
+            fail("scratch limit: plan of %zu x %zu x 4235", a, a);
+        if (p) pfh_plan_destroy(p);
+        return (double)b;
+    };
+    if (!(bytes(4) / 16 > 150e3)) fail("scratch limit: small plans split");
+    if (!(bytes(36) <= (double)pfh::kNoallocBytes)) fail("scratch limit: %.0f bytes", bytes(36));
+    if (!(bytes(64) / 4096 > 150e3)) fail("scratch limit: plans beyond it split");
+    std::printf("scratch limit: %s\n", g_fail == before ? "ok" : "FAILED");
+}
+
 // Tiles of f64 rows: two workgroups a CU, 16 lines of 256 points at exactly half of
 // its LDS among them, and k_line_fast where the line plan saves no pass.
 void row_tiles()
@@ -2620,6 +2641,7 @@ int main(int argc, char **argv)
         copy_rules();
         launch_bounds();
         row_tiles();
+        scratch_limit();
         std::printf("launches %d, failures %d\n", pfh::g_launches, g_fail);
         return g_fail ? 1 : 0;
     }

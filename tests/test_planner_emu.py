@@ -96,9 +96,11 @@ def test_lines_without_a_plan_keep_their_accuracy(emu):
 def test_copy_rules(emu):
     """Short axes and narrow rows are left to the callers' kernels; arrays of
     more than 2^24 workgroups run in parts or on kernels that loop. Rows of
-    long f64 lines share a CU's LDS by twos."""
+    long f64 lines share a CU's LDS by twos. Long lines' regions leave the
+    allocation-free entry point what it could run."""
     r = subprocess.run([emu, "copies"], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-2000:]
     assert "copy rules: ok" in r.stdout
     assert "launch bounds: ok" in r.stdout
     assert "row tiles: ok" in r.stdout
+    assert "scratch limit: ok" in r.stdout
